@@ -245,22 +245,20 @@ AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int ma
         part = part < 64 ? 64 : (part > 512 ? 512 : part);
         return {ATTN_SCHED_GRID, (int)part};
     }
-    // Measured on MI355X: while the (sequence, kv head) items fill at least a quarter of
-    // the resident workgroup slots, longest-first pieces (LPT: long items cut in equal
-    // pieces, dispatched longest first, split items merged inside the launch) balance
-    // ragged contexts best; beyond the sequences an LPT workgroup can rank, one workgroup
-    // per item (no split, no merge) when the items fill the slots. Otherwise stream-K
-    // splits evenly.
+    // Longest-first pieces (LPT: long items cut, dispatched longest first, split items merged
+    // inside the launch) at every batch the plan kernel can rank. Few items too: against the
+    // even stream-K split that served items below a quarter of the slots, per call with the
+    // plan of its step: one fp8 sequence of 3000 keys 38 -> 22.5 µs, eight of 300-1500 keys 49 ->
+    // 21.7 µs, two int8 sequences of 300 keys 60.5 -> 25.7 µs, eight int8 sequences of
+    // 16k-32k keys 121.1 -> 121.1 (112 without the plan launch); planned and run in one call,
+    // 34.3 -> 26.1 µs (one sequence), 45.6 -> 24.7 (eight), 137.0 -> 131.1 (eight long).
+    // Past kLptMaxSeqs sequences: one workgroup per item, or stream-K where contexts are long.
     const int G = num_q_heads / kv->num_kv_heads;
     const int nt = (G * rows + 15) / 16;
     const long long max_keys = (long long)max_blocks * kv->block_size;
     const long long items = (long long)num_seqs * kv->num_kv_heads;
     const long long slots = (long long)device_cu_count() * attn_occupancy((int)dtype_bytes(kv->dtype), nt);
-    // (With a merge launch of its own, LPT lost to stream-K at a quarter of the slots,
-    // config 4: 164 vs 117 µs. With the merge inside the launch and pieces of 4/3 of the
-    // mean slot load it wins there: 110.3 vs 112.7 µs, same box. At an eighth of the slots
-    // it loses: config 4 with two workgroups per CU, 120.2 vs 117.4 µs.)
-    if (4 * items >= slots && num_seqs <= kLptMaxSeqs) return {ATTN_SCHED_LPT, 0};
+    if (num_seqs <= kLptMaxSeqs) return {ATTN_SCHED_LPT, 0};
     if (items >= slots && max_keys <= kMfmaMaxPartition)
         return {ATTN_SCHED_GRID, (int)((max_keys + 63) / 64 * 64)};
     return {ATTN_SCHED_STREAMK, 0};

@@ -119,36 +119,39 @@ struct AttnPlan {
 
 // LPT schedule: most sequences the plan kernel ranks (one per thread).
 constexpr int kLptMaxSeqs = 1024;
-// LPT piece length: T = ceil(C * num / (slots * den)) chunks for C chunks of work over
-// `slots` resident workgroups, num/den = 2 of the mean slot load when the (sequence, kv
-// head) items fill the slots and 7/5 when they are fewer.
-//   - Items that fill the slots are cut into pieces of T chunks and a shorter last piece,
-//     which the longest-first order then runs at the end. Measured on MI355X (the call with
+// LPT piece length T, in chunks, for C chunks of work over `slots` resident workgroups:
+//   - (sequence, kv head) items that fill the slots: T = ceil(C * num / (slots * den)), twice
+//     the mean slot load; pieces of T chunks and a shorter last piece, which the
+//     longest-first order then runs at the end. Measured on MI355X (the call with
 //     its append, one layer, mean over eight seeded config-3 layouts, same box): equal
 //     pieces at 8/5 (the earlier rule) 127.1 µs; T pieces and a remainder at 8/5 / 9/5 / 2:
 //     124.1 / 123.9 / 123.3 (bench layout 123.7 -> 118.5 at 9/5 and 2); at 7/5, 6/5 and 1
-//     slower than equal pieces on the bench layout (123.7, 129.2, 132.7). With equal
-//     pieces the factors had measured 3/2 / 8/5 / 13/8 / 5/3 / 17/10: 131.0 / 128.4 /
-//     129.1 / 130.3 / 130.8 over eight layouts (an older build).
-//   - Fewer items than slots: every long item has to be cut to fill the slots, and equal
-//     pieces balance them (config 2 with remainder pieces: 71 -> 79 µs). Mean over eight
-//     seeded config-2 layouts (items = slots / 2), f = 6/5 / 5/4 / 11/8 / 4/3 / 10/7 / 7/5
-//     / 13/9 / 3/2: 69.9 / 67.9 / 61.5 / 63.1 / 61.4 / 60.7 / 61.4 / 62.8 µs (bench layout:
-//     7/5 70.4, 4/3 70.8).
-//   - Config 5 (items = 2 slots) cuts nothing at any of these factors.
-// The factors are tuned constants; the time moves in steps as items cross piece
-// boundaries.
-constexpr int kLptPieceNum = 2, kLptPieceDen = 1;            // items >= slots
-constexpr int kLptPieceNumFew = 7, kLptPieceDenFew = 5;      // items < slots
+//     slower than equal pieces on the bench layout (123.7, 129.2, 132.7). Config 5 (items =
+//     2 slots) cuts nothing at any of these factors.
+//   - Fewer items than slots: equal pieces of at most T, T the shortest length whose pieces
+//     still fit one round of slots (a longer T leaves slots idle, a shorter one starts a
+//     second, nearly empty round). Among 64 candidates, t_lo + i * ceil(t_lo / kLptTSpan)
+//     from the mean slot load t_lo; if none fits, the longest (over 3 times the mean). Against
+//     the fixed 7/5 of the mean, per call on one box: config-2-shaped bf16 items (slots / 2)
+//     68.2 -> 66.3 µs, config-4-shaped int8 items (slots / 8) 124 -> 112 µs.
+//   - Never shorter than lpt_min_chunks: a cut costs the item's records, their merge and a
+//     second piece start, about 5 µs. At 8 / 12 / 16 chunks of 64 tokens, 24 short int8
+//     sequences (200-900 keys) took 32.2 / 27.2 / 28.3 µs a call and one fp8 sequence of
+//     3000 keys 21.9 / 22.5 / 24.3; at 8 / 12 / 16 chunks of 32 tokens, 16 bf16 sequences of
+//     256-1024 keys took 25.9 / 27.0 / 23.3.
+constexpr int kLptPieceNum = 2, kLptPieceDen = 1;  // items >= slots
+constexpr int kLptTSpan = 31;
+__host__ __device__ constexpr int lpt_min_chunks(int tok) { return tok == 64 ? 12 : 16; }
 __host__ __device__ constexpr bool lpt_few_items(int slots, int num_seqs, int num_kv_heads) {
     return num_seqs * num_kv_heads < slots;
 }
-// Bound on the number of LPT pieces (= main-grid workgroups and partial records): the
-// cuts of every item at T chunks give at most C/T + items pieces, C/T <= slots * den / num
-// (the smaller factor, 7/5, gives the larger bound). (Stream-K needs grid + items records,
-// which is more: the workspace holds the larger of the two.)
+// Bound on the number of LPT pieces (= main-grid workgroups and partial records). Cutting at
+// T chunks gives at most C / T + items pieces, and C / T <= slots / 2 with items that fill
+// the slots or when no candidate fits; otherwise the pieces fit the slots. (Stream-K's
+// grid + items records are more: the workspace holds the larger of the two.)
 __host__ __device__ constexpr int lpt_records(int slots, int num_seqs, int num_kv_heads) {
-    return (slots * kLptPieceDenFew + kLptPieceNumFew - 1) / kLptPieceNumFew + num_seqs * num_kv_heads;
+    const int cut = slots / 2 + 1 + num_seqs * num_kv_heads;
+    return cut > slots ? cut : slots;
 }
 AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks,
                    int partition_tokens);

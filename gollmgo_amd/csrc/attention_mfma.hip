@@ -1071,9 +1071,9 @@ __global__ void __launch_bounds__(256, attn_occupancy(PoolTraits<DT>::kEB, NT)) 
 
 // ---- LPT schedule: pieces of a few mean slot loads at most, longest first ----
 //
-// Items longer than T = ceil(f * total chunks / resident slots) are cut: while the items
-// fill the slots, into pieces of T chunks and a shorter last piece; with fewer items, into
-// equal pieces of at most T chunks. attn_lpt_plan_kernel orders the pieces by size,
+// Items longer than T chunks (attention_common.h) are cut: while the items fill the slots,
+// into pieces of T chunks and a shorter last piece; with fewer items, into equal pieces of at
+// most T chunks. attn_lpt_plan_kernel orders the pieces by size,
 // descending (ties: sequence, then piece, then kv head), and the main launch runs them in
 // that order (with
 // few items the first round pairs long and shorter pieces per CU, lpt_slot): dispatched in
@@ -1167,6 +1167,7 @@ __device__ __forceinline__ int block_excl_scan_1024(int v, int* s_w, int* total)
 __global__ void __launch_bounds__(1024) attn_lpt_plan_kernel(AttnArgs a, int Hkv, int tok, int slots, int recs) {
     __shared__ __align__(16) int s_key[kLptMaxSeqs];  // piece size in chunks (0: no work)
     __shared__ __align__(16) int s_cnt[kLptMaxSeqs];  // pieces of the sequence over all kv heads
+    __shared__ int s_nch[kLptMaxSeqs], s_ctx[kLptMaxSeqs];
     __shared__ long long s_w[16];
     __shared__ int s_wi[16];
     const int B = a.num_seqs;
@@ -1175,10 +1176,9 @@ __global__ void __launch_bounds__(1024) attn_lpt_plan_kernel(AttnArgs a, int Hkv
     const int ctx = b < B ? seq_keys(a, b, kBS) : 0;
     const long long C = block_sum_1024((long long)Hkv * nch, s_w);
     const bool few = lpt_few_items(slots, B, Hkv);
-    const long long den = (long long)slots * (few ? kLptPieceDenFew : kLptPieceDen);
-    const long long num = few ? kLptPieceNumFew : kLptPieceNum;
-    const int T = (int)max((C * num + den - 1) / den, (long long)kStreamKMinChunks);
     if (!few) {
+        const int T = (int)max((C * kLptPieceNum + (long long)slots * kLptPieceDen - 1) / ((long long)slots * kLptPieceDen),
+                               (long long)lpt_min_chunks(tok));
         // Items that fill the slots: pieces of T chunks and the remainder last. The full
         // pieces come first (by sequence), then the last pieces by size, descending (ties:
         // sequence). Records by (sequence, piece, kv head): a sequence's first record is the
@@ -1229,51 +1229,88 @@ __global__ void __launch_bounds__(1024) attn_lpt_plan_kernel(AttnArgs a, int Hkv
         for (int q = total + b; q < recs; q += B) table[q] = make_int4(-1, 0, 0, 0);
         return;
     }
-    // Fewer items than slots: every long item has to be cut to fill the slots, and equal
-    // pieces balance them. Records by rank.
+    // Fewer items than slots: every long item has to be cut to fill the slots, into equal
+    // pieces. T is the shortest piece length whose pieces still fit one round of slots:
+    // 64 candidate lengths from the mean slot load up, each counted by 16 threads (one per
+    // wave) over a slice of the sequences.
+    const int t_lo = (int)max((C + slots - 1) / slots, (long long)lpt_min_chunks(tok));
+    const int t_step = (t_lo + kLptTSpan - 1) / kLptTSpan;
+    if (b < kLptMaxSeqs) s_key[b] = nch;
+    __syncthreads();
+    const int cand = t_lo + (threadIdx.x & 63) * t_step;
+    int pieces = 0;
+    for (int q = threadIdx.x >> 6; q < B; q += 16) {
+        const int n = s_key[q];
+        pieces += (n + cand - 1) / cand;
+    }
+    s_cnt[threadIdx.x] = pieces;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        int sum = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) sum += s_cnt[64 * w + threadIdx.x];
+        const unsigned long long fits = __ballot(sum * Hkv <= slots);
+        // (None fits, for instance when the items nearly fill the slots: the longest one.)
+        if (threadIdx.x == 0) s_wi[0] = t_lo + (fits ? __builtin_ctzll(fits) : 63) * t_step;
+    }
+    __syncthreads();
+    const int T = s_wi[0];
     const int np = nch ? (nch + T - 1) / T : 0;
     const int key = np ? (nch + np - 1) / np : 0;
     const int cnt = np * Hkv;
+    __syncthreads();  // (s_key and s_cnt are reused)
     // (Entries past B, up to a multiple of 8, read as empty.)
     if (b < ((B + 7) & ~7)) {
         s_key[b] = b < B ? key : 0;
         s_cnt[b] = b < B ? cnt : 0;
     }
-    const long long total = block_sum_1024(cnt, s_w);  // (its barriers also publish s_key / s_cnt)
+    const int total = (int)block_sum_1024(cnt, s_w);  // (its barriers also publish s_key / s_cnt)
     int* plan = a.plan;
     if (b == 0) {
-        plan[0] = (int)total;
+        plan[0] = total;
         plan[1] = 0;
     }
-    if (b >= B) return;
     // Pieces ahead of this sequence's: larger pieces, then equal pieces of lower sequences.
     // Eight sequences per step from 16-byte LDS reads (independent adds, no serial chain).
     int pos = 0;
-    for (int t0 = 0; t0 < B; t0 += 8) {
-        const int4 k0 = *(const int4*)&s_key[t0], k1 = *(const int4*)&s_key[t0 + 4];
-        const int4 n0 = *(const int4*)&s_cnt[t0], n1 = *(const int4*)&s_cnt[t0 + 4];
-        const int kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-        const int nn[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
+    if (b < B) {
+        for (int t0 = 0; t0 < B; t0 += 8) {
+            const int4 k0 = *(const int4*)&s_key[t0], k1 = *(const int4*)&s_key[t0 + 4];
+            const int4 n0 = *(const int4*)&s_cnt[t0], n1 = *(const int4*)&s_cnt[t0 + 4];
+            const int kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+            const int nn[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int t = t0 + e;
-            pos += (kk[e] > key || (kk[e] == key && t < b)) ? nn[e] : 0;
+            for (int e = 0; e < 8; ++e) {
+                const int t = t0 + e;
+                pos += (kk[e] > key || (kk[e] == key && t < b)) ? nn[e] : 0;
+            }
+        }
+        int* seq = lpt_seq(plan, recs) + 2 * b;
+        seq[0] = pos;
+        seq[1] = np;
+    }
+    __syncthreads();
+    // The table is written by all threads, one (sequence, kv head) at a time.
+    if (b < B) {
+        s_key[b] = pos;
+        s_cnt[b] = np;
+        s_nch[b] = nch;
+        s_ctx[b] = ctx;
+    }
+    __syncthreads();
+    int4* table = (int4*)lpt_table(plan);
+    for (int i = threadIdx.x; i < B * Hkv; i += 1024) {
+        const int q = i / Hkv, h = i % Hkv;
+        const int qp = s_key[q], qn = s_cnt[q], n = s_nch[q], qc = s_ctx[q];
+        lpt_count(plan, recs, B)[i] = 0;
+        for (int j = 0; j < qn; ++j) {
+            const int c0 = (int)((long long)j * n / qn), c1 = (int)((long long)(j + 1) * n / qn);
+            table[lpt_slot(qp + j * Hkv + h, slots, total, true)] =
+                make_int4(q, h | (qn << 16), c0 * tok, min(c1 * tok, qc));
         }
     }
-    int* seq = lpt_seq(plan, recs) + 2 * b;
-    seq[0] = pos;
-    seq[1] = np;
-    for (int h = 0; h < Hkv; ++h) lpt_count(plan, recs, B)[b * Hkv + h] = 0;
-    int4* table = (int4*)lpt_table(plan);
-    for (int j = 0; j < np; ++j) {
-        const int c0 = (int)((long long)j * nch / np), c1 = (int)((long long)(j + 1) * nch / np);
-        const int t0 = c0 * tok, t1 = min(c1 * tok, ctx);
-        for (int h = 0; h < Hkv; ++h)
-            table[lpt_slot(pos + j * Hkv + h, slots, (int)total, B * Hkv <= slots)] =
-                make_int4(b, h | (np << 16), t0, t1);
-    }
     // Entries past the last piece tell their workgroups to exit.
-    for (int q = (int)total + b; q < recs; q += B) table[q] = make_int4(-1, 0, 0, 0);
+    for (int q = total + threadIdx.x; q < recs; q += 1024) table[q] = make_int4(-1, 0, 0, 0);
 }
 
 // The piece of a split item that finishes last merges the item's records: the online
@@ -1314,19 +1351,33 @@ __device__ void lpt_merge_if_last(const AttnArgs& a, int Hkv, int b, int kvh, in
             const int r = e / (kD / 4), d4 = e % (kD / 4);
             float M = -1e30f, L = 0.f;
             float acc[4] = {0.f, 0.f, 0.f, 0.f};
-            for (int j = 0; j < np; ++j) {
-                const size_t q = (size_t)(first + j * Hkv + kvh) * RW + r;
-                const float mx = load_agent(a.ws_ml + q * 2), ly = load_agent(a.ws_ml + q * 2 + 1);
-                float v[4];
+            // Four records per step, their loads issued together.
+            int jp = 0;
+            auto merge = [&](auto n) {
+                constexpr int N = decltype(n)::value;
+                float mx[N], ly[N], v[N][4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = load_agent(a.ws_acc + q * kD + 4 * d4 + i);
-                const float mn = fmaxf(M, mx);
-                const float fo = __expf(M - mn), fn = __expf(mx - mn);
-                M = mn;
-                L = L * fo + ly * fn;
+                for (int u = 0; u < N; ++u) {
+                    const size_t q = (size_t)(first + (jp + u) * Hkv + kvh) * RW + r;
+                    mx[u] = load_agent(a.ws_ml + q * 2);
+                    ly[u] = load_agent(a.ws_ml + q * 2 + 1);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[i] = acc[i] * fo + v[i] * fn;
-            }
+                    for (int i = 0; i < 4; ++i) v[u][i] = load_agent(a.ws_acc + q * kD + 4 * d4 + i);
+                }
+#pragma unroll
+                for (int u = 0; u < N; ++u) {
+                    const float mn = fmaxf(M, mx[u]);
+                    const float fo = __expf(M - mn), fn = __expf(mx[u] - mn);
+                    M = mn;
+                    L = L * fo + ly[u] * fn;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[i] = acc[i] * fo + v[u][i] * fn;
+                }
+                jp += N;
+            };
+            while (jp + 4 <= np) merge(std::integral_constant<int, 4>{});
+            if (jp + 2 <= np) merge(std::integral_constant<int, 2>{});
+            if (jp < np) merge(std::integral_constant<int, 1>{});
             const float inv = L > 0.f ? 1.f / L : 0.f;
             const int j = r / G, g = r % G;
             const size_t obase = (((size_t)b * a.rows + j) * a.num_q_heads + (size_t)kvh * G + g) * kD + 4 * d4;
