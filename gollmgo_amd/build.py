@@ -39,6 +39,7 @@ HIPCC_FLAGS = [
 # unchanged, config 4 117.8 -> 118.1.
 SOURCE_FLAGS = {
     "attention_mfma.hip": ("-mllvm", "-amdgpu-sched-strategy=max-ilp"),
+    "attention_full.hip": ("-mllvm", "-amdgpu-sched-strategy=max-ilp"),
 }
 
 

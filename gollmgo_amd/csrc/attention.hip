@@ -11,12 +11,16 @@
 // (kernels/gollmgo_paged_attn.cu:234-384), whose reduce is not followed because it
 // normalises only in thread 0 and mixes partial strides.
 //
-// Two phase-1 kernels share one partial format and one combine kernel:
-//   - attn_mfma_kernel (attention_mfma.hip): gfx950 MFMA path for head_dim 128,
-//     block_size 16, BF16/F16/FP8/INT8 pools, G*R <= 64 rows per kv head;
+// Phase-1 kernels:
+//   - attention_mfma.hip: gfx950 MFMA path for head_dim 128, block_size 16,
+//     BF16/F16/FP8/INT8 pools, G*R <= 64 rows per kv head;
+//   - attention_full.hip: the same pieces for head_dim 64 and for more rows per kv head, at
+//     the precision of the per-row kernel (automatic schedule, up to kLptMaxSeqs sequences);
 //   - attn_generic_kernel (here): any head_dim <= 1024 / block size / pool dtype,
 //     one wave per (row, head, partition), scalar online softmax. Used for the
-//     shapes the MFMA tiling does not cover (e.g. fp32 pools, head_dim 64).
+//     shapes the MFMA tiling does not cover (fp32 pools, other head_dims and block sizes)
+//     and for explicit partitions of attention_full.hip's shapes. Its partitions and the
+//     MFMA partition grid share one partial format and one combine kernel.
 #include <type_traits>
 
 #include "gg_common.h"
@@ -233,6 +237,10 @@ gg_status_t launch_append_from_tables(const AttnArgs& a, const KVView& kv, hipSt
 AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks,
                    int partition_tokens) {
     if (partition_tokens > 0) return {ATTN_SCHED_GRID, partition_tokens};
+    const AttnShape sh = attn_shape(kv, rows, num_q_heads);
+    // (2^18 heads over all sequences: a plan of a few MB.)
+    if (sh.full && num_seqs <= kLptMaxSeqs && (long long)num_seqs * kv->num_kv_heads * sh.groups <= (1 << 18))
+        return {ATTN_SCHED_LPT, 0};
     if (!attn_mfma_supported(kv, rows, num_q_heads)) {
         // One wave per (row, head, partition): partitions of 64..512 keys, as many as
         // it takes to reach about 2048 waves (the kernel's time is the longest wave's
@@ -253,11 +261,9 @@ AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int ma
     // 16k-32k keys 121.1 -> 121.1 (112 without the plan launch); planned and run in one call,
     // 34.3 -> 26.1 µs (one sequence), 45.6 -> 24.7 (eight), 137.0 -> 131.1 (eight long).
     // Past kLptMaxSeqs sequences: one workgroup per item, or stream-K where contexts are long.
-    const int G = num_q_heads / kv->num_kv_heads;
-    const int nt = (G * rows + 15) / 16;
     const long long max_keys = (long long)max_blocks * kv->block_size;
     const long long items = (long long)num_seqs * kv->num_kv_heads;
-    const long long slots = (long long)device_cu_count() * attn_occupancy((int)dtype_bytes(kv->dtype), nt);
+    const long long slots = (long long)device_cu_count() * attn_occupancy((int)dtype_bytes(kv->dtype), sh.nt, kv->head_dim);
     if (num_seqs <= kLptMaxSeqs) return {ATTN_SCHED_LPT, 0};
     if (items >= slots && max_keys <= kMfmaMaxPartition)
         return {ATTN_SCHED_GRID, (int)((max_keys + 63) / 64 * 64)};
@@ -281,13 +287,16 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
                                                      a.partition % 64 == 0 && a.partition <= kMfmaMaxPartition);
     // Draft rows of the call: the MFMA kernels append them piece by piece (start_piece);
     // the generic path takes a launch of its own first.
-    if (a.k_new && !mfma) {
+    // So do the row groups of an INT8 item: each would re-quantise the block it appends to.
+    AttnArgs m = a;
+    if (a.k_new && (!mfma || (a.row_groups > 1 && kv->dtype == GG_DTYPE_INT8))) {
         const gg_status_t st = launch_append_from_tables(a, view, s);
         if (st != GG_OK) return st;
+        m.k_new = nullptr;
     }
     if (mfma) {
         // Stream-K and LPT launch their own merge over their record layout.
-        gg_status_t st = launch_attn_mfma(a, view, s);
+        gg_status_t st = launch_attn_mfma(m, view, s);
         if (st != GG_OK) return st;
         if (a.sched != ATTN_SCHED_GRID) return check_hip(hipGetLastError(), "verify_attention launch");
     } else {

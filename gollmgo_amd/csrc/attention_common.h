@@ -96,11 +96,11 @@ inline bool attn_mfma_supported(const KV* kv, int rows, int num_q_heads) {
 
 // MFMA kernel workgroups (of four waves) per CU for a pool's element size and row-tile
 // count: two while one wave's registers fit half the file (one or two row tiles; three
-// row tiles of a 1-byte pool in 32-token chunks, 217-248 VGPRs), else one. Shared by the
+// row tiles of a 1-byte pool in 32-token chunks, 217-248 VGPRs; head_dim 64), else one. Shared by the
 // launch bounds, the stream-K grid (one resident wave of workgroups) and the schedule
 // choice.
-__host__ __device__ constexpr int attn_occupancy(int elem_bytes, int nt) {
-    return nt <= 2 || (elem_bytes == 1 && nt == 3) ? 2 : 1;
+__host__ __device__ constexpr int attn_occupancy(int elem_bytes, int nt, int head_dim) {
+    return nt <= 2 || (elem_bytes == 1 && nt == 3) || head_dim == 64 ? 2 : 1;
 }
 
 // Tokens per MFMA chunk for a pool's element size and row-tile count. At one or two row
@@ -109,6 +109,29 @@ __host__ __device__ constexpr int attn_occupancy(int elem_bytes, int nt) {
 // halves the chunk's K/V, score and P registers next to the three or four O tiles.
 __host__ __device__ constexpr int attn_chunk_tokens(int elem_bytes, int nt) {
     return elem_bytes == 1 && nt <= 2 ? 64 : 32;
+}
+
+// How the MFMA kernels tile a shape: nt row tiles of 16 per workgroup, the G * rows query rows
+// of a kv head cut into `groups` of 16 * nt. `full`: the kernels that keep queries and
+// probabilities at fp32's precision (attention_full.hip).
+struct AttnShape {
+    bool full;
+    int nt, groups;
+};
+// Head_dim 64, or more than 64 query rows per kv head. At head_dim 128 two row tiles and the
+// three bf16 parts of P fit half the register file, at head_dim 64 four do. (A longer group
+// list than the plan's 16-bit head field holds goes to the generic kernel.)
+inline bool attn_full_supported(const KV* kv, int rows, int num_q_heads) {
+    const long long tiles = ((long long)(num_q_heads / kv->num_kv_heads) * rows + 15) / 16;
+    return kv->block_size == 16 && (kv->head_dim == 64 || (kv->head_dim == 128 && tiles > 4)) &&
+           kv->dtype != GG_DTYPE_F32 && kv->num_kv_heads * tiles <= 0x7fff;
+}
+inline AttnShape attn_shape(const KV* kv, int rows, int num_q_heads) {
+    const int tiles = (num_q_heads / kv->num_kv_heads * rows + 15) / 16;
+    if (!attn_full_supported(kv, rows, num_q_heads)) return {false, tiles, 1};
+    const int most = kv->head_dim == 64 ? 4 : 2;
+    const int groups = (tiles + most - 1) / most;
+    return {true, (tiles + groups - 1) / groups, groups};
 }
 
 // How one verify_attention call is scheduled.
@@ -145,18 +168,21 @@ __host__ __device__ constexpr int lpt_min_chunks(int tok) { return tok == 64 ? 1
 __host__ __device__ constexpr bool lpt_few_items(int slots, int num_seqs, int num_kv_heads) {
     return num_seqs * num_kv_heads < slots;
 }
-// Bound on the number of LPT pieces (= main-grid workgroups and partial records). Cutting at
-// T chunks gives at most C / T + items pieces, and C / T <= slots / 2 with items that fill
-// the slots or when no candidate fits; otherwise the pieces fit the slots. (Stream-K's
-// grid + items records are more: the workspace holds the larger of the two.)
-__host__ __device__ constexpr int lpt_records(int slots, int num_seqs, int num_kv_heads) {
-    const int cut = slots / 2 + 1 + num_seqs * num_kv_heads;
+// Bound on the number of LPT pieces (= main-grid workgroups), `heads` items per sequence.
+// Cutting at T chunks gives at most C / T + items pieces, and C / T <= slots / 2 with items that
+// fill the slots or when no candidate fits; otherwise the pieces fit the slots.
+__host__ __device__ constexpr int lpt_pieces(int slots, int num_seqs, int heads) {
+    const int cut = slots / 2 + 1 + num_seqs * heads;
     return cut > slots ? cut : slots;
 }
+// Bound on the partial records: a split item of n > T chunks has at most 2 n / T pieces, so
+// split items have at most 2 C / T <= slots.
+__host__ __device__ constexpr int lpt_records(int slots) { return slots; }
 AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks,
                    int partition_tokens);
 
 gg_status_t launch_attn_mfma(const AttnArgs& a, const KVView& kv, hipStream_t s);
+gg_status_t launch_attn_full(const AttnArgs& a, const KVView& kv, const AttnShape& sh, hipStream_t s);
 gg_status_t launch_append_from_tables(const AttnArgs& a, const KVView& kv, hipStream_t s);
 
 #ifdef __HIPCC__

@@ -83,7 +83,8 @@ struct AttnArgs {
     float* ws_ml;      // partition grid: [seqs][rows][Hq][max_parts][2]; stream-K: [records][G*R][2]
     float* ws_acc;     // partition grid: [seqs][rows][Hq][max_parts][D]; stream-K: [records][G*R][D]
     int sched;         // ATTN_SCHED_*: how the (sequence, kv head) items are cut
-    int sk_grid;       // stream-K / LPT: resident workgroup slots (attn_streamk_grid)
+    int sk_grid;       // stream-K / LPT: resident workgroup slots (attn_slots)
+    int row_groups;    // groups the query rows of a kv head are cut into (AttnShape)
     int* plan;         // LPT: piece plan in the workspace, after the records
     int plan_ready;    // LPT: the plan is already in the workspace (gg_verify_attention_plan)
     int sk_min_chunks;    // least chunks a stream-K workgroup takes
@@ -99,12 +100,12 @@ struct AttnArgs {
 enum { ATTN_SCHED_GRID = 0, ATTN_SCHED_STREAMK = 1, ATTN_SCHED_LPT = 2 };
 
 // Stream-K and LPT: resident workgroup slots for a shape on the current device, and the
-// workspace both need: grid + num_seqs * Hkv partial records of G*rows rows, as (max,
-// sum) pairs, then (64-float aligned) P.V rows, then the LPT plan (ints). ml_elems and
-// acc_elems receive the float counts of the first two parts.
-int attn_streamk_grid(const KV* kv, int rows, int num_q_heads);
-size_t attn_streamk_workspace_bytes(const KV* kv, int num_seqs, int rows, int num_q_heads,
-                                    size_t* ml_elems, size_t* acc_elems);
+// workspace of a schedule: partial records (LPT: one per piece of a split item; stream-K: grid
+// + items) as (max, sum) pairs, then (64-float aligned) P.V rows, then the LPT plan (ints).
+// ml_elems and acc_elems receive the float counts of the first two parts.
+int attn_slots(const KV* kv, int rows, int num_q_heads);
+size_t attn_record_workspace_bytes(const KV* kv, int sched, int num_seqs, int rows, int num_q_heads,
+                                   size_t* ml_elems, size_t* acc_elems);
 int device_cu_count();
 size_t attn_workspace_bytes(const KV* kv, int num_seqs, int rows, int num_q_heads,
                             int max_blocks, int partition);

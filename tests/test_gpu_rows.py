@@ -1,0 +1,74 @@
+"""GPU parity of the MFMA attention for head_dim 64 and for more than 64 query rows per kv head
+(row groups), against the float64 oracle and against the per-row kernel it took over from
+(an explicit partition still runs that one): no less exact, for every pool and query type."""
+import pytest
+import torch
+
+from gollmgo_amd.workloads import CONFIGS, VerifyConfig
+from helpers import TOL, say
+from test_gpu_kv import _fused_vs_separate, run_attention_case
+
+pytestmark = pytest.mark.gpu
+
+# (B, R, Hq, H, D, contexts): row tiles 1 to 4 at head_dim 64, then groups of rows.
+SHAPES = [
+    (2, 1, 2, 2, 64, [0, 130]),
+    (3, 5, 24, 4, 64, [40, 700, 1500]),        # 30 rows: two tiles
+    (2, 3, 32, 2, 64, [33, 5000]),             # 48 rows: three
+    (2, 16, 8, 2, 64, [17, 900]),              # 64 rows: four
+    (2, 9, 32, 4, 64, [300, 64]),              # 72 rows: two groups of three tiles
+    (2, 5, 32, 2, 128, [600, 90]),             # 80 rows: three groups of two tiles
+    (1, 65, 4, 1, 128, [2000]),                # 260 rows: nine groups
+]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "fp8", "int8"])
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_no_less_exact_than_the_per_row_kernel(gpu, dt, shape):
+    B, R, Hq, H, D, ctx = SHAPES[shape]
+    for q_dt in ("bf16", "f16", "f32"):
+        say(f"rows dt={dt} q={q_dt} shape={SHAPES[shape]}")
+        err = run_attention_case(dt, B, R, Hq, H, D, 16, ctx, src="bf16", q_dt=q_dt, seed=60 + shape)
+        ref = run_attention_case(dt, B, R, Hq, H, D, 16, ctx, src="bf16", q_dt=q_dt, seed=60 + shape, partition=64)
+        print(f"  rel err {err:.2e}, per-row kernel {ref:.2e}")
+        assert err <= TOL[dt]
+        # The largest of a few thousand fp32-level errors each; 2e-6 is 16 units of 2^-23.
+        assert err <= max(2 * ref, 2e-6), (err, ref)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("q_sd", [1e-6, 1e6])
+def test_queries_far_from_one(gpu, dt, q_sd):
+    """Queries are scaled into the f16 operand range by a power of two and back."""
+    say(f"rows q_sd={q_sd} dt={dt}")
+    for q_dt in ("bf16", "f32"):
+        B, R, Hq, H, D, ctx = SHAPES[1]
+        err = run_attention_case(dt, B, R, Hq, H, D, 16, ctx, src="bf16", q_dt=q_dt, seed=3, q_sd=q_sd,
+                                 kv_sd=3.0 / max(q_sd, 1.0), v_sd=1.0)
+        assert err <= TOL[dt]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp8"])
+def test_ragged_rows(gpu, dt):
+    """Row groups that a short sequence has no rows for write nothing."""
+    say(f"rows ragged dt={dt}")
+    err = run_attention_case(dt, 3, 6, 64, 4, 128, 16, [300, 1000, 17], row_counts=[6, 1, 3], src="bf16", q_dt="bf16",
+                             seed=7)
+    assert err <= TOL[dt]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "fp8", "int8"])
+@pytest.mark.parametrize("Hq,H,D,R,B,ctx", [
+    (32, 8, 64, 6, 5, (100, 2500)),    # rows patched from LDS (past the first chunks)
+    (32, 8, 64, 6, 5, (0, 40)),        # rows in the first chunks
+    (16, 2, 64, 8, 40, (200, 900)),    # four row tiles
+    (32, 2, 128, 6, 6, (100, 1500)),   # three row groups of an item append the same rows
+])
+def test_append_attention_equals_append_then_attention(gpu, monkeypatch, dt, Hq, H, D, R, B, ctx):
+    say(f"rows fused append dt={dt} Hq={Hq} H={H} D={D} R={R} ctx={ctx}")
+    monkeypatch.setitem(CONFIGS, 99, VerifyConfig("rows", B, R - 1, Hq, H, D, 16, ("uniform", *ctx), dt, "bf16", 1000,
+                                                  "f32", "greedy", seed=D + R))
+    # (Ragged row counts leave unwritten positions behind the context here, and an int8 block
+    # re-quantises whatever bytes they hold.)
+    _fused_vs_separate(99, dt, B, ("uniform", *ctx), dt != "int8")
+    torch.cuda.empty_cache()
