@@ -342,6 +342,227 @@ __global__ void __launch_bounds__(256) append_int8_block_kernel(AppendArgs a) {
     }
 }
 
+// ---- block size 16: whole block runs ----
+//
+// The rows that follow each other in one block (a run, led by its first row; skipped rows do
+// not break it) are written by one workgroup per kv head as one tile: 16-byte source loads, K
+// rows stored whole, V transposed in LDS so that a dim's 16 offsets leave as one 16-byte store
+// (partial runs: the 4-byte words that are whole, the rest by element). INT8 pools follow
+// append_int8_block_kernel's rule for the run.
+// Workgroup (g, h) takes the runs led by rows [g * grp, (g + 1) * grp): 16 rows, about one run
+// of a prompt, in large calls, 4 in small INT8 ones, where the rows are the verify rows of many
+// sequences and a workgroup with several runs does them one after the other.
+//
+// Bound by memory in large calls. The element kernels wrote V one element at a time, at the
+// tile's 16-offset stride, and INT8 started a workgroup per row, whose leader walked its run's
+// slots one load after the other. A prompt of 8192 rows of 8 heads x 128 dims, bf16 source, per
+// layer: FP8 38.9 -> 14.6 µs (50 MB, 3.4 TB/s), BF16 41.3 -> 16.7, INT8 1388 -> 17.4; 2000
+// rows 9.8 -> 7.0, 10.1 -> 7.2 and 296 -> 7.4.
+constexpr int kRunBs = 16;     // block size
+constexpr int kRunRows = 1024; // above: any pool (launch_kv_append)
+constexpr int kRunMaxD = 128;  // one 8-dim item per thread: 16 offsets x head_dim / 8 <= 256
+
+template <gg_dtype_t SRC, gg_dtype_t DST>
+__global__ void __launch_bounds__(256) append_run_kernel(AppendArgs a, int grp) {
+    constexpr int kEB = DST == GG_DTYPE_FP8_E4M3 || DST == GG_DTYPE_INT8 ? 1 : 2;
+    constexpr int kPitch = kRunBs * kEB + 4;  // bytes per dim in LDS: odd in 4-byte banks
+    __shared__ int s_row[kRunBs];             // row at each offset of the run's block, -1: none
+    __shared__ __align__(16) uint8_t s_v[kRunMaxD * kPitch];
+    __shared__ float s_red[2][4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = blockIdx.y, D = a.D, DG = D / 8;
+    const int r0 = blockIdx.x * grp;
+    // Slots of rows [r0 - 16, r0 + 48), one per lane, the same in every wave.
+    const int wr = r0 - 16 + lane;
+    const int slot = wr >= 0 && wr < a.n_rows ? a.slots[wr] : -1;
+    const int blk = slot_ok(slot, a.num_slots) ? slot / kRunBs : -1;
+    const unsigned long long valid = __ballot(blk >= 0);
+    // A row leads unless the nearest earlier row that is not skipped lands in its block.
+    bool lead = blk >= 0 && lane >= 16 && lane < 16 + grp;
+    {
+        const unsigned long long earlier = valid & ((1ull << lane) - 1);
+        const int p = earlier ? 63 - __builtin_clzll(earlier) : 0;
+        const int pblk = __shfl(blk, p);
+        if (lead && earlier) {
+            lead = pblk != blk;
+        } else if (lead) {
+            for (int q = r0 - 17; q >= 0; --q) {  // (sixteen or more skipped rows before it)
+                const int sq = a.slots[q];
+                if (!slot_ok(sq, a.num_slots)) continue;
+                lead = sq / kRunBs != blk;
+                break;
+            }
+        }
+    }
+    unsigned long long leaders = __ballot(lead);
+    if (!leaders) return;
+    float kinv = 1.f, vinv = 1.f;
+    if constexpr (DST == GG_DTYPE_FP8_E4M3) {
+        kinv = a.k_inv[h];
+        vinv = a.v_inv[h];
+    }
+    const int o = threadIdx.x / DG, g = threadIdx.x % DG;  // this thread's offset and dim group
+    while (leaders) {
+        const int i = __builtin_ctzll(leaders);
+        leaders &= leaders - 1;
+        const int B = __shfl(blk, i), lead_off = __shfl(slot, i) % kRunBs;
+        // The run ends at the first later row of another block.
+        const unsigned long long from = ~0ull << i;
+        const unsigned long long other = __ballot(blk >= 0 && blk != B) & from;
+        const unsigned long long upto = other ? (other & (0 - other)) - 1 : ~0ull;
+        const bool mine = blk == B && ((from & upto) >> lane & 1);
+        if (threadIdx.x < kRunBs) s_row[threadIdx.x] = -1;
+        __syncthreads();
+        if (wave == 0 && mine) s_row[slot % kRunBs] = wr;
+        if (!other && threadIdx.x == 0) {  // (only when skipped rows fill the rest of the window)
+            for (int q = r0 + 48; q < a.n_rows; ++q) {
+                const int sq = a.slots[q];
+                if (!slot_ok(sq, a.num_slots)) continue;
+                if (sq / kRunBs != B) break;
+                s_row[sq % kRunBs] = q;
+            }
+        }
+        __syncthreads();
+        const int row = o < kRunBs ? s_row[o] : -1;
+        const unsigned present = (unsigned)__ballot(lane < kRunBs && s_row[lane & (kRunBs - 1)] >= 0);
+        float kx[8], vx[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) kx[e] = vx[e] = 0.f;
+        if (row >= 0) {
+            const size_t src = ((size_t)row * a.Hkv + h) * D + 8 * g;
+            load8<SRC>(a.k, src, kx);
+            load8<SRC>(a.v, src, vx);
+        }
+        const size_t tile = ((size_t)B * a.Hkv + h) * (2 * (size_t)kRunBs * D);
+        float k_old = 0.f, v_old = 0.f, k_new = 0.f, v_new = 0.f;
+        const size_t si = (size_t)B * a.Hkv + h;
+        if constexpr (DST == GG_DTYPE_INT8) {
+            if (lead_off > 0) {
+                k_old = f16_bits_to_f32(a.k_bscale[si]);
+                v_old = f16_bits_to_f32(a.v_bscale[si]);
+            }
+            float mk = 0.f, mv = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                mk = fmaxf(mk, kx[e] == kx[e] ? fabsf(kx[e]) : 0.f);
+                mv = fmaxf(mv, vx[e] == vx[e] ? fabsf(vx[e]) : 0.f);
+            }
+            for (int x = 32; x > 0; x >>= 1) {
+                mk = fmaxf(mk, __shfl_xor(mk, x));
+                mv = fmaxf(mv, __shfl_xor(mv, x));
+            }
+            if (lane == 0) {
+                s_red[0][wave] = mk;
+                s_red[1][wave] = mv;
+            }
+            __syncthreads();
+            mk = fminf(fmaxf(fmaxf(s_red[0][0], s_red[0][1]), fmaxf(s_red[0][2], s_red[0][3])), 3.0e38f);
+            mv = fminf(fmaxf(fmaxf(s_red[1][0], s_red[1][1]), fmaxf(s_red[1][2], s_red[1][3])), 3.0e38f);
+            k_new = fmaxf(k_old, f16_bits_to_f32(f32_to_f16_rne_bits(mk / 127.0f)));
+            v_new = fmaxf(v_old, f16_bits_to_f32(f32_to_f16_rne_bits(mv / 127.0f)));
+            kinv = k_new > 0.f ? 1.0f / k_new : 0.f;
+            vinv = v_new > 0.f ? 1.0f / v_new : 0.f;
+        }
+        if (row >= 0) {
+            if constexpr (kEB == 1) {
+                uint32_t kw[2], vw[2];
+#pragma unroll
+                for (int e = 0; e < 8; e += 4) {
+                    if constexpr (DST == GG_DTYPE_FP8_E4M3) {
+                        kw[e >> 2] = f32x2_to_fp8e4m3_sat(kx[e] * kinv, kx[e + 1] * kinv) |
+                                     (f32x2_to_fp8e4m3_sat(kx[e + 2] * kinv, kx[e + 3] * kinv) << 16);
+                        vw[e >> 2] = f32x2_to_fp8e4m3_sat(vx[e] * vinv, vx[e + 1] * vinv) |
+                                     (f32x2_to_fp8e4m3_sat(vx[e + 2] * vinv, vx[e + 3] * vinv) << 16);
+                    } else {
+                        kw[e >> 2] = vw[e >> 2] = 0;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            kw[e >> 2] |= (uint32_t)(uint8_t)f32_to_i8_sat(kx[e + u] * kinv) << (8 * u);
+                            vw[e >> 2] |= (uint32_t)(uint8_t)f32_to_i8_sat(vx[e + u] * vinv) << (8 * u);
+                        }
+                    }
+                }
+                *(uint2*)(a.kc + tile + (size_t)o * D + 8 * g) = make_uint2(kw[0], kw[1]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s_v[(8 * g + e) * kPitch + o] = (uint8_t)(vw[e >> 2] >> (8 * (e & 3)));
+            } else {
+                uint16_t kb[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    kb[e] = DST == GG_DTYPE_BF16 ? f32_to_bf16_bits(kx[e]) : f32_to_f16_bits(kx[e]);
+                    const uint16_t vb = DST == GG_DTYPE_BF16 ? f32_to_bf16_bits(vx[e]) : f32_to_f16_bits(vx[e]);
+                    *(uint16_t*)&s_v[(8 * g + e) * kPitch + 2 * o] = vb;
+                }
+                *(uint4*)((uint16_t*)a.kc + tile + (size_t)o * D + 8 * g) =
+                    make_uint4(kb[0] | ((uint32_t)kb[1] << 16), kb[2] | ((uint32_t)kb[3] << 16),
+                               kb[4] | ((uint32_t)kb[5] << 16), kb[6] | ((uint32_t)kb[7] << 16));
+            }
+        }
+        __syncthreads();
+        // V: 16-byte runs of 16 / kEB offsets of one dim.
+        constexpr int kRuns = kEB;           // runs per dim
+        constexpr int kPer = kRunBs / kEB;   // offsets per run
+        constexpr int kWord = 4 / kEB;       // offsets per 4-byte word
+        for (int t = threadIdx.x; t < D * kRuns; t += 256) {
+            const int d = t / kRuns, o0 = (t % kRuns) * kPer;
+            const uint32_t* sv = (const uint32_t*)&s_v[d * kPitch + o0 * kEB];
+            const uint32_t w[4] = {sv[0], sv[1], sv[2], sv[3]};
+            uint8_t* dst = a.vc + (tile + (size_t)d * kRunBs + o0) * kEB;
+            const unsigned pm = present >> o0;
+            if ((pm & ((1u << kPer) - 1)) == (1u << kPer) - 1) {
+                *(uint4*)dst = make_uint4(w[0], w[1], w[2], w[3]);
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const unsigned m = (pm >> (u * kWord)) & ((1u << kWord) - 1);
+                    if (m == (1u << kWord) - 1) {
+                        ((uint32_t*)dst)[u] = w[u];
+                    } else if (m) {
+#pragma unroll
+                        for (int x = 0; x < kWord; ++x) {
+                            if (!((m >> x) & 1)) continue;
+                            if constexpr (kEB == 1) dst[4 * u + x] = (uint8_t)(w[u] >> (8 * x));
+                            else ((uint16_t*)dst)[2 * u + x] = (uint16_t)(w[u] >> (16 * x));
+                        }
+                    }
+                }
+            }
+        }
+        if constexpr (DST == GG_DTYPE_INT8) {
+            // Rows already in the block follow a grown scale.
+            if (lead_off > 0 && (k_new != k_old || v_new != v_old)) {
+                int8_t* kc = (int8_t*)a.kc + tile;
+                int8_t* vc = (int8_t*)a.vc + tile;
+                for (int x = threadIdx.x; x < lead_off * D; x += 256) {
+                    const int t = x / D, d = x % D;
+                    if (k_new != k_old) kc[x] = f32_to_i8_sat(((float)kc[x] * k_old) * kinv);
+                    if (v_new != v_old) {
+                        int8_t* p = vc + (size_t)d * kRunBs + t;
+                        *p = f32_to_i8_sat(((float)*p * v_old) * vinv);
+                    }
+                }
+            }
+            if (threadIdx.x == 0) {
+                a.k_bscale[si] = f32_to_f16_rne_bits(k_new);
+                a.v_bscale[si] = f32_to_f16_rne_bits(v_new);
+            }
+        }
+        __syncthreads();  // (s_row, s_v and s_red are reused)
+    }
+}
+
+template <gg_dtype_t SRC>
+void launch_run(const AppendArgs& a, hipStream_t s) {
+    const int grp = a.n_rows <= kRunRows ? 4 : kRunBs;
+    const dim3 grid((a.n_rows + grp - 1) / grp, a.Hkv);
+    switch (a.dst) {
+        case GG_DTYPE_F16: append_run_kernel<SRC, GG_DTYPE_F16><<<grid, 256, 0, s>>>(a, grp); break;
+        case GG_DTYPE_BF16: append_run_kernel<SRC, GG_DTYPE_BF16><<<grid, 256, 0, s>>>(a, grp); break;
+        case GG_DTYPE_FP8_E4M3: append_run_kernel<SRC, GG_DTYPE_FP8_E4M3><<<grid, 256, 0, s>>>(a, grp); break;
+        default: append_run_kernel<SRC, GG_DTYPE_INT8><<<grid, 256, 0, s>>>(a, grp); break;
+    }
+}
+
 }  // namespace
 
 gg_status_t launch_kv_append(KV* kv, int layer, const void* k, const void* v, gg_dtype_t src,
@@ -371,8 +592,23 @@ gg_status_t launch_kv_append(KV* kv, int layer, const void* k, const void* v, gg
     if (kv->scale_mode == GG_SCALE_PER_BLOCK) {
         a.k_bscale = (uint16_t*)kv->k_scales + (size_t)layer * kv->scale_layer_elems;
         a.v_bscale = (uint16_t*)kv->v_scales + (size_t)layer * kv->scale_layer_elems;
+    }
+    const bool vec = a.D % 8 == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0;
+    // Block runs: INT8 calls of any size, FP8 and 16-bit pools past kRunRows rows. Below, a
+    // thread per element (append_dim_kernel) has no tile to wait for: 5 verify rows 2.3 against
+    // 3.2 µs, 64 x 6 rows 3.7 against 5.7 at best, a prompt of 1000 rows 7.2 against 6.9, 2000 rows
+    // 9.8 against 7.0; 512 x 6 verify rows 15.8 against 13.5. INT8: 64 x 6 rows 16.1 -> 8.3,
+    // one sequence's five 7.1 -> 3.9.
+    const bool int8 = kv->scale_mode == GG_SCALE_PER_BLOCK;
+    if (vec && a.bs == kRunBs && a.D <= kRunMaxD && a.dst != GG_DTYPE_F32 && (int8 || a.n_rows > kRunRows)) {
+        switch (src) {
+            case GG_DTYPE_F32: launch_run<GG_DTYPE_F32>(a, s); break;
+            case GG_DTYPE_F16: launch_run<GG_DTYPE_F16>(a, s); break;
+            default: launch_run<GG_DTYPE_BF16>(a, s); break;
+        }
+    } else if (int8) {
         append_int8_block_kernel<<<dim3(n_rows, kv->num_kv_heads), 256, 0, s>>>(a);
-    } else if (a.D % 8 == 0 && a.dst != GG_DTYPE_INT8 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0) {
+    } else if (vec) {
         const bool per_dim = src != GG_DTYPE_F32 && a.dst != GG_DTYPE_F32;
         switch (src) {
             case GG_DTYPE_F32: launch_vec<GG_DTYPE_F32>(a, a.dst, s); break;

@@ -1,0 +1,62 @@
+"""GPU parity of the append by block runs (large calls; INT8 at every size), bit for bit against
+the oracle mirror: prompts that start inside a block, head_dims below the largest, runs of
+skipped rows longer than the kernel's slot window, rows in no order."""
+import numpy as np
+import pytest
+
+from helpers import PoolMirror, append_rows, say
+from test_gpu_kv import make_cache
+
+pytestmark = pytest.mark.gpu
+
+
+def check(dt, src, H, D, calls, nb, seed):
+    rng = np.random.default_rng(seed)
+    kv = make_cache(dt, H, D, 16, nb)
+    mirror = PoolMirror(kv)
+    if dt == "fp8":
+        sc = rng.uniform(0.005, 0.05, H).astype(np.float32)
+        kv.set_head_scales(0, sc, sc)
+        mirror.set_head_scales(sc, sc)
+    # Every byte written first, so that the whole pools compare.
+    calls = [np.arange(nb * 16)] + calls
+    for i, slots in enumerate(calls):
+        slots = np.asarray(slots, np.int32)
+        k = rng.normal(0, 1 + i, (len(slots), H, D)).astype(np.float32)
+        v = rng.normal(0, 1 + i, (len(slots), H, D)).astype(np.float32)
+        append_rows(kv, mirror, k, v, slots, src)
+        mirror.compare_with_device()
+    kv.close()
+
+
+def prompt(order, first, n):
+    p = first + np.arange(n)
+    return order[p // 16] * 16 + p % 16
+
+
+@pytest.mark.parametrize("dt", ["fp8", "bf16", "f16", "int8"])
+@pytest.mark.parametrize("src,D,first", [("bf16", 128, 0), ("f32", 64, 5), ("f16", 96, 15), ("bf16", 8, 1)])
+def test_prompt(gpu, dt, src, D, first):
+    say(f"append runs prompt dt={dt} src={src} D={D} first={first}")
+    order = np.random.default_rng(D).permutation(90)
+    check(dt, src, 2, D, [prompt(order, first, 1100), prompt(order, first + 1100, 17)], 90, D + first)
+
+
+@pytest.mark.parametrize("dt", ["fp8", "int8"])
+@pytest.mark.parametrize("n", [40, 1200])
+def test_skipped_rows_around_runs(gpu, dt, n):
+    """Skipped rows inside a run, before one and after one, in streaks that fill the slot
+    window (a run's other rows, or the row before it, then lie outside it)."""
+    say(f"append runs skipped rows dt={dt} n={n}")
+    order = np.random.default_rng(n).permutation(90)
+    slots = list(prompt(order, 3, n))
+    for at, streak in ((n - 3, 70), (20, 90), (9, 1), (0, 33)):
+        slots[at:at] = [-1] * streak
+    check(dt, "bf16", 2, 64, [slots], 90, n)
+
+
+@pytest.mark.parametrize("dt", ["fp8", "f16"])
+def test_rows_in_no_order(gpu, dt):
+    say(f"append runs shuffled dt={dt}")
+    slots = np.random.default_rng(4).permutation(90 * 16)[:1300]
+    check(dt, "bf16", 2, 128, [slots], 90, 8)
