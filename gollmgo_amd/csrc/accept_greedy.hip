@@ -3,8 +3,8 @@
 // Replaces the host-side Verify/argmax loop (internal/engine/speculative.go:68-84,
 // internal/engine/sampling.go:75-85) driven by emitSpeculative
 // (internal/engine/serving.go:514-566). Two launches:
-//   1) segment argmax: grid (segments, rows); each block scans 4096 logits of one
-//      row with 16-byte loads and writes (value, index) of its first maximum;
+//   1) segment argmax: each wave scans 4096 logits of one row with 16-byte loads and
+//      writes (value, index) of their first maximum;
 //   2) decide: one block per sequence merges the segments of rows 0..n, every row at
 //      once (a lane group per row), then walks the drafts in order: the first row whose
 //      argmax differs from its draft ends the accepted prefix and supplies the corrected
@@ -25,14 +25,6 @@ struct ArgBest {
     int i;
 };
 
-__device__ __forceinline__ void consider(ArgBest& b, float v, int i) {
-    // v == v filters NaN; ties keep the lower index.
-    if (v == v && (v > b.v || (v == b.v && i < b.i))) {
-        b.v = v;
-        b.i = i;
-    }
-}
-
 __device__ __forceinline__ ArgBest wave_best(ArgBest b) {
     for (int o = 32; o > 0; o >>= 1) {
         float ov = __shfl_xor(b.v, o);
@@ -45,64 +37,75 @@ __device__ __forceinline__ ArgBest wave_best(ArgBest b) {
     return b;
 }
 
+// First maximum of elements [base, end) of a row, by one wave: 16-byte vectors aligned in
+// memory, lane l taking vectors l, l + 64, ..., all of a segment's loads in flight at once.
+// A lane's indices ascend, so a strict `>` keeps its first maximum and never takes NaN. The
+// vectors that the segment cuts (a row need not start on 16 bytes) are read by element.
 template <gg_dtype_t DT>
-__device__ __forceinline__ void scan_vec(ArgBest& b, const void* row, int base, int V) {
-    // base is a multiple of kSeg; every 16-byte chunk is element-aligned because V*eb % 16 == 0.
-    constexpr int kPer = DT == GG_DTYPE_F32 ? 4 : 8;
-    constexpr int kIters = kSeg / (kThreads * kPer);
+__device__ __forceinline__ ArgBest scan_segment(const void* row, int base, int end) {
+    constexpr int kEB = DT == GG_DTYPE_F32 ? 4 : 2;
+    constexpr int kPer = 16 / kEB;
+    constexpr int kIters = kSeg / (64 * kPer);
+    const int lane = threadIdx.x & 63;
+    const uint8_t* p = (const uint8_t*)row + (size_t)base * kEB;
+    const int shift = (int)((uintptr_t)p & 15) / kEB;  // elements between the aligned start and base
+    const uint8_t* al = p - shift * kEB;
+    const int first = base - shift;
+    uint4 raw[kIters];
+    bool whole[kIters];
 #pragma unroll
     for (int it = 0; it < kIters; ++it) {
-        const int e0 = base + (it * kThreads + threadIdx.x) * kPer;
-        if (e0 >= V) break;
-        uint4 raw = *(const uint4*)((const uint8_t*)row + (size_t)e0 * (DT == GG_DTYPE_F32 ? 4 : 2));
-        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-        if constexpr (DT == GG_DTYPE_F32) {
+        const int j = it * 64 + lane, e0 = first + j * kPer;
+        whole[it] = e0 >= base && e0 + kPer <= end;
+        raw[it] = whole[it] ? *(const uint4*)(al + (size_t)j * 16) : make_uint4(0, 0, 0, 0);
+    }
+    ArgBest b{-INFINITY, kNone};
+    auto by_element = [&](int e0) {
+        for (int e = max(e0, base); e < min(e0 + kPer, end); ++e) {
+            const float v = load_as_f32(row, DT, e);
+            if (v > b.v) b = ArgBest{v, e};
+        }
+    };
 #pragma unroll
-            for (int k = 0; k < 4; ++k) consider(b, __uint_as_float(w[k]), e0 + k);
-        } else {
+    for (int it = 0; it < kIters; ++it) {
+        const int e0 = first + (it * 64 + lane) * kPer;
+        if (whole[it]) {
+            const uint32_t w[4] = {raw[it].x, raw[it].y, raw[it].z, raw[it].w};
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                uint16_t h = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
-                float f = DT == GG_DTYPE_BF16 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
-                consider(b, f, e0 + k);
+            for (int k = 0; k < kPer; ++k) {
+                float v;
+                if constexpr (DT == GG_DTYPE_F32) {
+                    v = __uint_as_float(w[k]);
+                } else {
+                    const uint16_t h = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
+                    v = DT == GG_DTYPE_BF16 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
+                }
+                if (v > b.v) b = ArgBest{v, e0 + k};
             }
+        } else if (e0 < end) {
+            by_element(e0);
         }
     }
+    if (first + kIters * 64 * kPer < end && lane == 0) by_element(first + kIters * 64 * kPer);
+    return b;
 }
 
-__global__ void __launch_bounds__(kThreads) greedy_segment_kernel(
-    const void* __restrict__ logits, gg_dtype_t dt, int R, int V, int nseg, int vec_ok,
-    const int32_t* __restrict__ n_drafts, float2* __restrict__ ws) {
-    const int row = blockIdx.y;  // b*R + j
+// One wave per 4096-element segment. A 256-thread block per segment had two loads in flight
+// per thread and spent most of its life in the reduction: 32 x 5 rows of 128256 bf16 logits
+// (41 MB) 15.4 -> 10.5 us, 128 x 6 rows (197 MB) 57 -> 34 us (5.8 TB/s).
+template <gg_dtype_t DT>
+__global__ void __launch_bounds__(kThreads) greedy_segment_kernel(const void* __restrict__ logits, int rows, int R, int V,
+                                                                  int nseg, const int32_t* __restrict__ n_drafts,
+                                                                  float2* __restrict__ ws) {
+    const int w = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);  // row * nseg + segment
+    const int row = __builtin_amdgcn_readfirstlane(w / nseg), seg = __builtin_amdgcn_readfirstlane(w % nseg);
+    if (row >= rows) return;
     const int b = row / R, j = row % R;
     const int nb = n_drafts[b];
     if (j > (nb < 0 ? 0 : nb)) return;  // rows 0..n, n clamped as the decide kernel clamps it
-    const int seg = blockIdx.x;
-    const int base = seg * kSeg;
-    ArgBest best{-INFINITY, kNone};
-    const size_t eb = dtype_bytes(dt);
-    const void* rowp = (const uint8_t*)logits + (size_t)row * V * eb;
-    if (vec_ok) {
-        if (dt == GG_DTYPE_F32) scan_vec<GG_DTYPE_F32>(best, rowp, base, V);
-        else if (dt == GG_DTYPE_BF16) scan_vec<GG_DTYPE_BF16>(best, rowp, base, V);
-        else scan_vec<GG_DTYPE_F16>(best, rowp, base, V);
-    } else {
-        const int end = min(base + kSeg, V);
-        for (int e = base + threadIdx.x; e < end; e += kThreads) consider(best, load_as_f32(rowp, dt, e), e);
-    }
-    best = wave_best(best);
-    __shared__ ArgBest sb[kThreads / 64];
-    const int wv = threadIdx.x / 64;
-    if ((threadIdx.x & 63) == 0) sb[wv] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        ArgBest r = sb[0];
-        for (int w = 1; w < kThreads / 64; ++w) {
-            ArgBest o = sb[w];
-            if (o.i != kNone && (r.i == kNone || o.v > r.v || (o.v == r.v && o.i < r.i))) r = o;
-        }
-        ws[(size_t)row * nseg + seg] = make_float2(r.v, __int_as_float(r.i));
-    }
+    const void* rowp = (const uint8_t*)logits + (size_t)row * V * dtype_bytes(DT);
+    const ArgBest best = wave_best(scan_segment<DT>(rowp, seg * kSeg, min(seg * kSeg + kSeg, V)));
+    if ((threadIdx.x & 63) == 0) ws[(size_t)row * nseg + seg] = make_float2(best.v, __int_as_float(best.i));
 }
 
 // Lane group of g = 2^ceil(log2 nseg) lanes per row (lane s of a group reads segment s,
@@ -176,10 +179,14 @@ gg_status_t launch_accept_greedy(const void* logits, gg_dtype_t dt, int num_seqs
     const int R = max_drafts + 1;
     if (R > kMaxRows) return fail(GG_ERR_INVALID, "accept_greedy: more than 64 drafts per sequence");
     const int nseg = (vocab + kSeg - 1) / kSeg;
-    const size_t eb = dtype_bytes(dt);
-    const int vec_ok = ((vocab * eb) % 16 == 0) && (((uintptr_t)logits) % 16 == 0);
-    greedy_segment_kernel<<<dim3(nseg, num_seqs * R), kThreads, 0, s>>>(logits, dt, R, vocab, nseg,
-                                                                       vec_ok, n_drafts, (float2*)ws);
+    const int rows = num_seqs * R;
+    const unsigned grid = (unsigned)(((long long)rows * nseg + kThreads / 64 - 1) / (kThreads / 64));
+    float2* seg = (float2*)ws;
+    switch (dt) {
+        case GG_DTYPE_F32: greedy_segment_kernel<GG_DTYPE_F32><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg); break;
+        case GG_DTYPE_BF16: greedy_segment_kernel<GG_DTYPE_BF16><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg); break;
+        default: greedy_segment_kernel<GG_DTYPE_F16><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg); break;
+    }
     greedy_decide_kernel<<<num_seqs, kDecideThreads, 0, s>>>(logits, dt, max_drafts, vocab, nseg, drafts,
                                                  n_drafts, (const float2*)ws, out_acc, out_tok);
     return check_hip(hipGetLastError(), "accept_greedy launch");
