@@ -12,6 +12,7 @@
 // Tie rule: first index of the maximum. NaN never wins; a NaN at element 0 makes
 // the row's argmax 0 (the reference scans with `>` from element 0).
 #include "gg_common.h"
+#include "gg_draw.h"
 
 namespace gg {
 namespace {
@@ -114,15 +115,21 @@ __global__ void __launch_bounds__(kThreads) greedy_segment_kernel(const void* __
 // previous row's decision, took 13 us for nine rows.)
 constexpr int kDecideThreads = 512;
 constexpr int kMaxRows = 65;  // rows per sequence: max_drafts + 1, max_drafts <= 64 (checked by the ABI)
+// DRAW: the sequence's draw is set up here too (its bonus row when every draft was accepted,
+// none otherwise): the row's maximum is at hand, and the draw needs no launch for it.
+template <bool DRAW>
 __global__ void __launch_bounds__(kDecideThreads) greedy_decide_kernel(
     const void* __restrict__ logits, gg_dtype_t dt, int K, int V, int nseg,
     const int32_t* __restrict__ drafts, const int32_t* __restrict__ n_drafts,
-    const float2* __restrict__ ws, int32_t* __restrict__ out_acc, int32_t* __restrict__ out_tok) {
+    const float2* __restrict__ ws, int32_t* __restrict__ out_acc, int32_t* __restrict__ out_tok,
+    fd::DrawParams P, int force_exact) {
     const int b = blockIdx.x;
     const int R = K + 1;
     int n = n_drafts[b];
     n = n < 0 ? 0 : (n > K ? K : n);
     __shared__ int s_am[kMaxRows];
+    __shared__ ArgBest s_last;  // row n's first maximum
+    __shared__ int s_draw;
     int g = 1;
     while (g < nseg && g < 64) g <<= 1;
     const int per_pass = kDecideThreads / g;
@@ -150,6 +157,7 @@ __global__ void __launch_bounds__(kDecideThreads) greedy_decide_kernel(
             }
         }
         if (live && sl == 0) s_am[j] = (first != first || best.i == kNone) ? 0 : best.i;
+        if (DRAW && j == n && sl == 0) s_last = best;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -163,6 +171,18 @@ __global__ void __launch_bounds__(kDecideThreads) greedy_decide_kernel(
         }
         out_acc[b] = accepted;
         out_tok[b] = token;
+        if constexpr (DRAW) {
+            s_draw = accepted == n;
+            fd::prep_row(P, b, accepted == n ? n : -1, -1, s_last.v, s_last.i != kNone, 0ull, 0.0, force_exact);
+        }
+    }
+    if constexpr (DRAW) {
+        __syncthreads();
+        if (!s_draw || !P.filtered) return;
+        for (int i = threadIdx.x; i < fd::kBins; i += kDecideThreads) {
+            P.hcnt[(size_t)b * fd::kBins + i] = 0;
+            if (!P.top_list) P.hmass[(size_t)b * fd::kBins + i] = 0.0;
+        }
     }
 }
 
@@ -175,7 +195,8 @@ size_t greedy_workspace_bytes(int num_seqs, int max_drafts, int vocab) {
 
 gg_status_t launch_accept_greedy(const void* logits, gg_dtype_t dt, int num_seqs, int max_drafts,
                                  int vocab, const int32_t* drafts, const int32_t* n_drafts,
-                                 int32_t* out_acc, int32_t* out_tok, void* ws, hipStream_t s) {
+                                 int32_t* out_acc, int32_t* out_tok, void* ws, hipStream_t s,
+                                 const fd::DrawParams* draw, bool force_exact) {
     const int R = max_drafts + 1;
     if (R > kMaxRows) return fail(GG_ERR_INVALID, "accept_greedy: more than 64 drafts per sequence");
     const int nseg = (vocab + kSeg - 1) / kSeg;
@@ -187,8 +208,12 @@ gg_status_t launch_accept_greedy(const void* logits, gg_dtype_t dt, int num_seqs
         case GG_DTYPE_BF16: greedy_segment_kernel<GG_DTYPE_BF16><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg); break;
         default: greedy_segment_kernel<GG_DTYPE_F16><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg); break;
     }
-    greedy_decide_kernel<<<num_seqs, kDecideThreads, 0, s>>>(logits, dt, max_drafts, vocab, nseg, drafts,
-                                                 n_drafts, (const float2*)ws, out_acc, out_tok);
+    if (draw)
+        greedy_decide_kernel<true><<<num_seqs, kDecideThreads, 0, s>>>(logits, dt, max_drafts, vocab, nseg, drafts, n_drafts,
+                                                                      seg, out_acc, out_tok, *draw, force_exact);
+    else
+        greedy_decide_kernel<false><<<num_seqs, kDecideThreads, 0, s>>>(logits, dt, max_drafts, vocab, nseg, drafts, n_drafts,
+                                                                       seg, out_acc, out_tok, fd::DrawParams{}, 0);
     return check_hip(hipGetLastError(), "accept_greedy launch");
 }
 

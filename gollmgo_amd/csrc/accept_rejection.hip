@@ -1192,9 +1192,7 @@ __device__ SeqPlan decide_seq(const DecideIn& in, int b) {
 // sequence's draw up itself (fd::prep_row), so the draw needs no launch for it.
 template <gg_dtype_t DT>
 __global__ void __launch_bounds__(64) rej_decide_kernel(DecideIn din, int32_t* __restrict__ out_acc,
-                                                        int* __restrict__ spec_row, int* __restrict__ spec_x,
-                                                        unsigned long long* __restrict__ spec_key,
-                                                        double* __restrict__ spec_s, fd::DrawParams P) {
+                                                        fd::DrawParams P) {
     const int b = blockIdx.x;
     const SeqPlan p = decide_seq<DT>(din, b);
     double sest = 0.0;
@@ -1203,10 +1201,7 @@ __global__ void __launch_bounds__(64) rej_decide_kernel(DecideIn din, int32_t* _
     if (p.d.residual && din.dprobs && !din.use_topp && finite_f(fm))  // uniform across the wave
         sest = gg_u128_to_double(row_z_wave(din.seg_max, din.seg_e, frow, din.nseg, fm, din.inv_t)) * 0x1p-70;
     if (threadIdx.x == 0) {
-        spec_s[b] = sest;
         out_acc[b] = p.d.accepted;
-        spec_row[b] = p.d.row;
-        spec_x[b] = p.d.residual ? din.drafts[(size_t)b * din.K + p.d.row] : -1;
         unsigned long long key = 0;
         double vlo = 0.0, vhi = 0.0;
         if (din.use_topp) {
@@ -1223,7 +1218,6 @@ __global__ void __launch_bounds__(64) rej_decide_kernel(DecideIn din, int32_t* _
                     key = ((unsigned long long)st.lam << 32) | (unsigned long long)(~(unsigned int)st.idx_cut);
             }
         }
-        spec_key[b] = key;
         const int x = p.d.residual ? din.drafts[(size_t)b * din.K + p.d.row] : -1;
         fd::prep_row(P, b, p.d.row, x, fm, fm > -INFINITY, P.hint_mode ? key : 0ull, x >= 0 ? sest : 0.0, 0,
                      P.hint_mode ? vlo : 0.0, P.hint_mode ? vhi : 0.0);
@@ -1237,10 +1231,6 @@ static int rej_nseg(int vocab) { return (vocab + kSegElems - 1) / kSegElems; }
 struct RejWs {
     float* seg_max;
     u64* seg_e;
-    int* spec_row;     // the final draw's row per sequence
-    int* spec_x;       // the rejected draft of a residual draw, -1 for a plain draw
-    unsigned long long* spec_key;  // top-p: the final row's fixed-point nucleus cut element
-    double* spec_s;                // dense residual draws: the row's fixed-point total (0: none)
     void* draw;        // the final draw's own workspace (launch_final_draw)
     RowStats* stats;   // top-p: exact nucleus statistics of flagged rows
     u64* seg_hist;     // top-p: coarse histogram per (row, segment)
@@ -1269,10 +1259,6 @@ static RejWs rej_layout(void* base, int num_seqs, int max_drafts, int vocab, boo
     };
     w.seg_max = (float*)take(rows * nseg * sizeof(float));
     w.seg_e = (u64*)take(rows * nseg * sizeof(u64));
-    w.spec_row = (int*)take((size_t)num_seqs * sizeof(int));
-    w.spec_x = (int*)take((size_t)num_seqs * sizeof(int));
-    w.spec_key = (unsigned long long*)take((size_t)num_seqs * sizeof(unsigned long long));
-    w.spec_s = (double*)take((size_t)num_seqs * sizeof(double));
     w.draw = take(final_draw_workspace_bytes(num_seqs, vocab));
     if (topp) {
         w.stats = (RowStats*)take(rows * sizeof(RowStats));
@@ -1326,14 +1312,9 @@ gg_status_t launch_accept_rejection(const void* logits, gg_dtype_t dt, const flo
     d.top_p = (double)top_p;
     d.uniforms_f32 = uniforms;
     d.draft_probs = q;
-    d.spec_row = w.spec_row;
-    d.spec_x = w.spec_x;
-    d.spec_key = w.spec_key;
-    d.spec_s = w.spec_s;
-    d.seg_max = w.seg_max;
-    d.nseg_max = nseg;
+    d.spec_key = true;
+    d.spec_s = true;
     d.out_tok = out_tok;
-    d.prepped = true;  // rej_decide_kernel sets each sequence's draw up
     const fd::DrawParams P = fd::final_draw_params(d, w.draw);
 #define GG_REJ(DTV)                                                                                          \
     if (use_topp) {                                                                                          \
@@ -1357,7 +1338,7 @@ gg_status_t launch_accept_rejection(const void* logits, gg_dtype_t dt, const flo
                                                                              w.seg_e, nullptr, nullptr,      \
                                                                              nullptr);                       \
     }                                                                                                        \
-    rej_decide_kernel<DTV><<<num_seqs, 64, 0, s>>>(din, out_acc, w.spec_row, w.spec_x, w.spec_key, w.spec_s, P);
+    rej_decide_kernel<DTV><<<num_seqs, 64, 0, s>>>(din, out_acc, P);
     switch (dt) {
         case GG_DTYPE_F32: GG_REJ(GG_DTYPE_F32) break;
         case GG_DTYPE_BF16: GG_REJ(GG_DTYPE_BF16) break;

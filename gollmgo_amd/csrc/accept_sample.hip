@@ -26,21 +26,25 @@
 // then index asc, NaN last; exp is gg_exp64 (gg_exp64.h), identical on host and device.
 //
 // Launches after the acceptance has decided which row of each sequence is drawn from:
-//   prep   (B blocks)       : which sequences draw, from which row; the row max from the
-//                             acceptance's segment maxima (the rejection acceptance's
-//                             decide kernel does this itself, fd::prep_row).
+//   (prep)                  : which sequences draw, from which row, and the row max: set up by
+//                             the acceptance's decide kernel (fd::prep_row).
 //   pass   (segments x B)   : e_i = exp(l_i/T - m) per element, segment sums, NaN/+inf
 //                             check; with top-k or top-p the coarse histograms (count and
 //                             mass per 1/64-nat slice below the row max), or, with the
 //                             caller's hint of the nucleus cut, the hinted bins' elements
 //                             and the mass above them; for a dense residual with an
-//                             estimate of its total, the residual's sums.
+//                             estimate of its total, the residual's sums. Top-k of at most
+//                             kTopK counts only: its elements' masses are summed later.
 //   select (B, top-k/p only): from the histograms, the crossing bin (select1) and its
 //                             elements (gather), unless hinted; then the top-k threshold
 //                             and the nucleus cut in LDS (select2), which draws itself
 //                             when no kept launch follows.
 //   kept   (segments x B)   : the draw's weight per segment (kept e, or the residual).
 //   draw   (B)              : the segment and then the element where u * total falls.
+//   top-k of at most kTopK  : after the pass, the elements from the top bin down to the
+//                             threshold bin (topk_gather, which finds that bin itself), then
+//                             threshold, nucleus and draw over that list in one block
+//                             (topk_draw): no further pass over the row.
 //   exact  (a few blocks)   : the literal rule for the rows flagged on the way.
 #include "gg_common.h"
 #include "gg_exp64.h"
@@ -56,11 +60,13 @@ using namespace fd;
 constexpr int kSeg = 8192;        // elements per block of the pass and kept launches
 constexpr int kSegThreads = 512;
 constexpr int kCap = 4096;        // items of one bin the select launch can gather
+constexpr int kTopK = 1024;       // largest top-k drawn from one list
+constexpr int kTopCap = kCap + kTopK;  // its list: the threshold bin, and fewer than kTopK elements above
+constexpr int kTopThreads = 512;
+constexpr int kTopSmall = 2 * kTopThreads;  // longest list ranked by comparing all pairs
 constexpr int kRowThreads = 1024;
 constexpr int kChunk = 4096;      // exact path: bitonic sort entries held in LDS at once
 constexpr int kExactSlots = 4;    // exact path: workgroups (each with its own scratch)
-constexpr int kGreedySeg = 4096;  // accept_greedy.hip's segment length
-constexpr int kNone = 0x7fffffff; // accept_greedy.hip's "no element" index
 
 
 
@@ -90,7 +96,7 @@ Layout layout(int B, int V) {
     L.segep = o;   o = align256(o + (size_t)B * nseg * sizeof(double));
     L.segqp = o;   o = align256(o + (size_t)B * nseg * sizeof(double));
     L.ncand = o;   o = align256(o + (size_t)B * sizeof(int));
-    L.cand = o;    o = align256(o + (size_t)B * kCap * sizeof(unsigned long long));
+    L.cand = o;    o = align256(o + (size_t)B * kTopCap * sizeof(unsigned long long));
     L.vpad = ((size_t)V + 63) & ~(size_t)63;
     size_t np = kChunk;
     while (np < (size_t)V) np <<= 1;
@@ -113,11 +119,6 @@ __device__ __forceinline__ unsigned long long comp_key(uint32_t key, int idx) {
 }
 __device__ __forceinline__ int comp_index(unsigned long long c) { return (int)(~(uint32_t)c); }
 
-
-__device__ __forceinline__ int clamp_n(const int32_t* n_drafts, int b, int K) {
-    const int n = n_drafts[b];
-    return n < 0 ? 0 : (n > K ? K : n);
-}
 
 __device__ __forceinline__ double exp_term(float l, double inv_t, double m) {
     if (l == -INFINITY) return 0.0;
@@ -282,63 +283,6 @@ __device__ uint32_t block_excl_scan_u32(uint32_t v, uint32_t* sh, uint32_t* tota
     return before + inc - v;
 }
 
-// ------------------------------------------------------------------------ prep
-
-// Sequence b draws from row spec_row[b] (-1: no draw), residual after draft spec_x[b]
-// (-1: plain) — or, for the greedy acceptance, from row n when all n drafts were accepted.
-// The row max comes from the acceptance's segment maxima: the greedy (value, index) pairs
-// of 4096-element segments (gws), or the rejection's finite maxima of 8192-element
-// segments (seg_max).
-__global__ void __launch_bounds__(256) sample_prep_kernel(
-    DrawParams P, const float2* __restrict__ gws, const float* __restrict__ seg_max, int nseg_m,
-    const int32_t* __restrict__ n_drafts, const int32_t* __restrict__ acc, const int* __restrict__ spec_row,
-    const int* __restrict__ spec_x, const unsigned long long* __restrict__ spec_key,
-    const double* __restrict__ spec_s, int force_exact) {
-    const int b = blockIdx.x;
-    const int K = P.K, R = K + 1;
-    int row, x = -1;
-    if (gws) {
-        const int n = clamp_n(n_drafts, b, K);
-        row = acc[b] == n ? n : -1;
-    } else {
-        row = spec_row[b];
-        x = spec_x[b];
-    }
-    if (row < 0) {
-        if (threadIdx.x == 0) P.state[b] = ST_NONE;
-        return;
-    }
-    // top-p alone with a hint of the cut element: the pass gathers its bin itself
-    const unsigned long long hint = P.hint_mode ? spec_key[b] : 0ull;
-    if (P.filtered && !P.hint_mode)
-        for (int i = threadIdx.x; i < kBins; i += blockDim.x) {
-            P.hcnt[(size_t)b * kBins + i] = 0;
-            P.hmass[(size_t)b * kBins + i] = 0.0;
-        }
-    if (threadIdx.x < 64) {
-        float mx = -INFINITY;
-        int any = 0;
-        for (int s = threadIdx.x; s < nseg_m; s += 64) {
-            if (gws) {
-                const float2 p = gws[((size_t)b * R + row) * nseg_m + s];
-                if (__float_as_int(p.y) != kNone) {
-                    any = 1;
-                    mx = fmaxf(mx, p.x);
-                }
-            } else {
-                const float v = seg_max[((size_t)b * R + row) * nseg_m + s];
-                if (v > -INFINITY) any = 1;
-                mx = fmaxf(mx, v);
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            mx = fmaxf(mx, __shfl_xor(mx, o));
-            any |= __shfl_xor(any, o);
-        }
-        if (threadIdx.x == 0) prep_row(P, b, row, x, mx, any != 0, hint, spec_s && x >= 0 ? spec_s[b] : 0.0, force_exact);
-    }
-}
-
 // ------------------------------------------------------------------------ pass
 
 // The draw itself, by one block of NT threads: the segment where u * total falls (sums
@@ -429,6 +373,7 @@ __device__ void draw_in_block(const DrawParams& P, int b, const RowInfo& ri, con
 // sum, the NaN / +inf check, and with top-k / top-p the coarse histograms.
 // Stage the elements of one coarse bin found by a block in LDS, one counter update per wave.
 constexpr int kBlockCap = 2048;  // a segment's hits staged in LDS; more: the row goes exact
+template <int CAP = kBlockCap>
 __device__ __forceinline__ void stage_hit(bool hit, unsigned long long comp, int* s_cnt, unsigned long long* s_buf) {
     const int lane = threadIdx.x & 63;
     const unsigned long long mask = __ballot(hit);
@@ -439,21 +384,22 @@ __device__ __forceinline__ void stage_hit(bool hit, unsigned long long comp, int
         base = __shfl(base, leader);
         if (hit) {
             const int slot = base + __popcll(mask & ((1ull << lane) - 1ull));
-            if (slot < kBlockCap) s_buf[slot] = comp;
+            if (slot < CAP) s_buf[slot] = comp;
         }
     }
 }
 // The staged elements appended to the sequence's list (one global update per block; an
-// overflow forces the count past kCap, so the row goes exact).
+// overflow forces the count past the list's capacity, so the row goes exact).
+template <int CAP = kBlockCap, int LIST = kCap>
 __device__ __forceinline__ void flush_hits(const DrawParams& P, int b, int* s_cnt, int* s_base,
                                            const unsigned long long* s_buf) {
     __syncthreads();
     const int n = *s_cnt;
-    if (threadIdx.x == 0 && n > 0) *s_base = atomicAdd(&P.ncand[b], n > kBlockCap ? kCap + 1 : n);
+    if (threadIdx.x == 0 && n > 0) *s_base = atomicAdd(&P.ncand[b], n > CAP ? LIST + 1 : n);
     __syncthreads();
-    if (n > 0 && n <= kBlockCap)
+    if (n > 0 && n <= CAP)
         for (int i = threadIdx.x; i < n; i += blockDim.x)
-            if (*s_base + i < kCap) P.cand[(size_t)b * kCap + *s_base + i] = s_buf[i];
+            if (*s_base + i < LIST) P.cand[(size_t)b * LIST + *s_base + i] = s_buf[i];
 }
 
 // Per (segment, sequence): e of every element (the parallel exponential), the segment's
@@ -566,6 +512,41 @@ __global__ void __launch_bounds__(kSegThreads) sample_pass_kernel(DrawParams P) 
             if (want_mass && s_mass[i] != 0.0) unsafeAtomicAdd(&P.hmass[(size_t)b * kBins + i], s_mass[i]);
         }
     }
+}
+
+// The pass of a top-k of at most kTopK: NaN / +inf check and the count histogram alone.
+template <gg_dtype_t DT>
+__global__ void __launch_bounds__(kSegThreads) sample_count_kernel(DrawParams P) {
+    const int b = blockIdx.y, seg = blockIdx.x;
+    if (P.state[b] != ST_DRAW) return;
+    __shared__ uint32_t s_cnt[kBins];
+    const double m = P.info[b].m, inv_t = P.inv_t;
+    const void* row = drawn_row(P, b, P.info[b].row);
+    constexpr int kIt = kSeg / 8 / kSegThreads;
+    float x[kIt][8];
+#pragma unroll
+    for (int i = 0; i < kIt; ++i) load8<DT>(row, P.V, seg * kSeg + (i * kSegThreads + threadIdx.x) * 8, P.vec, x[i]);
+    for (int i = threadIdx.x; i < kBins / 4; i += kSegThreads) ((uint4*)s_cnt)[i] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    int bad = 0;
+#pragma unroll
+    for (int i = 0; i < kIt; ++i) {
+        const int e0 = seg * kSeg + (i * kSegThreads + threadIdx.x) * 8;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float l = x[i][k];
+            if (e0 + k < P.V) {
+                if (l != l || l == INFINITY) bad = 1;
+                else atomicAdd(&s_cnt[bin_of(l, inv_t, m)], 1u);
+            }
+        }
+    }
+    if (__syncthreads_or(bad)) {
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+    for (int i = threadIdx.x; i < kBins; i += kSegThreads)
+        if (s_cnt[i]) atomicAdd(&P.hcnt[(size_t)b * kBins + i], s_cnt[i]);
 }
 
 // ---------------------------------------------------------------------- select
@@ -1213,6 +1194,296 @@ __global__ void __launch_bounds__(kSegThreads) sample_draw_kernel(DrawParams P) 
     draw_seq<DT, kSegThreads>(P, b, P.info[b], nullptr, s_tab);
 }
 
+// ------------------------------------------------------- top-k of at most kTopK
+//
+// The general path summed the mass of every bin, gathered the threshold bin and then, where the
+// nucleus ended above it, read the row again in one block (50 µs of 120) and once more for the
+// kept sums. At most kTopK elements lie above the threshold bin, so the list down to that bin
+// holds everything the threshold, the nucleus and the draw need. 32 sequences of 128256 bf16
+// logits (25 drawn rows), top-k 50 and top-p 0.95: the draw's launches 95 -> 30 µs (count 8.7,
+// gather 8.4, draw 9.0, exact check 3.8), bound by their latency (6.4 MB each). kTopK bounds the
+// list's LDS; larger k take the general path.
+
+// Per (segment, sequence): the bin where the count from the top first reaches k (every
+// block finds it from the row's histogram, next to its own loads in flight), and the
+// segment's elements from that bin up appended to the sequence's list.
+constexpr int kTopBlockCap = kBlockCap + kTopK;  // a segment's hits staged in LDS
+template <gg_dtype_t DT>
+__global__ void __launch_bounds__(kSegThreads) sample_topk_gather_kernel(DrawParams P) {
+    const int b = blockIdx.y, seg = blockIdx.x;
+    if (P.state[b] != ST_DRAW) return;
+    __shared__ unsigned long long s_buf[kTopBlockCap];
+    __shared__ uint32_t s_red[16];
+    __shared__ int s_cnt, s_base, s_bin;
+    const double m = P.info[b].m;
+    const void* row = drawn_row(P, b, P.info[b].row);
+    constexpr int kIt = kSeg / 8 / kSegThreads;
+    constexpr int kPer = kBins / kSegThreads;  // bins per thread, from the top
+    static_assert(kPer == 8, "two 16-byte loads of counts per thread");
+    float x[kIt][8];
+#pragma unroll
+    for (int i = 0; i < kIt; ++i) load8<DT>(row, P.V, seg * kSeg + (i * kSegThreads + threadIdx.x) * 8, P.vec, x[i]);
+    const uint4* hp = (const uint4*)(P.hcnt + (size_t)b * kBins + kBins - kPer * (threadIdx.x + 1));
+    const uint4 h0 = hp[0], h1 = hp[1];
+    const uint32_t c[kPer] = {h1.w, h1.z, h1.y, h1.x, h0.w, h0.z, h0.y, h0.x};  // descending bins
+    uint32_t sum = 0, total;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) sum += c[q];
+    if (threadIdx.x == 0) {
+        s_cnt = 0;
+        s_bin = -1;
+    }
+    uint32_t run = block_excl_scan_u32(sum, s_red, &total);  // (its barriers publish s_bin)
+    const uint32_t k = (uint32_t)P.top_k;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        if (run < k && run + c[q] >= k) s_bin = kBins - 1 - (kPer * (int)threadIdx.x + q);
+        run += c[q];
+    }
+    __syncthreads();
+    const int cbin = s_bin;
+    if (cbin < 0) {  // fewer counted elements than k
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < kIt; ++i) {
+        const int e0 = seg * kSeg + (i * kSegThreads + threadIdx.x) * 8;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int e = e0 + q;
+            stage_hit<kTopBlockCap>(e < P.V && bin_of(x[i][q], P.inv_t, m) >= cbin, comp_key(order_key(x[i][q]), e),
+                                    &s_cnt, s_buf);
+        }
+    }
+    flush_hits<kTopBlockCap, kTopCap>(P, b, &s_cnt, &s_base, s_buf);
+}
+
+// One block per sequence: the top-k threshold, the nucleus cut and the draw over the gathered
+// list. Lists up to kTopSmall are ranked by comparing all pairs (two elements per thread
+// against LDS broadcasts), first by (value desc, index asc) for the rule's two cuts, then the
+// kept ones by index for the draw; longer ones (a crowded threshold bin) take the radix
+// descents and the segment draw of the general select. Margins as there.
+template <gg_dtype_t DT>
+__global__ void __launch_bounds__(kTopThreads) sample_topk_draw_kernel(DrawParams P) {
+    const int b = blockIdx.x;
+    if (P.state[b] != ST_DRAW) return;
+    __shared__ unsigned long long s_comp[kTopCap];
+    __shared__ double s_e[kTopCap];
+    __shared__ double s_rank[kTopSmall];
+    __shared__ unsigned long long s_key[kTopSmall];
+    __shared__ double s_h[257];
+    __shared__ double s_red[16];
+    __shared__ unsigned long long s_u[16];
+    __shared__ double s_tab[64];
+    __shared__ double s_segk[64];
+    __shared__ int s_i, s_tok, s_bad;
+    __shared__ double s_cutmass;
+    RowInfo ri = P.info[b];
+    const double tau = P.tau, inv_t = P.inv_t, m = ri.m;
+    const int k = P.top_k, ng = P.ncand[b];
+    if (ng > kTopCap || ng < k) {  // a crowded bin: the literal rule decides
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+    for (int i = threadIdx.x; i < ng; i += kTopThreads) {
+        const unsigned long long c = P.cand[(size_t)b * kTopCap + i];
+        s_comp[i] = c;
+        s_e[i] = exp_term(key_value((uint32_t)(c >> 32)), inv_t, m);
+    }
+    if (threadIdx.x == 0) {
+        s_i = -1;
+        s_tok = -1;
+        s_bad = 0;
+    }
+    __syncthreads();
+    const bool small = ng <= kTopSmall;
+    unsigned long long tk = 0, cut = 0;
+    double tot = 0.0;
+    bool ok = true;
+    constexpr int kOwn = kTopSmall / kTopThreads;
+    if (small) {
+        // Rank of the thread's elements in (value desc, index asc) order.
+        unsigned long long mine[kOwn];
+        int rank[kOwn];
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) {
+            const int i = threadIdx.x * kOwn + q;
+            mine[q] = i < ng ? s_comp[i] : 0ull;
+            rank[q] = 0;
+        }
+        if ((int)(threadIdx.x & ~63u) * kOwn < ng)  // (whole waves past the list skip)
+            for (int t = 0; t < ng; ++t) {
+                const unsigned long long c = s_comp[t];
+#pragma unroll
+                for (int q = 0; q < kOwn; ++q) rank[q] += c > mine[q];
+            }
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) {
+            const int i = threadIdx.x * kOwn + q;
+            if (i < ng) {
+                s_rank[rank[q]] = s_e[i];
+                s_key[rank[q]] = mine[q];
+            }
+        }
+        __syncthreads();
+        tk = s_key[k - 1];
+        // Running mass in that order, the top k alone.
+        double v[kOwn], sum = 0.0;
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) {
+            const int i = threadIdx.x * kOwn + q;
+            v[q] = i < k ? s_rank[i] : 0.0;
+            sum += v[q];
+        }
+        double S;
+        const double before = block_excl_scan(sum, s_red, &S);
+        double run = before;
+        cut = tk;
+        tot = S;
+        if (P.use_p) {
+            // The first element whose running mass reaches p * S. (Rounding may let two threads
+            // see the crossing: the later one wins here, and its margins fail.)
+            const double pS = P.top_p * S;
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) {
+                if (run < pS && run + v[q] >= pS) atomicMax(&s_i, (int)threadIdx.x * kOwn + q);
+                run += v[q];
+            }
+            __syncthreads();
+            const int ci = s_i;
+            if (ci < 0) {  // uniform
+                if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+                return;
+            }
+            if (ci / kOwn == (int)threadIdx.x) {
+                double A = before;
+#pragma unroll
+                for (int q = 0; q < kOwn; ++q)
+                    if ((int)threadIdx.x * kOwn + q < ci) A += v[q];
+                const double ec = s_rank[ci];
+                bool fine = (pS - A) > tau * S && (A + ec - pS) > tau * S;
+                // An element after the cut with the same probability but another value would
+                // come first in the rule's order if its index is lower.
+                if (ci + 1 < k && s_rank[ci + 1] == ec && (s_key[ci + 1] >> 32) != (s_key[ci] >> 32)) fine = false;
+                s_cutmass = A + ec;
+                if (!fine) s_bad = 1;
+            }
+            __syncthreads();
+            cut = s_key[ci];
+            tot = s_cutmass;
+            ok = !s_bad;
+        }
+        if (!ok) {
+            if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+            return;
+        }
+        // The draw: the kept elements in index order (at most k of them).
+        const double u = uniform_of(P, b);
+        if (!(u >= tau && u < 1.0 - tau)) {
+            if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+            return;
+        }
+        __syncthreads();  // (s_rank and s_key are rewritten)
+        unsigned idx[kOwn];
+        int pos[kOwn];
+        bool kept[kOwn];
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) {
+            const int i = threadIdx.x * kOwn + q;
+            kept[q] = i < ng && mine[q] >= cut;
+            idx[q] = (unsigned)comp_index(mine[q]);
+            pos[q] = 0;
+        }
+        if ((int)(threadIdx.x & ~63u) * kOwn < ng)
+            for (int t = 0; t < ng; ++t) {
+                const unsigned long long c = s_comp[t];
+#pragma unroll
+                for (int q = 0; q < kOwn; ++q) pos[q] += c >= cut && (unsigned)comp_index(c) < idx[q];
+            }
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) s_rank[threadIdx.x * kOwn + q] = 0.0;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q)
+            if (kept[q]) {
+                s_rank[pos[q]] = s_e[threadIdx.x * kOwn + q];
+                s_key[pos[q]] = idx[q];
+            }
+        __syncthreads();
+        sum = 0.0;
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) {
+            v[q] = s_rank[threadIdx.x * kOwn + q];
+            sum += v[q];
+        }
+        double W;
+        run = block_excl_scan(sum, s_red, &W);
+        const double t = u * W, marg = tau * W;
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) {
+            const double nx = run + v[q];
+            if (run <= t && nx > t) {
+                if ((t - run) > marg && (nx - t) > marg) s_tok = (int)s_key[threadIdx.x * kOwn + q];
+                else s_bad = 1;
+            }
+            run = nx;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            if (s_tok >= 0 && !s_bad) P.out_tok[b] = s_tok;
+            else atomicOr(&P.state[b], ST_EXACT);
+        }
+        return;
+    }
+    // A long list: radix descents.
+    load_exp_table(s_tab);
+    double before;
+    const int ck = select_desc(s_comp, s_e, ng, (double)k, false, &before, s_h, s_red, &s_i);
+    if (ck < 0) {
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+    tk = s_comp[ck];
+    double part = 0.0;
+    for (int i = threadIdx.x; i < ng; i += kTopThreads) {
+        if (s_comp[i] >= tk) part += s_e[i];
+        else s_e[i] = 0.0;
+    }
+    const double S = block_sum(part, s_red);
+    cut = tk;
+    tot = S;
+    if (P.use_p) {
+        const double pS = P.top_p * S;
+        const int ci = select_desc(s_comp, s_e, ng, pS, true, &before, s_h, s_red, &s_i);
+        if (ci < 0) {
+            if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+            return;
+        }
+        const unsigned long long cc = s_comp[ci], nb = next_below(s_comp, ng, cc, s_u);
+        const double ec = s_e[ci];
+        bool fine = (pS - before) > tau * S && (before + ec - pS) > tau * S && cc >= tk;
+        if (nb != 0 && nb >= tk && (nb >> 32) != (cc >> 32) &&
+            exp_term(key_value((uint32_t)(nb >> 32)), inv_t, m) == ec)
+            fine = false;
+        if (!fine) {  // uniform
+            if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+            return;
+        }
+        cut = cc;
+        tot = before + ec;
+    }
+    if (threadIdx.x < 64) s_segk[threadIdx.x] = 0.0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < ng; i += kTopThreads)
+        if (s_comp[i] >= cut)
+            atomicAdd(&s_segk[comp_index(s_comp[i]) / kSeg], fast_term(key_value((uint32_t)(s_comp[i] >> 32)), inv_t, m, s_tab));
+    __syncthreads();
+    ri.cut = cut;
+    ri.tot = tot;
+    draw_seq<DT, kTopThreads>(P, b, ri, s_segk, s_tab);
+}
+
 // ----------------------------------------------------------------------- exact
 
 __device__ __forceinline__ bool ent_less(const Ent& a, const Ent& c) {
@@ -1502,7 +1773,8 @@ fd::DrawParams fd::final_draw_params(const FinalDraw& d, void* ws) {
     P.use_p = d.top_p > 0 && d.top_p < 1.0;
     P.filtered = P.use_k || P.use_p;
     P.hint_mode = d.spec_key && P.use_p && !P.use_k;
-    P.kept_launched = (d.draft_probs && (P.filtered || !d.spec_s)) || (P.use_k && P.use_p);
+    P.top_list = P.use_k && d.top_k <= kTopK && !d.draft_probs;
+    P.kept_launched = (d.draft_probs && (P.filtered || !d.spec_s)) || (P.use_k && P.use_p && !P.top_list);
     {
         const size_t eb = dtype_bytes(d.dt);
         P.vec = ((size_t)V * eb % 16 == 0) && ((uintptr_t)d.logits % 16 == 0);
@@ -1535,11 +1807,6 @@ gg_status_t launch_final_draw(const FinalDraw& d, void* ws, hipStream_t s) {
     const Layout L = layout(B, V);
     uint8_t* w = (uint8_t*)ws;
     const DrawParams P = fd::final_draw_params(d, ws);
-    const int force = d.force_exact ? 1 : 0;
-    const int nseg_m = d.greedy_seg ? (V + kGreedySeg - 1) / kGreedySeg : d.nseg_max;
-    if (!d.prepped)
-        sample_prep_kernel<<<B, 256, 0, s>>>(P, d.greedy_seg, d.seg_max, nseg_m, d.n_drafts, d.accepted, d.spec_row,
-                                             d.spec_x, d.spec_key, d.spec_s, force);
     // Without filters the draw takes the pass's segment sums (a dense residual: the kept
     // launch's). With filters: the bin of the cut (select1), its elements and the sums above
     // it (gather) — both done by the pass when the caller hints the cut — then the cut and
@@ -1549,6 +1816,12 @@ gg_status_t launch_final_draw(const FinalDraw& d, void* ws, hipStream_t s) {
     // pass and the draw form its sums.)
     const bool kept = P.kept_launched;
 #define GG_DRAW(DTV)                                                                                 \
+    if (P.top_list) {                                                                                \
+        sample_count_kernel<DTV><<<dim3(P.nseg, B), kSegThreads, 0, s>>>(P);                         \
+        sample_topk_gather_kernel<DTV><<<dim3(P.nseg, B), kSegThreads, 0, s>>>(P);                   \
+        sample_topk_draw_kernel<DTV><<<B, kTopThreads, 0, s>>>(P);                                   \
+        break;                                                                                       \
+    }                                                                                                \
     if (P.hint_mode) sample_pass_kernel<DTV, kPassPre><<<dim3(P.nseg, B), kSegThreads, 0, s>>>(P);   \
     else if (P.filtered) sample_pass_kernel<DTV, kPassHist><<<dim3(P.nseg, B), kSegThreads, 0, s>>>(P); \
     else sample_pass_kernel<DTV, kPassPlain><<<dim3(P.nseg, B), kSegThreads, 0, s>>>(P);             \
@@ -1582,9 +1855,8 @@ gg_status_t launch_accept_greedy_sample(const void* logits, gg_dtype_t dt, int B
                                         int top_k, double top_p, const double* uniforms, unsigned flags,
                                         int32_t* out_acc, int32_t* out_tok, void* ws, hipStream_t s) {
     uint8_t* w = (uint8_t*)ws;
-    gg_status_t st = launch_accept_greedy(logits, dt, B, K, V, drafts, n_drafts, out_acc, out_tok, w, s);
-    if (st != GG_OK) return st;
-    if (temperature <= 1e-9) return GG_OK;  // Sampler.Sample's greedy case (sampling.go:54-56)
+    if (temperature <= 1e-9)  // Sampler.Sample's greedy case (sampling.go:54-56)
+        return launch_accept_greedy(logits, dt, B, K, V, drafts, n_drafts, out_acc, out_tok, w, s);
     FinalDraw d{};
     d.logits = logits;
     d.dt = dt;
@@ -1595,12 +1867,13 @@ gg_status_t launch_accept_greedy_sample(const void* logits, gg_dtype_t dt, int B
     d.top_k = top_k;
     d.top_p = top_p;
     d.uniforms_f64 = uniforms;
-    d.n_drafts = n_drafts;
-    d.accepted = out_acc;
-    d.greedy_seg = (const float2*)w;
-    d.force_exact = (flags & GG_SAMPLE_EXACT) != 0;
     d.out_tok = out_tok;
-    return launch_final_draw(d, w + ((greedy_workspace_bytes(B, K, V) + 255) & ~(size_t)255), s);
+    uint8_t* dw = w + ((greedy_workspace_bytes(B, K, V) + 255) & ~(size_t)255);
+    // The decide kernel sets each sequence's draw up.
+    const fd::DrawParams P = fd::final_draw_params(d, dw);
+    const gg_status_t st = launch_accept_greedy(logits, dt, B, K, V, drafts, n_drafts, out_acc, out_tok, w, s, &P,
+                                                (flags & GG_SAMPLE_EXACT) != 0);
+    return st != GG_OK ? st : launch_final_draw(d, dw, s);
 }
 
 }  // namespace gg

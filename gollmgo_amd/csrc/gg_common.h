@@ -112,10 +112,16 @@ size_t attn_workspace_bytes(const KV* kv, int num_seqs, int rows, int num_q_head
 gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s);
 gg_status_t launch_attn_plan(const AttnArgs& a, hipStream_t s);  // no-op unless LPT
 
+namespace fd {
+struct DrawParams;
+}
+// draw: the sequences whose drafts were all accepted are set up for a draw of their bonus row
+// (fd::prep_row; force_exact: by the literal rule).
 size_t greedy_workspace_bytes(int num_seqs, int max_drafts, int vocab);
 gg_status_t launch_accept_greedy(const void* logits, gg_dtype_t dt, int num_seqs, int max_drafts,
                                  int vocab, const int32_t* drafts, const int32_t* n_drafts,
-                                 int32_t* out_acc, int32_t* out_tok, void* ws, hipStream_t s);
+                                 int32_t* out_acc, int32_t* out_tok, void* ws, hipStream_t s,
+                                 const fd::DrawParams* draw = nullptr, bool force_exact = false);
 
 // The float64 token draw shared by the greedy-with-sampled-bonus and the rejection
 // acceptance (accept_sample.hip): per sequence, a row drawn with Sampler.Sample's rule, or
@@ -130,23 +136,12 @@ struct FinalDraw {
     const double* uniforms_f64;  // uniform of sequence b: uniforms_f64[b], or
     const float* uniforms_f32;   //   uniforms_f32[b * (max_drafts + 1) + max_drafts]
     const float* draft_probs;    // residual draws: [num_seqs][max_drafts][vocab], or null (one-hot)
-    // Which row: either greedy (row n_drafts[b] when accepted[b] == n_drafts[b], the row
-    // maxima from the greedy segment pairs greedy_seg), or given (spec_row[b], -1 = none;
-    // spec_x[b] the rejected draft of a residual draw, -1 = plain; the row maxima from
-    // seg_max [rows][nseg_max], finite maxima of 8192-element segments).
-    const int32_t* n_drafts;
-    const int32_t* accepted;
-    const float2* greedy_seg;
-    const int* spec_row;
-    const int* spec_x;
-    const unsigned long long* spec_key;  // given rows, top-p: (order key << 32 | ~index) of an element
-                                         // at or near the nucleus cut (0: none)
-    const double* spec_s;                // given rows: an estimate of the drawn row's softmax sum
-                                         // within 1e-4 relative (0: none; dense residuals)
-    const float* seg_max;
-    int nseg_max;
-    bool force_exact;
-    bool prepped;                        // the caller set every sequence's row up (fd::prep_row)
+    // Which row, and what is known of it, each sequence's decide kernel sets up in the draw's
+    // workspace (fd::prep_row). spec_key: it may give an element at or near the nucleus cut, or a
+    // range around it (top-p); spec_s: it may give an estimate of the drawn row's softmax sum
+    // within 1e-4 relative (dense residuals).
+    bool spec_key;
+    bool spec_s;
     int32_t* out_tok;
 };
 size_t final_draw_workspace_bytes(int num_seqs, int vocab);

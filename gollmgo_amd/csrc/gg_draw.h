@@ -40,6 +40,7 @@ struct DrawParams {
     double top_p;
     int use_k, use_p, filtered;
     int hint_mode;            // top-p alone with the caller's cut hints: select1 / gather not launched
+    int top_list;             // small top-k: drawn from one list of the elements down to its bin
     int kept_launched;        // the kept launch runs (a row that needs it otherwise goes exact)
     int vec;                  // rows allow 16-byte loads
     int vec_q;                // so do the draft distributions' rows
@@ -140,7 +141,7 @@ __device__ inline void prep_row(const DrawParams& P, int b, int row, int x, floa
     if (ri.kept_pass && !P.kept_launched) st |= ST_EXACT;
     ri.pregather = hint != 0 || range;
     ri.hint = hint;
-    if (split_residual(P, ri)) P.ncand[b] = 0;
+    if (split_residual(P, ri) || P.top_list) P.ncand[b] = 0;
     if (hint != 0) {
         ri.cbin = ri.cbin_lo = bin_of(key_value((uint32_t)(hint >> 32)), P.inv_t, m);
         P.ncand[b] = 0;
