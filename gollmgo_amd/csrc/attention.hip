@@ -234,6 +234,19 @@ gg_status_t launch_append_from_tables(const AttnArgs& a, const KVView& kv, hipSt
     return check_hip(hipGetLastError(), "append launch");
 }
 
+int attn_generic_partition(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks) {
+    // One wave per (row, head, partition): partitions of 64..512 keys, as many as
+    // it takes to reach about 2048 waves (the kernel's time is the longest wave's
+    // chain of 64-key tiles; the merge costs one small launch).
+    const long long waves = (long long)num_seqs * rows * num_q_heads;
+    const long long want = waves > 0 ? (2048 + waves - 1) / waves : 1;
+    const long long keys = (long long)max_blocks * kv->block_size;
+    long long part = (keys + want - 1) / want;
+    part = (part + 63) / 64 * 64;
+    part = part < 64 ? 64 : (part > 512 ? 512 : part);
+    return (int)part;
+}
+
 AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks,
                    int partition_tokens) {
     if (partition_tokens > 0) return {ATTN_SCHED_GRID, partition_tokens};
@@ -242,16 +255,7 @@ AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int ma
     if (sh.full && num_seqs <= kLptMaxSeqs && (long long)num_seqs * kv->num_kv_heads * sh.groups <= (1 << 18))
         return {ATTN_SCHED_LPT, 0};
     if (!attn_mfma_supported(kv, rows, num_q_heads)) {
-        // One wave per (row, head, partition): partitions of 64..512 keys, as many as
-        // it takes to reach about 2048 waves (the kernel's time is the longest wave's
-        // chain of 64-key tiles; the merge costs one small launch).
-        const long long waves = (long long)num_seqs * rows * num_q_heads;
-        const long long want = waves > 0 ? (2048 + waves - 1) / waves : 1;
-        const long long keys = (long long)max_blocks * kv->block_size;
-        long long part = (keys + want - 1) / want;
-        part = (part + 63) / 64 * 64;
-        part = part < 64 ? 64 : (part > 512 ? 512 : part);
-        return {ATTN_SCHED_GRID, (int)part};
+        return {ATTN_SCHED_GRID, attn_generic_partition(kv, num_seqs, rows, num_q_heads, max_blocks)};
     }
     // Longest-first pieces (LPT: long items cut, dispatched longest first, split items merged
     // inside the launch) at every batch the plan kernel can rank. Few items too: against the

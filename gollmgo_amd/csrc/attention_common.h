@@ -158,10 +158,10 @@ constexpr int kLptMaxSeqs = 1024;
 //     the fixed 7/5 of the mean, per call on one box: config-2-shaped bf16 items (slots / 2)
 //     68.2 -> 66.3 µs, config-4-shaped int8 items (slots / 8) 124 -> 112 µs.
 //   - Never shorter than lpt_min_chunks: a cut costs the item's records, their merge and a
-//     second piece start, about 5 µs. At 8 / 12 / 16 chunks of 64 tokens, 24 short int8
-//     sequences (200-900 keys) took 32.2 / 27.2 / 28.3 µs a call and one fp8 sequence of
-//     3000 keys 21.9 / 22.5 / 24.3; at 8 / 12 / 16 chunks of 32 tokens, 16 bf16 sequences of
-//     256-1024 keys took 25.9 / 27.0 / 23.3.
+//     second piece start, about 4 µs. At 8 / 12 chunks of 64 tokens, 24 short int8 sequences
+//     (200-900 keys) took 28.1 / 25.3 µs a call and one fp8 sequence of 3000 keys 18.7 / 19.5;
+//     at 8 / 12 / 16 chunks of 32 tokens, 16 bf16 sequences of 256-1024 keys took 21.7 / 24.3 /
+//     21.1 and four of 1000-3000 keys 28.4 / 24.5 / 25.3.
 constexpr int kLptPieceNum = 2, kLptPieceDen = 1;  // items >= slots
 constexpr int kLptTSpan = 31;
 __host__ __device__ constexpr int lpt_min_chunks(int tok) { return tok == 64 ? 12 : 16; }
@@ -178,6 +178,8 @@ __host__ __device__ constexpr int lpt_pieces(int slots, int num_seqs, int heads)
 // Bound on the partial records: a split item of n > T chunks has at most 2 n / T pieces, so
 // split items have at most 2 C / T <= slots.
 __host__ __device__ constexpr int lpt_records(int slots) { return slots; }
+// Automatic partition of the per-row kernel (tokens).
+int attn_generic_partition(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks);
 AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks,
                    int partition_tokens);
 

@@ -19,6 +19,16 @@
 // Head dims are permuted consistently in K and Q (lane group g4 owns dims
 // 32*g4..32*g4+31), so every K load is a contiguous 32- or 64-byte run.
 //
+// A piece that is not the machine's whole life is bound by its chain of round trips: table
+// entry, block ids, queries, first chunk, then per chunk, then the merges. So a piece's table
+// entry holds everything its workgroup would look up (one load), its first block ids go out
+// next, its queries before its K/V (loads retire in order: the Q staging waits for them alone),
+// the four waves merge four dims per thread, and a split item's records are read two items and
+// four records at a time in 8-byte loads. Against one lookup after the other and element-wise
+// merges, per pass on one box: one fp8 sequence of 3000 keys over 16 layers 363.7 -> 311.9 µs,
+// 16 f16 sequences at head_dim 64 62.6 -> 56.3, 80 bf16 rows per kv head 92.8 -> 74.9, the
+// config-2 / 3 / 4 shapes 132.1 -> 127.2 / 239.4 -> 236.0 / 121.1 -> 113.9.
+//
 // Pool types: BF16 (bf16 MFMA; P split into bf16 hi+lo for two MFMAs so the
 // probabilities keep ~16 bits), F16 (f16 MFMA), FP8-E4M3 and INT8 (decoded in
 // registers to exact f16 values: E4M3 by the gfx950 pk_f16_fp8 conversion, int8
@@ -260,10 +270,10 @@ struct PieceIn {
 };
 
 // A piece: tokens [t0, t_end) of sequence b against kv head kvh, written to partition
-// slot `part` / record `rec` (both < 0: the output), for the query rows from row0 on.
-// Wave-uniform.
+// slot `part` / record `rec` (both < 0: the output), for the query rows from row0 on; ctx
+// and nrows are the sequence's keys and rows. Wave-uniform.
 struct PieceDesc {
-    int b, kvh, t0, t_end, part, rec, row0;
+    int b, kvh, t0, t_end, part, rec, row0, ctx, nrows;
 };
 
 template <gg_dtype_t DT, int TOK, int HD>
@@ -307,9 +317,13 @@ struct PieceIO {
         }
         return l;
     }
-    __device__ static __forceinline__ LaneBlocks chunk_blocks(const AttnArgs& a, const KVView& kv, int b, int t0,
-                                                              int t_end, int ch) {
-        return lane_blocks(kv, fetch_blocks(a, b, t0, ch), t_end);
+    // The block ids of the wave's first two chunks.
+    struct FirstBlocks {
+        RawBlocks r0, r1;
+    };
+    __device__ static __forceinline__ FirstBlocks first_blocks(const AttnArgs& a, const PieceDesc& d) {
+        const int wave_u = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        return FirstBlocks{fetch_blocks(a, d.b, d.t0, wave_u), fetch_blocks(a, d.b, d.t0, wave_u + kWaves)};
     }
     // K rows: lane supplies M index c16 of every tile. Loads are unconditional (missing
     // blocks read block 0); such tokens are always masked in S.
@@ -346,13 +360,12 @@ struct PieceIO {
             rg.v[dt] = *(const typename Geom::VReg*)(base + (size_t)d * kBS * kEB);
         }
     }
-    // Issue the first chunk of piece d (this wave's first chunk is chunk `wave`): the block
-    // ids of its first two chunks, then the first chunk's K rows and V columns.
-    __device__ static __forceinline__ void start(const AttnArgs& a, const KVView& kv, const PieceDesc& d,
+    // Issue the first chunk of piece d (this wave's first chunk is chunk `wave`): its K rows and
+    // V columns, from the block ids read ahead.
+    __device__ static __forceinline__ void start(const KVView& kv, const PieceDesc& d, const FirstBlocks& fb,
                                                  PieceIn<DT, TOK, HD>& in) {
-        const int wave_u = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        in.bl_cur = chunk_blocks(a, kv, d.b, d.t0, d.t_end, wave_u);
-        in.bl_next = chunk_blocks(a, kv, d.b, d.t0, d.t_end, wave_u + kWaves);
+        in.bl_cur = lane_blocks(kv, fb.r0, d.t_end);
+        in.bl_next = lane_blocks(kv, fb.r1, d.t_end);
         load_k(kv, in.bl_cur, d.kvh, in.cur);
         load_v(kv, in.bl_cur, d.kvh, in.cur);
     }
@@ -393,14 +406,15 @@ __device__ __forceinline__ void start_piece(const AttnArgs& a, const KVView& kv,
     // The in-register patch of the chunk holding the rows needs 16-byte V runs.
     constexpr bool kDefer = DT != GG_DTYPE_INT8 && Geo<PoolTraits<DT>::kEB, TOK, HD>::kVBytes == 16;
     if (ap) ap->j0 = ap->j1 = 0;
+    const auto fb = PieceIO<DT, TOK, HD>::first_blocks(a, d);
     if (a.k_new) {
-        const int ctx = seq_keys(a, d.b, kBS), nrows = seq_rows(a, d.b);
+        const int ctx = d.ctx, nrows = d.nrows;
         const int first = ctx - nrows;
         const int j0 = max(0, d.t0 - first), j1 = min(nrows, d.t_end - first);
         if (nrows > 0 && nrows <= ctx && j0 < j1) {
             const int items = (j1 - j0) * (HD / 8);
             if (kDefer && ap && items <= kAppMax && first + j0 >= d.t0 + kWaves * kTok) {
-                PieceIO<DT, TOK, HD>::start(a, kv, d, in);
+                PieceIO<DT, TOK, HD>::start(kv, d, fb, in);
                 ap->j0 = j0;
                 ap->j1 = j1;
                 ap->it.live = false;
@@ -415,16 +429,16 @@ __device__ __forceinline__ void start_piece(const AttnArgs& a, const KVView& kv,
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
                 __syncthreads();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                PieceIO<DT, TOK, HD>::start(a, kv, d, in);
+                PieceIO<DT, TOK, HD>::start(kv, d, fb, in);
             } else {
                 append_item_rows(a, kv, d.b, d.kvh, j0, j1);
                 __syncthreads();
-                PieceIO<DT, TOK, HD>::start(a, kv, d, in);
+                PieceIO<DT, TOK, HD>::start(kv, d, fb, in);
             }
             return;
         }
     }
-    PieceIO<DT, TOK, HD>::start(a, kv, d, in);
+    PieceIO<DT, TOK, HD>::start(kv, d, fb, in);
 }
 
 // One piece of work: tokens [t0, t_end) of sequence b against kv head kvh. The result
@@ -436,17 +450,62 @@ __device__ __forceinline__ void start_piece(const AttnArgs& a, const KVView& kv,
 // bypass the per-XCD caches' stale copies, so a workgroup on another XCD reads what was
 // written. Ordering before the merge counter comes from waiting for the stores to
 // complete (every record store of the workgroup) before the counter's atomic add.
-__device__ __forceinline__ void store_agent(float* p, float v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ float2 load_agent2(const float* p) {
+    const unsigned long long v =
+        __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
 }
-__device__ __forceinline__ float load_agent(const float* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void store_agent2(float* p, float a, float b) {
+    const unsigned long long v = ((unsigned long long)__float_as_uint(b) << 32) | __float_as_uint(a);
+    __hip_atomic_store((unsigned long long*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Four consecutive output elements in one store. The struct types promise no more than the
+// element's own alignment, whatever the caller's buffer has.
+__device__ __forceinline__ void store4_from_f32(void* p, gg_dtype_t dt, size_t i, const float (&v)[4]) {
+    struct __attribute__((packed, aligned(4))) F4 { float4 v; };
+    struct __attribute__((packed, aligned(2))) H4 { uint2 v; };
+    if (dt == GG_DTYPE_F32) {
+        ((F4*)((float*)p + i))->v = make_float4(v[0], v[1], v[2], v[3]);
+        return;
+    }
+    uint32_t h[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) h[k] = dt == GG_DTYPE_BF16 ? f32_to_bf16_bits(v[k]) : f32_to_f16_bits(v[k]);
+    ((H4*)((uint16_t*)p + i))->v = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+}
+
+// The piece's queries of a 16-bit type, as the Q staging below takes them (f32 ones are read
+// there). Issued before the piece's K and V: loads retire in order, so the staging then waits
+// for these alone.
+template <int NT>
+struct QRaw {
+    uint4 v[NT];
+};
+template <int NT, int HD>
+__device__ __forceinline__ QRaw<NT> load_q16(const AttnArgs& a, const KVView& kv, const PieceDesc& d) {
+    struct __attribute__((packed, aligned(2))) U4 { uint4 v; };
+    QRaw<NT> q;
+    if (a.q_dtype == GG_DTYPE_F32) {
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt) q.v[rt] = make_uint4(0, 0, 0, 0);
+        return q;
+    }
+    const int G = a.num_q_heads / kv.Hkv, rows = G * d.nrows - d.row0;
+    const int c16 = threadIdx.x & 15, g4 = (threadIdx.x >> 4) & 3, mm = (threadIdx.x >> 6) & (HD / 32 - 1);
+#pragma unroll
+    for (int rt = 0; rt < NT; ++rt) {
+        const int r = rt * 16 + c16 < rows ? d.row0 + rt * 16 + c16 : 0;
+        const size_t i = (((size_t)d.b * a.rows + r / G) * a.num_q_heads + (size_t)d.kvh * G + r % G) * HD +
+                         HD / 4 * g4 + 8 * mm;
+        q.v[rt] = ((const U4*)((const uint16_t*)a.q + i))->v;
+    }
+    return q;
 }
 
 template <gg_dtype_t DT, int NT, int HD, bool FULL>
 __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, const PieceDesc pd,
                                            PieceIn<DT, attn_chunk_tokens(PoolTraits<DT>::kEB, NT), HD>& in,
-                                           const DeferredRows* ap) {
+                                           const DeferredRows* ap, const QRaw<NT>& q16) {
     const int b = pd.b, kvh = pd.kvh, t0 = pd.t0, t_end = pd.t_end, part = pd.part, rec = pd.rec;
     using T = PoolTraits<DT>;
     // FULL: FP8 and INT8 values go through bf16 as well, whose range holds any block scale.
@@ -459,9 +518,9 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
     constexpr int kTok = Geom::kTok;
     constexpr int kNS = Geom::kNS;
 
-    const int ctx = seq_keys(a, b, kBS);
+    const int ctx = pd.ctx;
     const int R = a.rows;
-    const int nrows = seq_rows(a, b);
+    const int nrows = pd.nrows;
     if (nrows <= 0 || nrows > ctx) return;
     const int Hq = a.num_q_heads;
     const int G = Hq / kv.Hkv;
@@ -560,13 +619,10 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
                     for (int e = 0; e < 8; ++e) f[rt][e] = qvalid[rt] ? v[e] : 0.f;
                 }
             } else {
-                uint4 raw[NT];
-#pragma unroll
-                for (int rt = 0; rt < NT; ++rt) raw[rt] = *(const uint4*)((const uint16_t*)a.q + qb[rt]);
                 const bool src_bf16 = a.q_dtype == GG_DTYPE_BF16;
 #pragma unroll
                 for (int rt = 0; rt < NT; ++rt) {
-                    const uint32_t w[4] = {raw[rt].x, raw[rt].y, raw[rt].z, raw[rt].w};
+                    const uint32_t w[4] = {q16.v[rt].x, q16.v[rt].y, q16.v[rt].z, q16.v[rt].w};
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const uint16_t h = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
@@ -685,7 +741,7 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
             const bool src_bf16 = a.q_dtype == GG_DTYPE_BF16;
 #pragma unroll
             for (int rt = 0; rt < NT; ++rt) {
-                op[rt] = *(const uint4*)((const uint16_t*)a.q + qb[rt]);
+                op[rt] = q16.v[rt];
                 opl[rt] = zero4();
             }
             // Convert when the Q type differs from the MFMA operand type.
@@ -1031,7 +1087,7 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
     // ---- merge the four waves' states through LDS ----
     __shared__ float s_m[kWaves][64];
     __shared__ float s_l[kWaves][64];
-    __shared__ float s_o[kWaves][16][HD + 4];
+    __shared__ __align__(16) float s_o[kWaves][16][HD + 4];
 #pragma unroll
     for (int rt = 0; rt < NT; ++rt) {
         float lt = l_run[rt];
@@ -1059,36 +1115,41 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
             for (int dt = 0; dt < Geom::kDT; ++dt) s_o[wave][rr][dt * 16 + c16] = o[rt][dt][i] * f;
         }
         __syncthreads();
-        // 256 threads sum the 4 wave copies of 16 rows x 128 dims.
-        for (int e = threadIdx.x; e < 16 * HD; e += 256) {
-            const int rr = e / HD, d = e % HD;
+        // 256 threads sum the four waves' copies, four dims of a row at a time.
+#pragma unroll
+        for (int e = threadIdx.x; e < 16 * (HD / 4); e += 256) {
+            const int rr = e / (HD / 4), d = 4 * (e % (HD / 4));
             const int r = rt * 16 + rr;
             if (r >= nvalid_rows) continue;
             float mx = s_m[0][r];
 #pragma unroll
             for (int w = 1; w < kWaves; ++w) mx = fmaxf(mx, s_m[w][r]);
-            float L = 0.f, acc = 0.f;
+            float L = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) {
                 L += s_l[w][r] * __builtin_amdgcn_exp2f(s_m[w][r] - mx);
-                acc += s_o[w][rr][d];
+                const float4 v = *(const float4*)&s_o[w][rr][d];
+                acc[0] += v.x;
+                acc[1] += v.y;
+                acc[2] += v.z;
+                acc[3] += v.w;
             }
             const int j = (row0 + r) / G, g = (row0 + r) % G;
             const size_t z = zbase + j;
             const int h = kvh * G + g;
             if (final_out) {
-                const float val = L > 0.f ? acc * vfold / L : 0.f;
-                store_from_f32(a.out, a.out_dtype, (z * Hq + h) * HD + d, val);
+                float val[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) val[k] = L > 0.f ? acc[k] * vfold / L : 0.f;
+                store4_from_f32(a.out, a.out_dtype, (z * Hq + h) * HD + d, val);
             } else {
                 const size_t pidx = rec >= 0 ? (size_t)rec * (size_t)(FULL ? 16 * NT : G * R) + (size_t)r
                                              : (z * Hq + h) * a.max_parts + part;
                 // Device-scope stores: they reach the point every XCD reads from, so the
                 // last piece of an LPT item can merge the records in the same launch.
-                store_agent(a.ws_acc + pidx * HD + d, acc * vfold);
-                if (d == 0) {
-                    store_agent(a.ws_ml + pidx * 2 + 0, mx > -1e29f ? mx * kLn2 : -1e30f);
-                    store_agent(a.ws_ml + pidx * 2 + 1, L);
-                }
+                store_agent2(a.ws_acc + pidx * HD + d, acc[0] * vfold, acc[1] * vfold);
+                store_agent2(a.ws_acc + pidx * HD + d + 2, acc[2] * vfold, acc[3] * vfold);
+                if (d == 0) store_agent2(a.ws_ml + pidx * 2, mx > -1e29f ? mx * kLn2 : -1e30f, L);
             }
         }
         __syncthreads();
@@ -1120,13 +1181,13 @@ __device__ __forceinline__ int seq_chunks(const AttnArgs& a, int b, int tok) {
 // Plan layout (ints, in the workspace after the records), P = piece bound (lpt_pieces), B =
 // sequences, H = heads (kv heads, times the row groups of a shape whose rows are cut):
 //   [0 .. 15]                 unused
-//   [16 + 4p ..]              piece p: (sequence | piece j of the item * kLptMaxSeqs, head |
-//                             pieces per item << 16, first token, end token); -1 past the
-//                             last piece
-//   [16 + 4P + b]             first record of sequence b (split sequences only)
-//   [16 + 4P + B + b*H + h]   merge counter of (sequence b, head h)
-// The records of split sequence b are first + j*H + h for its piece j, numbered by sequence;
-// pieces of uncut items have none.
+//   [16 + 8p ..]              piece p: sequence (-1 past the last piece), head | pieces of
+//                             the item << 16, first token, end token, keys and rows of the
+//                             sequence, the item's first record, piece j of the item: all a
+//                             workgroup needs to start, in one load
+//   [16 + 8P + b*H + h]       merge counter of (sequence b, head h)
+// The records of split item (b, h) are first, first + H, ... in piece order, numbered by
+// sequence; items of one piece have none.
 __device__ __forceinline__ int* lpt_table(int* plan) { return plan + 16; }
 // Workgroup of the piece of rank r. While the
 // (sequence, kv head) items do not outnumber the S slots: over the first W = min(S,
@@ -1156,10 +1217,9 @@ __device__ __forceinline__ int lpt_slot(int r, int S, int total, bool pair) {
     }
     return r;
 }
-__device__ __forceinline__ int* lpt_seq(int* plan, int pieces) { return plan + 16 + 4 * pieces; }
 // Merge counters, one per (sequence, kv head): pieces of a split item that have written
 // their records. The plan clears them; the piece that merges an item clears its counter.
-__device__ __forceinline__ int* lpt_count(int* plan, int pieces, int B) { return lpt_seq(plan, pieces) + B; }
+__device__ __forceinline__ int* lpt_count(int* plan, int pieces) { return plan + 16 + 8 * pieces; }
 
 // The piece of a split item that finishes last merges the item's records: the online
 // log-sum-exp over its pieces in piece order, as a merge launch of its own would. Each
@@ -1180,61 +1240,65 @@ __device__ __forceinline__ int* lpt_count(int* plan, int pieces, int B) { return
 // record's store. The language-level way (a release add and an acquire read) writes back
 // and invalidates the whole XCD L2 on this device and costs config 3 about 4 % (measured).
 // h: the item's head (with row groups, group * kv heads + kv head); RW: rows per record;
-// row0, rows: its query rows [row0, row0 + rows) (rows of the sequence's G * row count).
+// first: the item's first record, the others `heads` apart.
 template <int HD>
-__device__ __forceinline__ void lpt_merge_if_last(const AttnArgs& a, int Hkv, int heads, int b, int kvh, int h, int np,
-                                                  int RW, int row0) {
+__device__ __forceinline__ void lpt_merge_if_last(const AttnArgs& a, int Hkv, int heads, const PieceDesc& d, int h, int np,
+                                                  int first, int RW) {
     __shared__ int s_last;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's record stores are done
     __syncthreads();
-    const int recs = lpt_pieces(a.sk_grid, a.num_seqs, heads);
-    int* cnt = lpt_count(a.plan, recs, a.num_seqs) + b * heads + h;
+    int* cnt = lpt_count(a.plan, lpt_pieces(a.sk_grid, a.num_seqs, heads)) + d.b * heads + h;
     if (threadIdx.x == 0)
         s_last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == np - 1;
     __syncthreads();
     if (!s_last) return;
-    const int first = lpt_seq(a.plan, recs)[b];
     const int G = a.num_q_heads / Hkv;
-    const int nrows = seq_rows(a, b), ctx = seq_keys(a, b, kBS);
-    if (nrows > 0 && nrows <= ctx) {
-        const int rows = min(G * nrows - row0, RW);
-        // Thread pairs (row, 4 dims): HD / 4 threads per row.
-        for (int e = threadIdx.x; e < rows * (HD / 4); e += blockDim.x) {
-            const int r = e / (HD / 4), d4 = e % (HD / 4);
-            float M = -1e30f, L = 0.f;
-            float acc[4] = {0.f, 0.f, 0.f, 0.f};
-            // Four records per step, their loads issued together.
-            int jp = 0;
-            auto merge = [&](auto n) {
-                constexpr int N = decltype(n)::value;
-                float mx[N], ly[N], v[N][4];
+    const int items = min(G * d.nrows - d.row0, RW) * (HD / 4);  // (row, 4 dims)
+    // Two items per thread and up to four records per step, their loads issued together: the
+    // merge is a chain of round trips to the coherence point.
+    for (int e0 = threadIdx.x; e0 < items; e0 += 2 * blockDim.x) {
+        const int e[2] = {e0, min(e0 + (int)blockDim.x, items - 1)};
+        float M[2] = {-1e30f, -1e30f}, L[2] = {0.f, 0.f}, acc[2][4] = {};
+        int jp = 0;
+        auto merge = [&](auto n) {
+            constexpr int N = decltype(n)::value;
+            float2 ml[2][N], v[2][N][2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int u = 0; u < N; ++u) {
-                    const size_t q = (size_t)(first + (jp + u) * heads + h) * RW + r;
-                    mx[u] = load_agent(a.ws_ml + q * 2);
-                    ly[u] = load_agent(a.ws_ml + q * 2 + 1);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) v[u][i] = load_agent(a.ws_acc + q * HD + 4 * d4 + i);
+                    const size_t q = (size_t)(first + (jp + u) * heads) * RW + e[i] / (HD / 4);
+                    const float* x = a.ws_acc + q * HD + 4 * (e[i] % (HD / 4));
+                    ml[i][u] = load_agent2(a.ws_ml + q * 2);
+                    v[i][u][0] = load_agent2(x);
+                    v[i][u][1] = load_agent2(x + 2);
                 }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int u = 0; u < N; ++u) {
-                    const float mn = fmaxf(M, mx[u]);
-                    const float fo = __expf(M - mn), fn = __expf(mx[u] - mn);
-                    M = mn;
-                    L = L * fo + ly[u] * fn;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[i] = acc[i] * fo + v[u][i] * fn;
+                    const float mn = fmaxf(M[i], ml[i][u].x);
+                    const float fo = __expf(M[i] - mn), fn = __expf(ml[i][u].x - mn);
+                    M[i] = mn;
+                    L[i] = L[i] * fo + ml[i][u].y * fn;
+                    acc[i][0] = acc[i][0] * fo + v[i][u][0].x * fn;
+                    acc[i][1] = acc[i][1] * fo + v[i][u][0].y * fn;
+                    acc[i][2] = acc[i][2] * fo + v[i][u][1].x * fn;
+                    acc[i][3] = acc[i][3] * fo + v[i][u][1].y * fn;
                 }
-                jp += N;
-            };
-            while (jp + 4 <= np) merge(std::integral_constant<int, 4>{});
-            if (jp + 2 <= np) merge(std::integral_constant<int, 2>{});
-            if (jp < np) merge(std::integral_constant<int, 1>{});
-            const float inv = L > 0.f ? 1.f / L : 0.f;
-            const int j = (row0 + r) / G, g = (row0 + r) % G;
-            const size_t obase = (((size_t)b * a.rows + j) * a.num_q_heads + (size_t)kvh * G + g) * HD + 4 * d4;
+            jp += N;
+        };
+        while (jp + 4 <= np) merge(std::integral_constant<int, 4>{});
+        if (jp + 2 <= np) merge(std::integral_constant<int, 2>{});
+        if (jp < np) merge(std::integral_constant<int, 1>{});
 #pragma unroll
-            for (int i = 0; i < 4; ++i) store_from_f32(a.out, a.out_dtype, obase + i, acc[i] * inv);
+        for (int i = 0; i < 2; ++i) {
+            if (i == 1 && e0 + (int)blockDim.x >= items) break;
+            const int r = d.row0 + e[i] / (HD / 4), d4 = 4 * (e[i] % (HD / 4));
+            const float inv = L[i] > 0.f ? 1.f / L[i] : 0.f;
+            const float o[4] = {acc[i][0] * inv, acc[i][1] * inv, acc[i][2] * inv, acc[i][3] * inv};
+            store4_from_f32(a.out, a.out_dtype,
+                            (((size_t)d.b * a.rows + r / G) * a.num_q_heads + (size_t)d.kvh * G + r % G) * HD + d4, o);
         }
     }
     if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // next layer
@@ -1249,22 +1313,20 @@ __global__ void __launch_bounds__(256, attn_occupancy(PoolTraits<DT>::kEB, NT, H
     const long long tr_t0 = wall_clock64();
 #endif
     // One load tells the workgroup everything about its piece.
-    const int4 e = ((const int4*)lpt_table(a.plan))[p];
+    const int4 e = ((const int4*)lpt_table(a.plan))[2 * p], f = ((const int4*)lpt_table(a.plan))[2 * p + 1];
     if (e.x < 0) return;  // past the last piece
-    const int b = e.x & (kLptMaxSeqs - 1), j = e.x / kLptMaxSeqs;
     const int h = e.y & 0xffff, np = e.y >> 16;
     const int heads = FULL ? kv.Hkv * a.row_groups : kv.Hkv;
     const int kvh = FULL ? h % kv.Hkv : h;
     const int row0 = FULL ? h / kv.Hkv * (16 * NT) : 0;
-    int rec = -1;
-    if (np > 1) rec = lpt_seq(a.plan, lpt_pieces(a.sk_grid, a.num_seqs, heads))[b] + j * heads + h;
-    const PieceDesc d{b, kvh, e.z, e.w, -1, rec, row0};
+    const PieceDesc d{e.x, kvh, e.z, e.w, -1, np > 1 ? f.z + f.w * heads : -1, row0, f.x, f.y};
     PieceIn<DT, attn_chunk_tokens(PoolTraits<DT>::kEB, NT), HD> in;
     DeferredRows ap;
+    const QRaw<NT> q16 = load_q16<NT, HD>(a, kv, d);
     start_piece(a, kv, d, in, &ap);
-    attn_piece<DT, NT, HD, FULL>(a, kv, d, in, &ap);
-    if (np > 1)
-        lpt_merge_if_last<HD>(a, kv.Hkv, heads, b, kvh, h, np, FULL ? 16 * NT : a.num_q_heads / kv.Hkv * a.rows, row0);
+    attn_piece<DT, NT, HD, FULL>(a, kv, d, in, &ap, q16);
+    if (np > 1 && (!FULL || a.num_q_heads / kv.Hkv * d.nrows > row0))
+        lpt_merge_if_last<HD>(a, kv.Hkv, heads, d, h, np, f.z, FULL ? 16 * NT : a.num_q_heads / kv.Hkv * a.rows);
 #ifdef GG_TRACE
     if (threadIdx.x == 0) {
         g_trace[4 * p + 0] = tr_t0;

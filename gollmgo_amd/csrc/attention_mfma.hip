@@ -17,11 +17,12 @@ __global__ void __launch_bounds__(256, attn_occupancy(PoolTraits<DT>::kEB, NT, k
     const int P = a.partition;
     const int nparts = (ctx + P - 1) / P;
     if (part >= nparts) return;
-    const PieceDesc d{b, kvh, part * P, min(part * P + P, ctx), nparts == 1 ? -1 : part, -1, 0};
+    const PieceDesc d{b, kvh, part * P, min(part * P + P, ctx), nparts == 1 ? -1 : part, -1, 0, ctx, seq_rows(a, b)};
     PieceIn<DT, attn_chunk_tokens(PoolTraits<DT>::kEB, NT), kHD> in;
     DeferredRows ap;
+    const QRaw<NT> q16 = load_q16<NT, kHD>(a, kv, d);
     start_piece(a, kv, d, in, &ap);
-    attn_piece<DT, NT, kHD, false>(a, kv, d, in, &ap);
+    attn_piece<DT, NT, kHD, false>(a, kv, d, in, &ap, q16);
 }
 
 // Stream-K: the (sequence, kv head) items are laid end to end in chunk units; the grid
@@ -102,7 +103,8 @@ __global__ void __launch_bounds__(256, attn_occupancy(PoolTraits<DT>::kEB, NT, k
             const int item = b * Hkv + kvh;
             const bool whole = c0 == 0 && c1 == nch;
             const int ctx = __builtin_amdgcn_readfirstlane(seq_keys(a, b, kBS));
-            d = PieceDesc{b, kvh, c0 * kTok, min(c1 * kTok, ctx), -1, whole ? -1 : w + item, 0};
+            d = PieceDesc{b, kvh, c0 * kTok, min(c1 * kTok, ctx), -1, whole ? -1 : w + item, 0, ctx,
+                          __builtin_amdgcn_readfirstlane(seq_rows(a, b))};
             g = __builtin_amdgcn_readfirstlane(g + (c1 - c0));
             return true;
         }
@@ -111,8 +113,9 @@ __global__ void __launch_bounds__(256, attn_occupancy(PoolTraits<DT>::kEB, NT, k
     PieceDesc d;
     while (next_piece(d)) {
         PieceIn<DT, attn_chunk_tokens(PoolTraits<DT>::kEB, NT), kHD> in;
+        const QRaw<NT> q16 = load_q16<NT, kHD>(a, kv, d);
         start_piece(a, kv, d, in, nullptr);
-        attn_piece<DT, NT, kHD, false>(a, kv, d, in, nullptr);
+        attn_piece<DT, NT, kHD, false>(a, kv, d, in, nullptr, q16);
     }
 }
 
@@ -157,7 +160,7 @@ __device__ __forceinline__ unsigned long long block_excl_scan2_1024(int lo, int 
 __global__ void __launch_bounds__(1024) attn_lpt_plan_kernel(AttnArgs a, int Hkv, int tok, int slots, int pieces) {
     __shared__ __align__(16) int s_key[kLptMaxSeqs];  // piece size in chunks (0: no work)
     __shared__ __align__(16) int s_cnt[kLptMaxSeqs];  // pieces of the sequence over all kv heads
-    __shared__ int s_nch[kLptMaxSeqs], s_ctx[kLptMaxSeqs];
+    __shared__ int s_nch[kLptMaxSeqs], s_ctx[kLptMaxSeqs], s_rows[kLptMaxSeqs], s_first[kLptMaxSeqs];
     __shared__ long long s_w[16];
     __shared__ unsigned long long s_scan[16];
     __shared__ int s_t;
@@ -165,6 +168,7 @@ __global__ void __launch_bounds__(1024) attn_lpt_plan_kernel(AttnArgs a, int Hkv
     const int b = threadIdx.x;
     const int nch = b < B ? seq_chunks(a, b, tok) : 0;
     const int ctx = b < B ? seq_keys(a, b, kBS) : 0;
+    const int nrows = b < B ? seq_rows(a, b) : 0;
     const long long C = block_sum_1024((long long)Hkv * nch, s_w);
     const bool few = lpt_few_items(slots, B, Hkv);
     if (!few) {
@@ -201,18 +205,19 @@ __global__ void __launch_bounds__(1024) attn_lpt_plan_kernel(AttnArgs a, int Hkv
                 pos += (kk[e] > rem || (kk[e] == rem && t < b)) ? nn[e] : 0;
             }
         }
-        lpt_seq(plan, pieces)[b] = rec_first;
-        for (int h = 0; h < Hkv; ++h) lpt_count(plan, pieces, B)[b * Hkv + h] = 0;
+        for (int h = 0; h < Hkv; ++h) lpt_count(plan, pieces)[b * Hkv + h] = 0;
         int4* table = (int4*)lpt_table(plan);
         for (int j = 0; j < np; ++j) {
             const int c0 = j * T, c1 = j == np - 1 ? nch : (j + 1) * T;
             const int t0 = c0 * tok, t1 = min(c1 * tok, ctx);
             for (int h = 0; h < Hkv; ++h) {
                 const int r = j < np - 1 ? full_pos + j * Hkv + h : pos + h;
-                table[lpt_slot(r, slots, total, B * Hkv <= slots)] = make_int4(b | j * kLptMaxSeqs, h | (np << 16), t0, t1);
+                int4* t = table + 2 * lpt_slot(r, slots, total, B * Hkv <= slots);
+                t[0] = make_int4(b, h | (np << 16), t0, t1);
+                t[1] = make_int4(ctx, nrows, rec_first + h, j);
             }
         }
-        for (int q = total + b; q < pieces; q += B) table[q] = make_int4(-1, 0, 0, 0);
+        for (int q = total + b; q < pieces; q += B) table[2 * q] = make_int4(-1, 0, 0, 0);
         return;
     }
     // Fewer items than slots: every long item has to be cut to fill the slots, into equal
@@ -269,7 +274,6 @@ __global__ void __launch_bounds__(1024) attn_lpt_plan_kernel(AttnArgs a, int Hkv
                 pos += (kk[e] > key || (kk[e] == key && t < b)) ? nn[e] : 0;
             }
         }
-        lpt_seq(plan, pieces)[b] = rec_first;
     }
     __syncthreads();
     // The table is written by all threads, one (sequence, kv head) at a time.
@@ -278,21 +282,24 @@ __global__ void __launch_bounds__(1024) attn_lpt_plan_kernel(AttnArgs a, int Hkv
         s_cnt[b] = np;
         s_nch[b] = nch;
         s_ctx[b] = ctx;
+        s_rows[b] = nrows;
+        s_first[b] = rec_first;
     }
     __syncthreads();
     int4* table = (int4*)lpt_table(plan);
     for (int i = threadIdx.x; i < B * Hkv; i += 1024) {
         const int q = i / Hkv, h = i % Hkv;
         const int qp = s_key[q], qn = s_cnt[q], n = s_nch[q], qc = s_ctx[q];
-        lpt_count(plan, pieces, B)[i] = 0;
+        lpt_count(plan, pieces)[i] = 0;
         for (int j = 0; j < qn; ++j) {
             const int c0 = (int)((long long)j * n / qn), c1 = (int)((long long)(j + 1) * n / qn);
-            table[lpt_slot(qp + j * Hkv + h, slots, total, true)] =
-                make_int4(q | j * kLptMaxSeqs, h | (qn << 16), c0 * tok, min(c1 * tok, qc));
+            int4* t = table + 2 * lpt_slot(qp + j * Hkv + h, slots, total, true);
+            t[0] = make_int4(q, h | (qn << 16), c0 * tok, min(c1 * tok, qc));
+            t[1] = make_int4(qc, s_rows[q], s_first[q] + h, j);
         }
     }
     // Entries past the last piece tell their workgroups to exit.
-    for (int q = total + threadIdx.x; q < pieces; q += 1024) table[q] = make_int4(-1, 0, 0, 0);
+    for (int q = total + threadIdx.x; q < pieces; q += 1024) table[2 * q] = make_int4(-1, 0, 0, 0);
 }
 
 template <gg_dtype_t DT>
@@ -436,22 +443,30 @@ int attn_slots(const KV* kv, int rows, int num_q_heads) {
     return device_cu_count() * attn_occupancy((int)dtype_bytes(kv->dtype), attn_shape(kv, rows, num_q_heads).nt, kv->head_dim);
 }
 
-size_t attn_record_workspace_bytes(const KV* kv, int sched, int num_seqs, int rows, int num_q_heads, size_t* ml_elems,
-                                   size_t* acc_elems) {
+size_t attn_record_workspace_bytes(const KV* kv, int sched, int num_seqs, int rows, int num_q_heads, int max_blocks,
+                                   size_t* ml_elems, size_t* acc_elems) {
     const AttnShape sh = attn_shape(kv, rows, num_q_heads);
     const int slots = attn_slots(kv, rows, num_q_heads);
     const int heads = kv->num_kv_heads * sh.groups;
     const size_t items = (size_t)num_seqs * heads;
+    const size_t gr = (size_t)(num_q_heads / kv->num_kv_heads) * rows;
     const bool lpt = sched == ATTN_SCHED_LPT;
+    auto bytes = [&](size_t records, size_t rw, size_t plan_ints) {
+        return ((records * rw * 2 + 63) / 64 * 64 + records * rw * kv->head_dim) * sizeof(float) + plan_ints * sizeof(int);
+    };
     // LPT: records of split items only. Stream-K: one per workgroup and item.
     const size_t records = lpt ? (size_t)lpt_records(slots) : (size_t)slots + items;
-    const size_t rw = sh.full ? (size_t)16 * sh.nt : (size_t)(num_q_heads / kv->num_kv_heads) * rows;
-    const size_t n_ml = records * rw * 2;
-    const size_t n_acc = records * rw * kv->head_dim;
-    const size_t plan_ints = lpt ? 16 + 4 * (size_t)lpt_pieces(slots, num_seqs, heads) + (size_t)num_seqs + items : 0;
-    if (ml_elems) *ml_elems = n_ml;
-    if (acc_elems) *acc_elems = n_acc;
-    return (((n_ml + 63) / 64) * 64 + n_acc) * sizeof(float) + plan_ints * sizeof(int);
+    const size_t rw = sh.full ? (size_t)16 * sh.nt : gr;
+    if (ml_elems) *ml_elems = records * rw * 2;
+    if (acc_elems) *acc_elems = records * rw * kv->head_dim;
+    const size_t need = bytes(records, rw, lpt ? 16 + 8 * (size_t)lpt_pieces(slots, num_seqs, heads) + items : 0);
+    // The size asked for is never below a record per slot and item and its plan, or, for the
+    // shapes the per-row kernel also serves, that kernel's: callers size buffers by it, and
+    // gg_verify_attention_noalloc takes the calls that fit its fixed array by this measure.
+    const size_t asked = sh.full ? attn_workspace_bytes(kv, num_seqs, rows, num_q_heads, max_blocks,
+                                                        attn_generic_partition(kv, num_seqs, rows, num_q_heads, max_blocks))
+                                 : bytes((size_t)slots + items, gr, 16 + 4 * ((size_t)slots + items) + 2 * (size_t)num_seqs + items);
+    return std::max(need, asked);
 }
 
 #ifdef GG_TRACE

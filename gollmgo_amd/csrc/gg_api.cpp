@@ -267,7 +267,8 @@ GG_API size_t gg_verify_attention_workspace_size(gg_kv_t kv, int num_seqs, int r
     if (partition_tokens < 0 || partition_tokens % 64 != 0) return 0;
     const AttnPlan plan = attn_plan(kv, num_seqs, rows_per_seq, num_q_heads, max_blocks_per_seq, partition_tokens);
     if (plan.sched != ATTN_SCHED_GRID)
-        return attn_record_workspace_bytes(kv, plan.sched, num_seqs, rows_per_seq, num_q_heads, nullptr, nullptr);
+        return attn_record_workspace_bytes(kv, plan.sched, num_seqs, rows_per_seq, num_q_heads, max_blocks_per_seq, nullptr,
+                                           nullptr);
     return attn_workspace_bytes(kv, num_seqs, rows_per_seq, num_q_heads, max_blocks_per_seq, plan.partition);
 }
 
@@ -318,7 +319,8 @@ static gg_status_t verify_attention_impl(gg_kv_t kv, int layer, const void* q, g
     if (a.sched != ATTN_SCHED_GRID) {
         a.sk_grid = attn_slots(kv, rows_per_seq, num_q_heads);
         a.row_groups = attn_shape(kv, rows_per_seq, num_q_heads).groups;
-        need = attn_record_workspace_bytes(kv, a.sched, num_seqs, rows_per_seq, num_q_heads, &n_ml, &n_acc);
+        need = attn_record_workspace_bytes(kv, a.sched, num_seqs, rows_per_seq, num_q_heads, max_blocks_per_seq, &n_ml,
+                                           &n_acc);
     } else {
         need = attn_workspace_bytes(kv, num_seqs, rows_per_seq, num_q_heads, max_blocks_per_seq, a.partition);
         n_ml = (size_t)num_seqs * rows_per_seq * num_q_heads * a.max_parts * 2;

@@ -104,7 +104,7 @@ enum { ATTN_SCHED_GRID = 0, ATTN_SCHED_STREAMK = 1, ATTN_SCHED_LPT = 2 };
 // + items) as (max, sum) pairs, then (64-float aligned) P.V rows, then the LPT plan (ints).
 // ml_elems and acc_elems receive the float counts of the first two parts.
 int attn_slots(const KV* kv, int rows, int num_q_heads);
-size_t attn_record_workspace_bytes(const KV* kv, int sched, int num_seqs, int rows, int num_q_heads,
+size_t attn_record_workspace_bytes(const KV* kv, int sched, int num_seqs, int rows, int num_q_heads, int max_blocks,
                                    size_t* ml_elems, size_t* acc_elems);
 int device_cu_count();
 size_t attn_workspace_bytes(const KV* kv, int num_seqs, int rows, int num_q_heads,
