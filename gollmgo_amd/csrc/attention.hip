@@ -58,51 +58,56 @@ struct Pool16 {
     }
 };
 
-template <gg_dtype_t DT, int DC>
-__global__ void __launch_bounds__(64) attn_generic_kernel(AttnArgs a, KVView kv) {
-    const int part = blockIdx.x;
-    const int h = blockIdx.y;
-    const int z = blockIdx.z;  // b*R + j
-    const int b = z / a.rows, j = z % a.rows;
-    const int nrows = seq_rows(a, b);
-    if (j >= nrows) return;
-    const int ctx = seq_keys(a, b, kv.bs);
-    if (ctx <= 0 || nrows > ctx) return;
-    const int P = a.partition;
-    const int nparts = (ctx + P - 1) / P;
-    if (part >= nparts) return;
-    const int pos = ctx - nrows + j;
-    const int t0 = part * P;
-    const int t1 = min(t0 + P, pos + 1);
-    const int G = a.num_q_heads / kv.Hkv;
-    const int kvh = h / G;
-    const int lane = threadIdx.x;
-    const int D = kv.D;
+// Most partitions of a (row, head) that one workgroup takes, a wave each, merging them in LDS.
+constexpr int kFuseParts = 8;
 
-    // A tile of 64 keys per step: lane i scores key t0 + 64k + i against the whole query
-    // (read from LDS), one wave max / sum per tile, then P.V with each lane owning dims
-    // lane + 64c and the tile's probabilities broadcast from their lanes.
-    __shared__ float s_q[64 * kMaxDC];
-    __shared__ float s_p[64];        // the tile's probabilities (times the V scale)
-    __shared__ size_t s_vrow[64];    // element offset of each key's V column 0
-    float acc[DC];
-    const size_t qbase = ((size_t)z * a.num_q_heads + h) * D;
-#pragma unroll
-    for (int c = 0; c < DC; ++c) {
-        const int d = lane + 64 * c;
-        if (d < D) s_q[d] = load_as_f32(a.q, a.q_dtype, qbase + d);
-        acc[c] = 0.f;
-    }
-    __syncthreads();
+// One partition of one (row, head), by one wave: keys in tiles of 64, lane i scoring key i of
+// the tile against the whole query (in LDS), one wave max and sum per tile, then P.V with each
+// lane owning dims lane + 64c. A tile's K rows and V runs are all requested before its scores
+// are needed, so a tile waits for one round trip to its block ids and one to its K and V. V
+// comes in 16-byte runs of offsets where blocks are whole runs and tiles whole blocks
+// (kVRun), by element elsewhere; the products are added in key order either way.
+// Bound by those round trips: with four K vectors and sixteen V elements in flight (V at a
+// line per lane and key) and the merge in a launch, 4 x 5 rows of 8 heads over 64-256 fp32 keys
+// took 14.0 + 4.2 µs, now 8.8; per call on one box, four fp32 sequences of 100-700 keys at
+// head_dim 128 64 -> 25 µs, eight bf16 ones at head_dim 96 132 -> 24.
+template <gg_dtype_t DT, int DC, bool kVRun>
+__device__ __forceinline__ void generic_partition(const AttnArgs& a, const KVView& kv, int b, int kvh, int t0, int t1,
+                                                  const float* s_q, float* s_p, size_t* s_vrow, float (&acc)[DC], float& m,
+                                                  float& l) {
+    const int lane = threadIdx.x & 63;
+    const int D = kv.D;
     const int32_t* bt = a.block_tables + (size_t)b * a.max_blocks;
-    float m = -1e30f, l = 0.f;
+    const uint8_t* vc = kv.vc;
+    constexpr int kN = Pool16<DT>::kN;
+    constexpr int kRuns = 64 / kN;  // 16-byte V runs of a tile per dim
+    m = -1e30f;
+    l = 0.f;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) acc[c] = 0.f;
     for (int tb = t0; tb < t1; tb += 64) {
         const int t = tb + lane;
+        const int ntile = min(64, t1 - tb);
         int blk = -1, off = 0;
         if (t < t1) {
             blk = bt[t / kv.bs];
             off = t % kv.bs;
             if (blk < 0 || blk >= kv.num_blocks) blk = -1;  // invalid table entry: key skipped
+        }
+        // (Skipped keys read block 0.)
+        const size_t vrow = kv.tile0(max(blk, 0), kvh) + off;
+        [[maybe_unused]] uint4 vr[kVRun ? DC : 1][kVRun ? kRuns : 1];
+        if constexpr (kVRun) {
+#pragma unroll
+            for (int r = 0; r < kRuns; ++r) {
+                const size_t base = ((size_t)__shfl((unsigned)(vrow >> 32), r * kN) << 32) | (unsigned)__shfl((unsigned)vrow, r * kN);
+#pragma unroll
+                for (int c = 0; c < DC; ++c) {
+                    const int d = min(lane + 64 * c, D - 1);
+                    // (A run past the tile reads its key 0's block: not used.)
+                    vr[c][r] = *(const uint4*)(vc + (base + (size_t)d * kv.bs) * dtype_bytes(DT));
+                }
+            }
         }
         float sc = -INFINITY;
         if (blk >= 0) {
@@ -110,9 +115,8 @@ __global__ void __launch_bounds__(64) attn_generic_kernel(AttnArgs a, KVView kv)
             // multiples of 16 bytes (pools are 256-byte aligned), else element loads.
             const uint8_t* krow = kv.kc + (kv.tile0(blk, kvh) + (size_t)off * D) * dtype_bytes(DT);
             float dot = 0.f;
-            constexpr int kN = Pool16<DT>::kN;
             if (D % kN == 0) {
-#pragma unroll 4
+#pragma unroll(DT == GG_DTYPE_F32 ? 16 : 4)
                 for (int v = 0; v < D / kN; ++v) {
                     float f[kN];
                     Pool16<DT>::decode(((const uint4*)krow)[v], f);
@@ -136,25 +140,101 @@ __global__ void __launch_bounds__(64) attn_generic_kernel(AttnArgs a, KVView kv)
         m = m_new;
 #pragma unroll
         for (int c = 0; c < DC; ++c) acc[c] *= alpha;
-        // The tile's probabilities and V offsets go through LDS, so the key loop below
-        // has no cross-lane operations and unrolls into batches of independent loads.
-        // (Masked and skipped keys have p = 0 and read block 0.)
-        __syncthreads();  // the previous tile's readers are done
+        // The tile's probabilities (and by element, V offsets) go through LDS, so the key loop
+        // below has no cross-lane operations. (Masked and skipped keys have p = 0.)
+        // One wave's own slots: its LDS operations complete in order.
+        __builtin_amdgcn_wave_barrier();
         s_p[lane] = blk >= 0 ? p * kv.v_scale(blk, kvh) : 0.f;
-        s_vrow[lane] = kv.tile0(max(blk, 0), kvh) + off;
-        __syncthreads();
-        const int ntile = min(64, t1 - tb);
-        const uint8_t* vc = kv.vc;
-#pragma unroll 16
-        for (int i = 0; i < ntile; ++i) {
-            const float pi = s_p[i];
-            const size_t vr = s_vrow[i];
+        if constexpr (!kVRun) s_vrow[lane] = vrow;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if constexpr (kVRun) {
 #pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                const int d = lane + 64 * c;
-                if (d < D) acc[c] += pi * pool_elem<DT>(vc, vr + (size_t)d * kv.bs);
+            for (int r = 0; r < kRuns; ++r) {
+                if (r * kN >= ntile) break;
+                float pi[kN];
+#pragma unroll
+                for (int e = 0; e < kN; ++e) pi[e] = s_p[r * kN + e];
+#pragma unroll
+                for (int c = 0; c < DC; ++c) {
+                    float f[kN];
+                    Pool16<DT>::decode(vr[c][r], f);
+#pragma unroll
+                    for (int e = 0; e < kN; ++e) acc[c] += pi[e] * (r * kN + e < ntile ? f[e] : 0.f);
+                }
+            }
+        } else {
+#pragma unroll 16
+            for (int i = 0; i < ntile; ++i) {
+                const float pi = s_p[i];
+                const size_t vr0 = s_vrow[i];
+#pragma unroll
+                for (int c = 0; c < DC; ++c) {
+                    const int d = lane + 64 * c;
+                    if (d < D) acc[c] += pi * pool_elem<DT>(vc, vr0 + (size_t)d * kv.bs);
+                }
             }
         }
+    }
+}
+
+// kFused: workgroup (h, z) takes every partition of a (row, head), wave w partition w, and
+// merges them through LDS in partition order (the combine kernel's sums); else workgroup
+// (part, h, z) takes one and the combine kernel merges.
+template <gg_dtype_t DT, int DC, bool kVRun, bool kFused>
+__global__ void __launch_bounds__(kFused ? 64 * kFuseParts : 64) attn_generic_kernel(AttnArgs a, KVView kv) {
+    const int wave = kFused ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+    const int part = kFused ? wave : (int)blockIdx.x;
+    const int h = blockIdx.y;
+    const int z = blockIdx.z;  // b*R + j
+    const int b = z / a.rows, j = z % a.rows;
+    const int nrows = seq_rows(a, b);
+    if (j >= nrows) return;
+    const int ctx = seq_keys(a, b, kv.bs);
+    if (ctx <= 0 || nrows > ctx) return;
+    const int P = a.partition;
+    const int nparts = (ctx + P - 1) / P;
+    if (!kFused && part >= nparts) return;
+    const int pos = ctx - nrows + j;
+    const int t0 = part * P;
+    const int t1 = min(t0 + P, pos + 1);
+    const int kvh = h / (a.num_q_heads / kv.Hkv);
+    const int lane = threadIdx.x & 63;
+    const int D = kv.D;
+    constexpr int kW = kFused ? kFuseParts : 1;
+    __shared__ float s_q[64 * DC];
+    __shared__ __align__(16) float s_p[kW][64];
+    __shared__ size_t s_vrow[kVRun ? 1 : kW][kVRun ? 1 : 64];
+    const size_t qbase = ((size_t)z * a.num_q_heads + h) * D;
+    for (int d = threadIdx.x; d < D; d += blockDim.x) s_q[d] = load_as_f32(a.q, a.q_dtype, qbase + d);
+    __syncthreads();
+    float acc[DC], m, l;
+    generic_partition<DT, DC, kVRun>(a, kv, b, kvh, t0, part < nparts ? t1 : t0, s_q, s_p[wave], s_vrow[kVRun ? 0 : wave],
+                                     acc, m, l);
+    if constexpr (kFused) {
+        __shared__ float s_acc[kFuseParts][64 * DC];
+        __shared__ float s_ml[kFuseParts][2];
+        if (nparts > 1) {
+#pragma unroll
+            for (int c = 0; c < DC; ++c) s_acc[wave][lane + 64 * c] = acc[c];
+            if (lane == 0) {
+                s_ml[wave][0] = m;
+                s_ml[wave][1] = l;
+            }
+            __syncthreads();
+            float M = -1e30f, total = 0.f;
+            for (int p = 0; p < nparts; ++p) M = fmaxf(M, s_ml[p][0]);
+            for (int p = 0; p < nparts; ++p) total += __expf(s_ml[p][0] - M) * s_ml[p][1];
+            const float inv = total > 0.f ? 1.0f / total : 0.f;
+            for (int d = threadIdx.x; d < D; d += blockDim.x) {
+                float o = 0.f;
+                for (int p = 0; p < nparts; ++p) o += __expf(s_ml[p][0] - M) * s_acc[p][d];
+                store_from_f32(a.out, a.out_dtype, qbase + d, o * inv);
+            }
+            return;
+        }
+        if (wave) return;
     }
     if (nparts == 1) {
         const float inv = l > 0.f ? 1.0f / l : 0.f;
@@ -165,15 +245,17 @@ __global__ void __launch_bounds__(64) attn_generic_kernel(AttnArgs a, KVView kv)
         }
         return;
     }
-    const size_t pidx = ((size_t)z * a.num_q_heads + h) * a.max_parts + part;
-    if (lane == 0) {
-        a.ws_ml[pidx * 2 + 0] = m;
-        a.ws_ml[pidx * 2 + 1] = l;
-    }
+    if constexpr (!kFused) {
+        const size_t pidx = ((size_t)z * a.num_q_heads + h) * a.max_parts + part;
+        if (lane == 0) {
+            a.ws_ml[pidx * 2 + 0] = m;
+            a.ws_ml[pidx * 2 + 1] = l;
+        }
 #pragma unroll
-    for (int c = 0; c < DC; ++c) {
-        const int d = lane + 64 * c;
-        if (d < D) a.ws_acc[pidx * D + d] = acc[c];
+        for (int c = 0; c < DC; ++c) {
+            const int d = lane + 64 * c;
+            if (d < D) a.ws_acc[pidx * D + d] = acc[c];
+        }
     }
 }
 
@@ -291,6 +373,7 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
                                                      a.partition % 64 == 0 && a.partition <= kMfmaMaxPartition);
     // Draft rows of the call: the MFMA kernels append them piece by piece (start_piece);
     // the generic path takes a launch of its own first.
+    bool combine = true;  // (the partition grid's merge launch)
     // So do the row groups of an INT8 item: each would re-quantise the block it appends to.
     AttnArgs m = a;
     if (a.k_new && (!mfma || (a.row_groups > 1 && kv->dtype == GG_DTYPE_INT8))) {
@@ -308,17 +391,31 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
         const int dc = (kv->head_dim + 63) / 64;
         const int DC = dc <= 1 ? 1 : dc <= 2 ? 2 : dc <= 4 ? 4 : dc <= 8 ? 8 : 16;
         if (dc > kMaxDC) return fail(GG_ERR_INVALID, "attention: head_dim too large");
-        dim3 grid(a.max_parts, a.num_q_heads, a.num_seqs * a.rows);
+        // V by 16-byte runs: a block is whole runs, a tile of 64 keys whole blocks, and a lane's
+        // runs of a tile fit its registers. Every partition of a row in one workgroup: few
+        // partitions, few enough dims for the LDS they meet in.
+        const bool vrun = kv->block_size * dtype_bytes(kv->dtype) % 16 == 0 && 64 % kv->block_size == 0 && DC <= 2;
+        const bool fused = a.max_parts <= kFuseParts && DC <= 2;
+        const dim3 grid(fused ? 1 : a.max_parts, a.num_q_heads, a.num_seqs * a.rows);
+        const int threads = fused ? 64 * a.max_parts : 64;
         auto launch = [&](auto dt_tag) {
             constexpr gg_dtype_t DT = decltype(dt_tag)::value;
+            auto small = [&](auto dc_tag) {
+                constexpr int N = decltype(dc_tag)::value;
+                if (vrun && fused) attn_generic_kernel<DT, N, true, true><<<grid, threads, 0, s>>>(a, view);
+                else if (vrun) attn_generic_kernel<DT, N, true, false><<<grid, threads, 0, s>>>(a, view);
+                else if (fused) attn_generic_kernel<DT, N, false, true><<<grid, threads, 0, s>>>(a, view);
+                else attn_generic_kernel<DT, N, false, false><<<grid, threads, 0, s>>>(a, view);
+            };
             switch (DC) {
-                case 1: attn_generic_kernel<DT, 1><<<grid, 64, 0, s>>>(a, view); break;
-                case 2: attn_generic_kernel<DT, 2><<<grid, 64, 0, s>>>(a, view); break;
-                case 4: attn_generic_kernel<DT, 4><<<grid, 64, 0, s>>>(a, view); break;
-                case 8: attn_generic_kernel<DT, 8><<<grid, 64, 0, s>>>(a, view); break;
-                default: attn_generic_kernel<DT, 16><<<grid, 64, 0, s>>>(a, view); break;
+                case 1: small(std::integral_constant<int, 1>{}); break;
+                case 2: small(std::integral_constant<int, 2>{}); break;
+                case 4: attn_generic_kernel<DT, 4, false, false><<<grid, threads, 0, s>>>(a, view); break;
+                case 8: attn_generic_kernel<DT, 8, false, false><<<grid, threads, 0, s>>>(a, view); break;
+                default: attn_generic_kernel<DT, 16, false, false><<<grid, threads, 0, s>>>(a, view); break;
             }
         };
+        combine = !fused;
         switch (kv->dtype) {
             case GG_DTYPE_F32: launch(std::integral_constant<gg_dtype_t, GG_DTYPE_F32>{}); break;
             case GG_DTYPE_F16: launch(std::integral_constant<gg_dtype_t, GG_DTYPE_F16>{}); break;
@@ -328,7 +425,7 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
             default: return fail(GG_ERR_INVALID, "attention: pool dtype");
         }
     }
-    if (a.max_parts > 1) {
+    if (combine && a.max_parts > 1) {
         attn_combine_kernel<<<dim3(a.num_q_heads, a.num_seqs * a.rows), 128, 0, s>>>(a, kv->head_dim);
     }
     static_assert(kMaxDC == 16, "generic kernel instantiations cover head_dim <= 1024");
