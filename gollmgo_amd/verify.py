@@ -34,8 +34,12 @@ def dtype_of(t: torch.Tensor) -> DType:
 
 
 def _stream(stream: Optional[torch.cuda.Stream]) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    """Raw handle of `stream`, or of the current stream of the current device. The handle is
+    asked for directly: torch.cuda.current_stream() builds a Stream object around it, 2.8 of the
+    5 to 8 us of host time that a call takes, against 0.5."""
+    if stream is not None:
+        return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dev(t: torch.Tensor, name: str, dtype=None) -> int:
