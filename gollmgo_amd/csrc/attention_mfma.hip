@@ -155,6 +155,16 @@ __device__ __forceinline__ unsigned long long block_excl_scan2(int lo, int hi, u
     return before + inc - v;
 }
 
+// Place of row group rg of unit u (a piece of one kv head) in a block of `units` equal pieces
+// of each of `groups` groups: the groups of a unit eight places apart, in blocks of eight
+// units. Workgroup w runs on XCD w mod 8, so the groups of a unit, which read the same K/V at
+// the same time, share one XCD's L2. (One group: u itself.) Three groups of 80 bf16 rows per kv
+// head, two kv heads, 16 sequences: 34.1 -> 30.3 µs a call.
+__device__ __forceinline__ int lpt_place(int u, int rg, int units, int groups) {
+    const int first = u & ~7;
+    return first * groups + rg * min(8, units - first) + (u & 7);
+}
+
 // One workgroup of N threads (one sequence per thread): sizes, ranks and lays out the pieces.
 // A chain of barriers and short loops of one workgroup, paid once per step: N is 256 for up
 // to 256 sequences (four waves meet at its barriers), the table is written by all threads, and
@@ -245,6 +255,7 @@ __global__ void __launch_bounds__(N) attn_lpt_plan_kernel(AttnArgs a, int Hkv, i
     int* plan = a.plan;
     int4* table = (int4*)lpt_table(plan);
     const int heads = B * Hkv;
+    const int kvh_n = Hkv / a.row_groups;
     int sub = 1;
     while (sub * 2 * heads <= N) sub *= 2;
     for (int i = threadIdx.x; i < heads * sub; i += N) {
@@ -256,7 +267,12 @@ __global__ void __launch_bounds__(N) attn_lpt_plan_kernel(AttnArgs a, int Hkv, i
         for (int j = i % sub; j < qn; j += sub) {
             const int c0 = j * size + min(j, extra);
             const int c1 = few ? c0 + size + (j < extra ? 1 : 0) : min(c0 + size, n);
-            const int r = few ? qp + j * Hkv + h : j < qn - 1 ? qf + j * Hkv + h : qp + h;
+            // Equal pieces of a sequence have a block of ranks: few, all of them; else its full
+            // pieces, and its last ones.
+            const bool full = !few && j < qn - 1;
+            const int units = (few ? qn : full ? qn - 1 : 1) * kvh_n;
+            const int u = (few || full ? j * kvh_n : 0) + h % kvh_n;
+            const int r = (full ? qf : qp) + lpt_place(u, h / kvh_n, units, a.row_groups);
             int4* t = table + 2 * lpt_slot(r, slots, total, heads <= slots);
             t[0] = make_int4(q, h | (qn << 16), c0 << tok_log2, min(c1 << tok_log2, qc));
             t[1] = make_int4(qc, qr, first, j);
