@@ -448,40 +448,53 @@ __global__ void __launch_bounds__(kSegThreads) sample_pass_kernel(DrawParams P) 
     }
     if (threadIdx.x == 0) s_hits = 0;
     __syncthreads();
+    // The hinted bins as distances d = l/T - m <= 0: bin_of is floor(-64 d) counted down from
+    // kBins - 1, so a bin's bounds are exact multiples of 1/64.
+    const double d_above = -(double)(kBins - 1 - ri.cbin) / 64.0;                          // bin > cbin: d > d_above
+    const double d_below = ri.cbin_lo > 0 ? -(double)(kBins - ri.cbin_lo) / 64.0 : -INFINITY;  // bin < cbin_lo: d <= d_below
     double acc = 0.0, above = 0.0, ep = 0.0, qp = 0.0;
-    int bad = 0;
+    bool bad = false;
     for (int c0 = 0; c0 < kSeg / 8; c0 += blockDim.x) {
         const int e0 = seg * kSeg + (c0 + threadIdx.x) * 8;
         float x[8], y[8];
-        load8<DT>(row, V, e0, P.vec, x);
+        load8<DT>(row, V, e0, P.vec, x);  // (-inf past the row: e = 0)
         if (split) load8q(qr, V, e0, P.vec_q, y);
+        unsigned hits = 0;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const float l = x[k];
-            const bool in = e0 + k < V;
-            if (in && (l != l || l == INFINITY)) bad = 1;
-            const double ev = (!in || l != l || l == INFINITY) ? 0.0 : fast_term(l, inv_t, m, s_tab);
+            bad |= __builtin_amdgcn_classf(l, 0x203);  // NaN or +inf: the row's sums are not used
+            const double d = (double)l * inv_t - m;
+            const double ev = gg_fast_exp64_tab(d, s_tab);
             acc += ev;
-            const uint32_t key = order_key(l);
-            const int bin = bin_of(l, inv_t, m);
             if (pre) {
-                if (in && bin > ri.cbin) above += ev;
-                stage_hit(in && bin <= ri.cbin && bin >= ri.cbin_lo, comp_key(key, e0 + k), &s_hits, s_buf);
+                above += d > d_above ? ev : 0.0;
+                hits |= (unsigned)(!(d > d_above) && (d > d_below || ri.cbin_lo == 0)) << k;
             } else if (split) {
-                const int e = e0 + k;
-                const bool cand = in && e != ri.x;
+                const bool cand = e0 + k < V && e0 + k != ri.x;
                 const float qf = (y[k] > 0.0f && y[k] <= 3.402823466e38f) ? fminf(y[k], 1.0f) : 0.0f;  // clean_q
                 const float ef = (float)ev;
                 const bool pos = cand && ef > qf * shi;
-                const bool amb = cand && !pos && ef != 0.0f && ef >= qf * slo;
-                if (pos) {
-                    ep += ev;
-                    qp += (double)qf;
-                }
-                if (__any(amb)) stage_hit(amb, (unsigned long long)e, &s_hits, s_buf);
-            } else if ((want_cnt || want_mass) && in) {
+                ep += pos ? ev : 0.0;
+                qp += pos ? (double)qf : 0.0;
+                hits |= (unsigned)(cand && !pos && ef != 0.0f && ef >= qf * slo) << k;
+            } else if ((want_cnt || want_mass) && e0 + k < V) {
+                const int bin = bin_of(l, inv_t, m);
                 if (want_cnt) atomicAdd(&s_cnt[bin], 1u);
                 if (want_mass && ev != 0.0) atomicAdd(&s_mass[bin], ev);
+            }
+        }
+        if (!kHist) {
+            if (pre && e0 + 8 > V) hits &= e0 < V ? (1u << (V - e0)) - 1u : 0u;
+            if (hits) {
+                int slot = atomicAdd(&s_hits, __popc(hits));
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    if (hits >> k & 1) {
+                        if (slot < kBlockCap)
+                            s_buf[slot] = pre ? comp_key(order_key(x[k]), e0 + k) : (unsigned long long)(e0 + k);
+                        ++slot;
+                    }
             }
         }
     }

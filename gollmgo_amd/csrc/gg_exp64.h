@@ -97,7 +97,9 @@ GG_HD64 void gg_exp64_table(double* tab) {
     for (int j = 0; j < 64; ++j) tab[j] = t[j];
 }
 GG_HD64 double gg_fast_exp64_tab(double x, const double* tab) {
-    if (!(x >= -745.2)) return 0.0;
+    // e^-746 is below half the smallest denormal, so the clamp gives 0 for everything under it
+    // (and for NaN) without a branch: a loop over elements then overlaps their table reads.
+    x = __builtin_fmax(x, -746.0);
     const double nd = __builtin_rint(x * (64.0 * 1.4426950408889634));
     double r = __builtin_fma(nd, -6.93147180369123816490e-01 / 64.0, x);
     r = __builtin_fma(nd, -1.90821492927058770002e-10 / 64.0, r);
