@@ -285,52 +285,18 @@ __device__ uint32_t block_excl_scan_u32(uint32_t v, uint32_t* sh, uint32_t* tota
 
 // ------------------------------------------------------------------------ pass
 
-// The draw itself, by one block of NT threads: the segment where u * total falls (sums
-// per segment of the draw's weights), then the element inside it (kSeg / NT per thread). A plain
-// draw's margins are tau * total (e units); a residual's tau * (1 + total) (probability
-// units: the parallel p carries up to tau of error summed over the row, whatever q is). A
-// residual total within a few margins of 0 may be 0 in the rule, whose fallbacks then
-// apply. Undecided: the row is left to the literal rule.
+// The element of segment `seg` where t falls (base: the weights of the segments before it),
+// by one block of NT threads, kSeg / NT elements per thread.
 template <gg_dtype_t DT, int NT>
-__device__ void draw_in_block(const DrawParams& P, int b, const RowInfo& ri, const double* sums,
-                              const double* s_tab) {
+__device__ void draw_in_segment(const DrawParams& P, int b, const RowInfo& ri, int seg, double base, double t,
+                                double marg, const double* s_tab) {
     __shared__ double s_red[16];
-    __shared__ int s_seg, s_tok, s_bad;
-    __shared__ double s_base, s_tot;
-    const double tau = P.tau;
-    const double u = uniform_of(P, b);
-    const int nseg = P.nseg;
-    const double inv_tot = 1.0 / ri.tot;
-    if (threadIdx.x == 0) {
-        double tot = 0.0;
-        for (int s = 0; s < nseg; ++s) tot += sums[s];
-        const double t = u * tot;
-        double run = 0.0;
-        int sel = -1;
-        for (int s = 0; s < nseg; ++s) {
-            if (run + sums[s] > t) {
-                sel = s;
-                break;
-            }
-            run += sums[s];
-        }
-        const double marg = ri.x < 0 ? tau * tot : tau * (1.0 + tot);
-        if (ri.x >= 0 && tot <= 8.0 * marg) sel = -1;
-        if (!(u >= tau && u < 1.0 - tau)) sel = -1;  // near 0, near or past 1, NaN
-        s_seg = sel;
-        s_base = run;
-        s_tot = tot;
+    __shared__ int s_tok, s_bad;
+    if (threadIdx.x == 0) {  // (published by the scan's barriers)
         s_tok = -1;
         s_bad = 0;
     }
-    __syncthreads();
-    const int seg = s_seg;
-    if (seg < 0) {
-        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
-        return;
-    }
-    const double tot = s_tot, t = u * tot;
-    const double marg = ri.x < 0 ? tau * tot : tau * (1.0 + tot);
+    const double inv_tot = 1.0 / ri.tot;
     const void* row = drawn_row(P, b, ri.row);
     const float* qr = q_row(P, b, ri);
     constexpr int kPer = kSeg / NT;
@@ -351,7 +317,7 @@ __device__ void draw_in_block(const DrawParams& P, int b, const RowInfo& ri, con
         loc += ev[q];
     }
     double btot;
-    double run = s_base + block_excl_scan(loc, s_red, &btot);
+    double run = base + block_excl_scan(loc, s_red, &btot);
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
         const double nx = run + ev[q];
@@ -367,6 +333,50 @@ __device__ void draw_in_block(const DrawParams& P, int b, const RowInfo& ri, con
         if (s_tok >= 0 && !s_bad) P.out_tok[b] = s_tok;
         else atomicOr(&P.state[b], ST_EXACT);
     }
+}
+
+// The draw itself, by one block of NT threads: the segment where u * total falls (sums
+// per segment of the draw's weights), then the element inside it (kSeg / NT per thread). A plain
+// draw's margins are tau * total (e units); a residual's tau * (1 + total) (probability
+// units: the parallel p carries up to tau of error summed over the row, whatever q is). A
+// residual total within a few margins of 0 may be 0 in the rule, whose fallbacks then
+// apply. Undecided: the row is left to the literal rule.
+template <gg_dtype_t DT, int NT>
+__device__ void draw_in_block(const DrawParams& P, int b, const RowInfo& ri, const double* sums,
+                              const double* s_tab) {
+    __shared__ int s_seg;
+    __shared__ double s_base, s_tot;
+    const double tau = P.tau;
+    const double u = uniform_of(P, b);
+    const int nseg = P.nseg;
+    if (threadIdx.x == 0) {
+        double tot = 0.0;
+        for (int s = 0; s < nseg; ++s) tot += sums[s];
+        const double t = u * tot;
+        double run = 0.0;
+        int sel = -1;
+        for (int s = 0; s < nseg; ++s) {
+            if (run + sums[s] > t) {
+                sel = s;
+                break;
+            }
+            run += sums[s];
+        }
+        const double marg = ri.x < 0 ? tau * tot : tau * (1.0 + tot);
+        if (ri.x >= 0 && tot <= 8.0 * marg) sel = -1;
+        if (!(u >= tau && u < 1.0 - tau)) sel = -1;  // near 0, near or past 1, NaN
+        s_seg = sel;
+        s_base = run;
+        s_tot = tot;
+    }
+    __syncthreads();
+    const int seg = s_seg;
+    if (seg < 0) {
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+    const double tot = s_tot;
+    draw_in_segment<DT, NT>(P, b, ri, seg, s_base, u * tot, ri.x < 0 ? tau * tot : tau * (1.0 + tot), s_tab);
 }
 
 // Per (segment, sequence): e of every element (the parallel exponential), the segment's
@@ -1207,6 +1217,229 @@ __global__ void __launch_bounds__(kSegThreads) sample_draw_kernel(DrawParams P) 
     draw_seq<DT, kSegThreads>(P, b, P.info[b], nullptr, s_tab);
 }
 
+// ------------------------------------------------- top-p alone, no dense residual
+//
+// The nucleus cut and the draw over the gathered bins, one block per sequence. The general
+// select's radix descent ran a histogram, a scan and seven barriers of sixteen waves per
+// 8-bit digit, added the kept elements of a segment to one LDS word 64 lanes at a time, and
+// walked the segments in one thread. Here one histogram of kFine slices of the gathered
+// range finds the slice the cut lies in, the slice's few elements are ranked by comparing all
+// pairs, and every wave walks the segments by itself. 128 rows of 128256 f32 logits, T 0.8,
+// top-p 0.95 (about 1300 gathered elements each): 34 -> 16.6 µs, latency-bound (a chain of
+// dependent loads, thirty barriers).
+constexpr int kFine = 1024;   // slices of the gathered range
+constexpr int kPairs = 1024;  // most elements of a slice ranked by pairs; more: the radix descent
+
+// Sum and inclusive scan over a wave, the same in every wave that calls them.
+__device__ __forceinline__ double wave_sum(double v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+__device__ __forceinline__ double wave_incl_scan(double v) {
+    const int lane = threadIdx.x & 63;
+    for (int o = 1; o < 64; o <<= 1) {
+        const double t = __shfl_up(v, o);
+        if (lane >= o) v += t;
+    }
+    return v;
+}
+
+template <gg_dtype_t DT>
+__global__ void __launch_bounds__(kTopThreads) sample_topp_draw_kernel(DrawParams P) {
+    const int b = blockIdx.x, lane = threadIdx.x & 63;
+    __shared__ unsigned long long s_comp[kCap];
+    __shared__ double s_e[kCap];
+    __shared__ double s_mass[kFine];
+    __shared__ unsigned long long s_key[kPairs];
+    __shared__ double s_val[kPairs];
+    __shared__ unsigned short s_slice[kCap];
+    __shared__ double s_segk[64];
+    __shared__ double s_tab[64];
+    __shared__ double s_h[257];
+    __shared__ double s_red[16];
+    __shared__ unsigned long long s_u[16];
+    __shared__ int s_i, s_n, s_bin;
+    __shared__ unsigned long long s_cut;
+    __shared__ double s_before, s_A, s_ec;
+    // Every load the row's set-up gives goes out before the first is waited for (a row that is
+    // not drawn leaves them unused).
+    const int st = P.state[b], ng = P.ncand[b];
+    RowInfo ri = P.info[b];
+    constexpr int kAhead = 4;
+    unsigned long long ahead[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) ahead[j] = P.cand[(size_t)b * kCap + j * kTopThreads + threadIdx.x];
+    const bool has = lane < P.nseg;
+    const double segsum = has ? P.segsum[(size_t)b * P.nseg + lane] : 0.0;
+    const double segabove = has ? P.segabove[(size_t)b * P.nseg + lane] : 0.0;
+    if (st != ST_DRAW) return;
+    if (ri.cbin < 0 || ng > kCap) {  // no bin found, or a crowded one: the literal rule decides
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+    const double tau = P.tau, inv_t = P.inv_t, m = ri.m;
+    const int lo = ri.pregather ? ri.cbin_lo : ri.cbin;
+    // (a hint's pass summed the row; without one select1 did, from the histograms)
+    const double S = ri.pregather ? wave_sum(segsum) : ri.S;
+    const double above = ri.pregather ? wave_sum(segabove) : ri.above;
+    const double pS = P.top_p * S, target = pS - above;
+    const double u = uniform_of(P, b);
+    for (int i = threadIdx.x; i < kFine; i += kTopThreads) s_mass[i] = 0.0;
+    if (threadIdx.x < 64) s_segk[threadIdx.x] = 0.0;
+    if (threadIdx.x == 0) {
+        s_i = -1;
+        s_n = 0;
+        s_bin = kFine;
+    }
+    load_exp_table(s_tab);  // (its barrier publishes the words cleared above)
+    // Slice of an element: its distance below the row max, from the top of the gathered bins
+    // down; monotone in the value, equal values in one slice.
+    const double x0 = (double)(kBins - 1 - ri.cbin), fine = (double)kFine / (double)(ri.cbin - lo + 1);
+    for (int i = threadIdx.x, j = 0; i < ng; i += kTopThreads, ++j) {
+        unsigned long long c = 0;
+        if (j < kAhead) {
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q)
+                if (q == j) c = ahead[q];
+        } else {
+            c = P.cand[(size_t)b * kCap + i];
+        }
+        const float l = key_value((uint32_t)(c >> 32));
+        const double e = exp_term(l, inv_t, m);
+        const double f = ((m - (double)l * inv_t) * 64.0 - x0) * fine;
+        const int slice = (int)fmin(fmax(f, 0.0), (double)(kFine - 1));
+        s_comp[i] = c;
+        s_e[i] = e;
+        s_slice[i] = (unsigned short)slice;
+        atomicAdd(&s_mass[slice], e);
+    }
+    __syncthreads();
+    // The first slice whose running mass reaches the target.
+    constexpr int kOwn = kFine / kTopThreads;
+    double v[kOwn], sum = 0.0, all;
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) {
+        v[q] = s_mass[threadIdx.x * kOwn + q];
+        sum += v[q];
+    }
+    double run = block_excl_scan(sum, s_red, &all);
+    // (Rounding may let two slices claim the crossing: the first wins, and its margins fail.)
+    double mine = 0.0;
+    int claim = -1;
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) {
+        if (claim < 0 && run < target && run + v[q] >= target) {
+            claim = (int)threadIdx.x * kOwn + q;
+            mine = run;
+        }
+        run += v[q];
+    }
+    if (claim >= 0) atomicMin(&s_bin, claim);
+    __syncthreads();
+    const int slice = s_bin;
+    if (claim == slice) s_before = mine;
+    if (slice == kFine) {  // uniform: the target lies outside the gathered mass
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+    for (int i = threadIdx.x; i < ng; i += kTopThreads)
+        if ((int)s_slice[i] == slice) {
+            const int n = atomicAdd(&s_n, 1);
+            if (n < kPairs) {
+                s_key[n] = s_comp[i];
+                s_val[n] = s_e[i];
+            }
+        }
+    __syncthreads();
+    const int n = s_n;
+    if (n <= kPairs) {
+        int own = -1;
+        double own_A = 0.0;
+        for (int i = threadIdx.x; i < n; i += kTopThreads) {
+            const unsigned long long c = s_key[i];
+            double A = s_before;
+            for (int t = 0; t < n; ++t) A += s_key[t] > c ? s_val[t] : 0.0;
+            if (A < target && A + s_val[i] >= target) {  // (as above, for two claims: one wins and fails)
+                own = i;
+                own_A = A;
+                atomicMax(&s_i, i);
+            }
+        }
+        __syncthreads();
+        if (own >= 0 && own == s_i) {
+            s_cut = s_key[own];
+            s_A = own_A;
+            s_ec = s_val[own];
+        }
+        __syncthreads();
+        if (s_i < 0) {  // uniform
+            if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+            return;
+        }
+    } else {
+        double A;
+        const int ci = select_desc(s_comp, s_e, ng, target, true, &A, s_h, s_red, &s_i);
+        if (ci < 0) {
+            if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+            return;
+        }
+        if (threadIdx.x == 0) {
+            s_cut = s_comp[ci];
+            s_A = A;
+            s_ec = s_e[ci];
+        }
+        __syncthreads();
+    }
+    const unsigned long long cut = s_cut, nb = next_below(s_comp, ng, cut, s_u);
+    const double A = above + s_A, ec = s_ec;
+    bool ok = (pS - A) > tau * S && (A + ec - pS) > tau * S;
+    // An element after the cut with the same probability but another value would come first
+    // in the rule's (probability desc, index asc) order if its index is lower.
+    if (nb != 0) {
+        if ((nb >> 32) != (cut >> 32) && exp_term(key_value((uint32_t)(nb >> 32)), inv_t, m) == ec) ok = false;
+    } else if (lo > 0 && gg_exp64(-(double)(kBins - lo) / 64.0) >= ec) {  // bound of the bins below
+        ok = false;
+    }
+    if (!(u >= tau && u < 1.0 - tau)) ok = false;  // near 0, near or past 1, NaN
+    if (!ok) {  // uniform
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+    ri.cut = cut;
+    ri.tot = A + ec;
+    // The kept elements by segment. Neighbours in the list come from one segment, so a wave's
+    // lanes take elements far apart.
+    const int per = (ng + 63) / 64;
+    for (int q = threadIdx.x >> 6; q < per; q += kTopThreads / 64) {
+        const int i = lane * per + q;
+        if (i < ng && s_comp[i] >= cut) atomicAdd(&s_segk[comp_index(s_comp[i]) / kSeg], s_e[i]);
+    }
+    __syncthreads();
+    // The segment where u * total falls, by every wave: the kept e, or for a one-hot residual
+    // (kept e - e of the rejected draft) / total.
+    double w = has ? segabove + s_segk[lane] : 0.0;
+    if (ri.x >= 0) {
+        if (ri.x < P.V && ri.x / kSeg == lane) {
+            const float lx = load_as_f32(drawn_row(P, b, ri.row), P.dt, ri.x);
+            if (comp_key(order_key(lx), ri.x) >= cut) w -= fast_term(lx, inv_t, m, s_tab);
+        }
+        w /= ri.tot;
+    }
+    const double inc = wave_incl_scan(w);
+    const double tot = lane_val(inc, 63), t = u * tot;
+    const double marg = ri.x < 0 ? tau * tot : tau * (1.0 + tot);
+    const unsigned long long past = __ballot(has && inc > t);
+    // A residual total within a few margins of 0 may be 0 in the rule.
+    if (past == 0 || (ri.x >= 0 && tot <= 8.0 * marg)) {
+        if (threadIdx.x == 0) atomicOr(&P.state[b], ST_EXACT);
+        return;
+    }
+    const int seg = __ffsll((long long)past) - 1;
+    const double before = __shfl_up(inc, 1);
+    const double base = seg > 0 ? lane_val(before, seg) : 0.0;
+    draw_in_segment<DT, kTopThreads>(P, b, ri, seg, base, t, marg, s_tab);
+}
+
 // ------------------------------------------------------- top-k of at most kTopK
 //
 // The general path summed the mass of every bin, gathered the threshold bin and then, where the
@@ -1841,6 +2074,10 @@ gg_status_t launch_final_draw(const FinalDraw& d, void* ws, hipStream_t s) {
     if (P.filtered && !P.hint_mode) {                                                                \
         sample_select1_kernel<<<B, kRowThreads, 0, s>>>(P);                                          \
         sample_gather_kernel<DTV><<<dim3(P.nseg, B), kSegThreads, 0, s>>>(P);                        \
+    }                                                                                                \
+    if (P.use_p && !P.use_k && !kept) {                                                              \
+        sample_topp_draw_kernel<DTV><<<B, kTopThreads, 0, s>>>(P);                                   \
+        break;                                                                                       \
     }                                                                                                \
     if (P.filtered && !kept) sample_select2_kernel<DTV, true><<<B, kRowThreads, 0, s>>>(P);           \
     if (P.filtered && kept) sample_select2_kernel<DTV, false><<<B, kRowThreads, 0, s>>>(P);           \
