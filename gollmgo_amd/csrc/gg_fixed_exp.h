@@ -26,7 +26,11 @@
 // are exact in double.
 GG_HD float gg_weight_f(float l, float m, float inv_t) {
     const float y = (l - m) * inv_t;
+#ifdef __HIP_DEVICE_COMPILE__
+    const float x = __builtin_amdgcn_fmed3f(y, -80.0f, 0.0f);  // (one instruction; NaN gives the minimum, -80)
+#else
     const float x = __builtin_fminf(y >= -80.0f ? y : -80.0f, 0.0f);  // (the compare maps NaN to -80)
+#endif
     const float kf = __builtin_floorf(__builtin_fmaf(x, 1.44269504088896341f, 0.5f));
     float r = __builtin_fmaf(kf, -0.693145751953125f, x);
     r = __builtin_fmaf(kf, -1.42860682030941723212e-6f, r);
