@@ -45,6 +45,8 @@
 //                             threshold bin (topk_gather, which finds that bin itself), then
 //                             threshold, nucleus and draw over that list in one block
 //                             (topk_draw): no further pass over the row.
+//   top-p alone, q not dense: after the gather (or the hinted pass), the cut and the draw over
+//                             the gathered bins in one block (topp_draw).
 //   exact  (a few blocks)   : the literal rule for the rows flagged on the way.
 #include "gg_common.h"
 #include "gg_exp64.h"
@@ -2056,7 +2058,7 @@ gg_status_t launch_final_draw(const FinalDraw& d, void* ws, hipStream_t s) {
     // Without filters the draw takes the pass's segment sums (a dense residual: the kept
     // launch's). With filters: the bin of the cut (select1), its elements and the sums above
     // it (gather) — both done by the pass when the caller hints the cut — then the cut and
-    // the segment sums (select2); the kept launch only for dense residuals and for a nucleus
+    // the segment sums (topp_draw for top-p alone, which draws too; else select2); the kept launch only for dense residuals and for a nucleus
     // cut above the top-k bin.
     // (A dense residual without filters but with the caller's estimate of S needs none: the
     // pass and the draw form its sums.)
