@@ -377,8 +377,10 @@ struct DeferredRows {
     AppendItem it;
     int j0, j1;
 };
-// Most work items (rows x 16 dim groups) a piece stages in LDS: 8 draft rows.
-constexpr int kAppMax = 128;
+// Most draft rows a piece stages in LDS, at any head_dim: the V staging holds a dim's rows in 16
+// bytes, eight of a 2-byte pool, and the patch shifts them as one 128-bit value.
+constexpr int kAppRows = 8;
+static_assert(kAppRows * 2 <= (int)sizeof(uint4), "a dim's staged rows are one 16-byte word");
 
 // Start piece d (PieceIO::start) and, when the call carries draft rows (a.k_new), take
 // care of the rows whose key positions lie in the piece. A key position belongs to exactly
@@ -386,7 +388,7 @@ constexpr int kAppMax = 128;
 // chunks are multiples of 16 tokens, so a block's tokens (its K rows and its V columns)
 // are all read by one chunk, and so by one wave.
 //   - Rows inside the first chunks that `start` issues (short pieces), more rows than
-//     kAppMax, no `ap` (the stream-K loop over pieces, whose registers are full), or a
+//     kAppRows, no `ap` (the stream-K loop over pieces, whose registers are full), or a
 //     PER_BLOCK INT8 pool (a block's new rows re-scale the whole block; a block lies in one
 //     piece, since pieces are whole chunks): appended here by the whole workgroup, then a
 //     barrier orders the stores before the piece's loads (within a workgroup a barrier
@@ -413,7 +415,8 @@ __device__ __forceinline__ void start_piece(const AttnArgs& a, const KVView& kv,
         const int j0 = max(0, d.t0 - first), j1 = min(nrows, d.t_end - first);
         if (nrows > 0 && nrows <= ctx && j0 < j1) {
             const int items = (j1 - j0) * (HD / 8);
-            if (kDefer && ap && items <= kAppMax && first + j0 >= d.t0 + kWaves * kTok) {
+            static_assert(kAppRows * (HD / 8) <= 256, "one work item per thread");
+            if (kDefer && ap && j1 - j0 <= kAppRows && first + j0 >= d.t0 + kWaves * kTok) {
                 PieceIO<DT, TOK, HD>::start(kv, d, fb, in);
                 ap->j0 = j0;
                 ap->j1 = j1;
@@ -552,7 +555,7 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
     // stores (on gfx950 stores count in vmcnt, so a store ahead of a chunk's loads would
     // hold up the wait for that chunk). s_app keeps each work item (row, 8 dims) in the
     // pool's format; s_vt the same V values by dim: element r of s_vt[d] is row r's V[d].
-    __shared__ AppendBytes s_app[kAppMax];
+    __shared__ AppendBytes s_app[kAppRows * (HD / 8)];
     __shared__ uint4 s_vt[HD];
     int app_lo = 0, app_hi = 0;  // their key positions [app_lo, app_hi)
     if constexpr (DT != GG_DTYPE_INT8) {
@@ -1022,7 +1025,7 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
                     for (int dt = 0; dt < Geom::kDT; ++dt) {
                         const uint4 sv = s_vt[dt * 16 + c16];
                         u128 nv = ((u128)sv.w << 96) | ((u128)sv.z << 64) | ((u128)sv.y << 32) | sv.x;
-                        if (kEB == 1) nv &= ((u128)1 << 64) - 1;  // 8 staged rows of one byte
+                        if (kEB == 1) nv &= ((u128)1 << (8 * kAppRows)) - 1;  // (staged rows of one byte)
                         nv = base < 0 ? nv << ((-base) * kE) : nv >> (base * kE);
                         const uint4 c = cur.v[dt];
                         u128 cv = ((u128)c.w << 96) | ((u128)c.z << 64) | ((u128)c.y << 32) | c.x;

@@ -72,3 +72,19 @@ def test_append_attention_equals_append_then_attention(gpu, monkeypatch, dt, Hq,
     # re-quantises whatever bytes they hold.)
     _fused_vs_separate(99, dt, B, ("uniform", *ctx), dt != "int8")
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "fp8"])
+@pytest.mark.parametrize("R", [8, 9, 12, 16])
+@pytest.mark.parametrize("Hq,H,D", [(4, 4, 64), (8, 4, 64), (16, 4, 64), (8, 1, 128)])
+def test_append_attention_around_the_staged_rows(gpu, monkeypatch, dt, R, Hq, H, D):
+    """Draft rows at the number a piece stages in LDS and above it (appended before the piece's
+    loads there), for one to four row tiles: rows that start at block offsets 0, 4 and 13, in and
+    past the first chunks, all rows or ragged counts; pool bytes and outputs bit for bit."""
+    ctx = (40, 320, 324, 333, 896, 900, 909)
+    say(f"rows fused append around the staged rows dt={dt} R={R} Hq={Hq} H={H} D={D}")
+    monkeypatch.setitem(CONFIGS, 99, VerifyConfig("rows", len(ctx), R - 1, Hq, H, D, 16, ("list", *ctx), dt, "bf16", 1000,
+                                                  "f32", "greedy", seed=D + R))
+    for rc in (False, True):
+        _fused_vs_separate(99, dt, len(ctx), ("list", *ctx), rc)
+    torch.cuda.empty_cache()
