@@ -369,13 +369,22 @@ size_t attn_workspace_bytes(const KV* kv, int num_seqs, int rows, int num_q_head
 gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
     const KV* kv = a.kv;
     KVView view = make_kv_view(kv, a.layer);
-    const bool mfma = a.sched != ATTN_SCHED_GRID || (attn_mfma_supported(kv, a.rows, a.num_q_heads) &&
-                                                     a.partition % 64 == 0 && a.partition <= kMfmaMaxPartition);
+    const bool mfma = attn_mfma_scale(a.scale) &&
+                      (a.sched != ATTN_SCHED_GRID || (attn_mfma_supported(kv, a.rows, a.num_q_heads) &&
+                                                      a.partition % 64 == 0 && a.partition <= kMfmaMaxPartition));
     // Draft rows of the call: the MFMA kernels append them piece by piece (start_piece);
     // the generic path takes a launch of its own first.
     bool combine = true;  // (the partition grid's merge launch)
     // So do the row groups of an INT8 item: each would re-quantise the block it appends to.
     AttnArgs m = a;
+    if (!mfma && a.sched != ATTN_SCHED_GRID) {
+        // A planned shape at another scale: partitions that one workgroup merges, which need none
+        // of the workspace. (The schedules' shapes have head_dim 64 or 128.)
+        const long long keys = (long long)a.max_blocks * kv->block_size;
+        m.sched = ATTN_SCHED_GRID;
+        m.partition = (int)(((keys + kFuseParts - 1) / kFuseParts + 63) / 64 * 64);
+        m.max_parts = (int)((keys + m.partition - 1) / m.partition);
+    }
     if (a.k_new && (!mfma || (a.row_groups > 1 && kv->dtype == GG_DTYPE_INT8))) {
         const gg_status_t st = launch_append_from_tables(a, view, s);
         if (st != GG_OK) return st;
@@ -395,24 +404,24 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
         // runs of a tile fit its registers. Every partition of a row in one workgroup: few
         // partitions, few enough dims for the LDS they meet in.
         const bool vrun = kv->block_size * dtype_bytes(kv->dtype) % 16 == 0 && 64 % kv->block_size == 0 && DC <= 2;
-        const bool fused = a.max_parts <= kFuseParts && DC <= 2;
-        const dim3 grid(fused ? 1 : a.max_parts, a.num_q_heads, a.num_seqs * a.rows);
-        const int threads = fused ? 64 * a.max_parts : 64;
+        const bool fused = m.max_parts <= kFuseParts && DC <= 2;
+        const dim3 grid(fused ? 1 : m.max_parts, m.num_q_heads, m.num_seqs * m.rows);
+        const int threads = fused ? 64 * m.max_parts : 64;
         auto launch = [&](auto dt_tag) {
             constexpr gg_dtype_t DT = decltype(dt_tag)::value;
             auto small = [&](auto dc_tag) {
                 constexpr int N = decltype(dc_tag)::value;
-                if (vrun && fused) attn_generic_kernel<DT, N, true, true><<<grid, threads, 0, s>>>(a, view);
-                else if (vrun) attn_generic_kernel<DT, N, true, false><<<grid, threads, 0, s>>>(a, view);
-                else if (fused) attn_generic_kernel<DT, N, false, true><<<grid, threads, 0, s>>>(a, view);
-                else attn_generic_kernel<DT, N, false, false><<<grid, threads, 0, s>>>(a, view);
+                if (vrun && fused) attn_generic_kernel<DT, N, true, true><<<grid, threads, 0, s>>>(m, view);
+                else if (vrun) attn_generic_kernel<DT, N, true, false><<<grid, threads, 0, s>>>(m, view);
+                else if (fused) attn_generic_kernel<DT, N, false, true><<<grid, threads, 0, s>>>(m, view);
+                else attn_generic_kernel<DT, N, false, false><<<grid, threads, 0, s>>>(m, view);
             };
             switch (DC) {
                 case 1: small(std::integral_constant<int, 1>{}); break;
                 case 2: small(std::integral_constant<int, 2>{}); break;
-                case 4: attn_generic_kernel<DT, 4, false, false><<<grid, threads, 0, s>>>(a, view); break;
-                case 8: attn_generic_kernel<DT, 8, false, false><<<grid, threads, 0, s>>>(a, view); break;
-                default: attn_generic_kernel<DT, 16, false, false><<<grid, threads, 0, s>>>(a, view); break;
+                case 4: attn_generic_kernel<DT, 4, false, false><<<grid, threads, 0, s>>>(m, view); break;
+                case 8: attn_generic_kernel<DT, 8, false, false><<<grid, threads, 0, s>>>(m, view); break;
+                default: attn_generic_kernel<DT, 16, false, false><<<grid, threads, 0, s>>>(m, view); break;
             }
         };
         combine = !fused;
@@ -425,8 +434,8 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
             default: return fail(GG_ERR_INVALID, "attention: pool dtype");
         }
     }
-    if (combine && a.max_parts > 1) {
-        attn_combine_kernel<<<dim3(a.num_q_heads, a.num_seqs * a.rows), 128, 0, s>>>(a, kv->head_dim);
+    if (combine && m.max_parts > 1) {
+        attn_combine_kernel<<<dim3(m.num_q_heads, m.num_seqs * m.rows), 128, 0, s>>>(m, kv->head_dim);
     }
     static_assert(kMaxDC == 16, "generic kernel instantiations cover head_dim <= 1024");
     return check_hip(hipGetLastError(), "verify_attention launch");

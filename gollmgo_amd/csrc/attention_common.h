@@ -94,6 +94,12 @@ inline bool attn_mfma_supported(const KV* kv, int rows, int num_q_heads) {
             kv->dtype == GG_DTYPE_FP8_E4M3 || kv->dtype == GG_DTYPE_INT8);
 }
 
+// The MFMA kernels' softmax takes the score multiplier as positive: the maximum of the scaled
+// scores is the scaled maximum, and a masked score stays -inf (times 0 it would be NaN). Any other
+// scale, or one so small that it may underflow times a block scale (f16, from 2^-24), runs the
+// per-row kernel, which scales each score by itself.
+inline bool attn_mfma_scale(float scale) { return scale >= 0x1p-100f; }
+
 // MFMA kernel workgroups (of four waves) per CU for a pool's element size and row-tile
 // count: two while one wave's registers fit half the file (one or two row tiles; three
 // row tiles of a 1-byte pool in 32-token chunks, 217-248 VGPRs; head_dim 64), else one. Shared by the

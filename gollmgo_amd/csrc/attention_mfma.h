@@ -677,6 +677,8 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
                     s_q[part][rt][mm][lane] = make_uint4(h[0], h[1], h[2], h[3]);
                 }
             }
+            // (Positive, whatever the head's scale and the queries' made of it: attn_mfma_scale.)
+            sscale = fmaxf(sscale, 0x1p-126f);
             __syncthreads();
         } else {
         // One uniform dtype branch around all row tiles, so their loads issue together.

@@ -135,7 +135,7 @@ def test_append_random_cases(gpu, seed):
 # ------------------------------------------------------------------ attention
 
 def run_attention_case(dt, B, R, Hq, H, D, bs, ctx, partition=0, src="f32", seed=0, q_dt="f32",
-                       row_counts=None, kv_sd=1.0, q_sd=1.0, v_sd=None):
+                       row_counts=None, kv_sd=1.0, q_sd=1.0, v_sd=None, scale=None):
     rng = np.random.default_rng(seed)
     keys = np.asarray(ctx, np.int32) + R
     nbs = [(int(k) + bs - 1) // bs for k in keys]
@@ -165,7 +165,7 @@ def run_attention_case(dt, B, R, Hq, H, D, bs, ctx, partition=0, src="f32", seed
     rc_t = torch.from_numpy(np.asarray(row_counts, np.int32)).cuda() if row_counts is not None else None
     if row_counts is not None:
         keys = np.asarray(ctx, np.int32) + np.asarray(row_counts, np.int32)
-    scale = 1.0 / math.sqrt(D)
+    scale = 1.0 / math.sqrt(D) if scale is None else scale
     kv.attention(0, qt, out, torch.from_numpy(keys).cuda(), torch.from_numpy(bt).cuda(), scale,
                  row_counts=rc_t, partition_tokens=partition)
     torch.cuda.synchronize()
@@ -774,7 +774,7 @@ def test_append_attention_fused_with_missing_blocks(gpu, dt):
     _fused_vs_separate(3 if dt == "fp8" else 5, dt, 64, ("uniform", 300, 3000), False, corrupt=True)
 
 
-def _fused_vs_separate(cid, dt, B, ctx, rc, corrupt=False):
+def _fused_vs_separate(cid, dt, B, ctx, rc, corrupt=False, scale=None):
     cfg = scaled(CONFIGS[cid], num_seqs=B, ctx=ctx, layers=1, kv_dtype=dt)
     lay = build_layout(cfg)
     H, D, bs, R, Hq = cfg.num_kv_heads, cfg.head_dim, cfg.block_size, cfg.rows, cfg.num_q_heads
@@ -787,6 +787,7 @@ def _fused_vs_separate(cid, dt, B, ctx, rc, corrupt=False):
             pos = int(lay.keys[b_]) - 1
             tables[b_, pos // bs] = lay.num_blocks + 3 if b_ % 2 else -2
         lay = type(lay)(**{**lay.__dict__, "block_tables": tables})
+    scale = 1 / math.sqrt(D) if scale is None else scale
     gen = torch.Generator(device="cuda").manual_seed(cfg.seed + 11)
     fill = torch.from_numpy(lay.fill_slots).cuda()
     kx = torch.randn(len(fill), H, D, device="cuda", dtype=torch.bfloat16, generator=gen)
@@ -813,10 +814,10 @@ def _fused_vs_separate(cid, dt, B, ctx, rc, corrupt=False):
         kv.attention_plan(keys, R, Hq, bt.shape[1], ws, row_counts=rc_t)
         out = torch.zeros(q.shape, dtype=torch.float32, device="cuda")
         if fused:
-            kv.append_attention(0, k_new, v_new, q, out, keys, bt, 1 / math.sqrt(D), ws, row_counts=rc_t)
+            kv.append_attention(0, k_new, v_new, q, out, keys, bt, scale, ws, row_counts=rc_t)
         else:
             kv.append(0, k_new, v_new, torch.from_numpy(slots).cuda())
-            kv.attention(0, q, out, keys, bt, 1 / math.sqrt(D), row_counts=rc_t, workspace=ws, planned=True)
+            kv.attention(0, q, out, keys, bt, scale, row_counts=rc_t, workspace=ws, planned=True)
         torch.cuda.synchronize()
         sc = kv.scales(0) if dt in ("fp8", "int8") else (torch.zeros(1), torch.zeros(1))
         results.append((kv.k_pool(0).cpu().numpy(), kv.v_pool(0).cpu().numpy(), out.cpu().numpy(),

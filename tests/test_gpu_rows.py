@@ -1,12 +1,14 @@
 """GPU parity of the MFMA attention for head_dim 64 and for more than 64 query rows per kv head
 (row groups), against the float64 oracle and against the per-row kernel it took over from
 (an explicit partition still runs that one): no less exact, for every pool and query type."""
+import math
+
 import pytest
 import torch
 
 from gollmgo_amd.workloads import CONFIGS, VerifyConfig
 from helpers import TOL, say
-from test_gpu_kv import _fused_vs_separate, run_attention_case
+from test_gpu_kv import _fused_vs_separate, make_cache, run_attention_case
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +90,27 @@ def test_append_attention_around_the_staged_rows(gpu, monkeypatch, dt, R, Hq, H,
     for rc in (False, True):
         _fused_vs_separate(99, dt, len(ctx), ("list", *ctx), rc)
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "fp8", "int8"])
+@pytest.mark.parametrize("shape", [0, 1, 3, 5, 6, 7])
+def test_any_finite_scale(gpu, dt, shape):
+    """Softmax scales at and below zero, and so small that the score multiplier underflows:
+    masked keys stay masked, a negative scale turns the order of the scores round."""
+    B, R, Hq, H, D, ctx = (SHAPES + [(2, 5, 16, 2, 128, [40, 700])])[shape]  # (the last: 40 rows at head_dim 128)
+    for scale in (0.0, -0.0, -0.125, 1e-44, -1e-44):
+        for q_dt in ("bf16", "f16", "f32"):
+            say(f"rows dt={dt} q={q_dt} scale={scale} shape={shape}")
+            err = run_attention_case(dt, B, R, Hq, H, D, 16, ctx, src="bf16", q_dt=q_dt, seed=70 + shape, scale=scale)
+            assert err <= TOL[dt]
+
+
+@pytest.mark.parametrize("dt", ["f16", "fp8", "int8"])
+@pytest.mark.parametrize("Hq,H,D,R", [(16, 4, 64, 9), (32, 2, 128, 5), (16, 4, 128, 5)])
+def test_append_attention_at_a_negative_scale(gpu, monkeypatch, dt, Hq, H, D, R):
+    """A planned call at such a scale appends its rows and leaves the plan as it was."""
+    ctx = (40, 333, 900)
+    say(f"rows fused append at a negative scale dt={dt} Hq={Hq} H={H} D={D} R={R}")
+    monkeypatch.setitem(CONFIGS, 99, VerifyConfig("rows", len(ctx), R - 1, Hq, H, D, 16, ("list", *ctx), dt, "bf16", 1000,
+                                                  "f32", "greedy", seed=D + R))
+    _fused_vs_separate(99, dt, len(ctx), ("list", *ctx), False, scale=-0.125)
