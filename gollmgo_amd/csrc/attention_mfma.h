@@ -37,6 +37,7 @@
 #pragma once
 #include "gg_common.h"
 #include "attention_common.h"
+#include "attention_rows.h"
 
 #include <type_traits>
 
@@ -458,6 +459,9 @@ __device__ __forceinline__ float2 load_agent2(const float* p) {
         __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
 }
+__device__ __forceinline__ void store_agent(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void store_agent2(float* p, float a, float b) {
     const unsigned long long v = ((unsigned long long)__float_as_uint(b) << 32) | __float_as_uint(a);
     __hip_atomic_store((unsigned long long*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -503,6 +507,42 @@ __device__ __forceinline__ QRaw<NT> load_q16(const AttnArgs& a, const KVView& kv
         q.v[rt] = ((const U4*)((const uint16_t*)a.q + i))->v;
     }
     return q;
+}
+
+// The piece by the per-row kernel's steps, a row per wave and round: for pieces whose sums are not
+// finite (attn_piece). s_row: HD query elements and 64 probabilities per wave. rec_rows: rows per
+// record.
+template <gg_dtype_t DT, int HD>
+__device__ __forceinline__ void piece_by_rows(const AttnArgs& a, const KVView& kv, const PieceDesc& d, int rows, int rec_rows,
+                                              float* s_row) {
+    constexpr int kDC = HD / 64;
+    const int G = a.num_q_heads / kv.Hkv, lane = threadIdx.x & 63;
+    float* s_q = s_row;
+    float* s_p = s_row + HD;
+    for (int r = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); r < rows; r += kWaves) {
+        const int j = (d.row0 + r) / G, g = (d.row0 + r) % G;
+        const size_t obase = (((size_t)d.b * a.rows + j) * a.num_q_heads + (size_t)d.kvh * G + g) * HD;
+        __builtin_amdgcn_wave_barrier();  // (the previous row's reads)
+#pragma unroll
+        for (int c = 0; c < kDC; ++c) s_q[lane + 64 * c] = load_as_f32(a.q, a.q_dtype, obase + lane + 64 * c);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        float acc[kDC], m, l;
+        generic_partition<DT, kDC, true>(a, kv, d.b, d.kvh, d.t0, min(d.t_end, d.ctx - d.nrows + j + 1), s_q, s_p, nullptr,
+                                         acc, m, l);
+        if (d.rec < 0) {
+            const float inv = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+            for (int c = 0; c < kDC; ++c) store_from_f32(a.out, a.out_dtype, obase + lane + 64 * c, acc[c] * inv);
+        } else {
+            const size_t q = (size_t)d.rec * rec_rows + r;
+            constexpr float kUnit = DT == GG_DTYPE_F16 ? 16384.f : 1.f;  // (P in units of 2^-14)
+#pragma unroll
+            for (int c = 0; c < kDC; ++c) store_agent(a.ws_acc + q * HD + lane + 64 * c, acc[c] * kUnit);
+            if (lane == 0) store_agent2(a.ws_ml + q * 2, m, l * kUnit);
+        }
+    }
 }
 
 template <gg_dtype_t DT, int NT, int HD, bool FULL>
@@ -1103,7 +1143,27 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
             s_l[wave][rt * 16 + c16] = lt;
         }
     }
-    __syncthreads();
+    if constexpr (FULL) {
+        // A NaN or infinity among the queries, keys or values reaches rows that it should not
+        // touch: a hidden key's P is 0, and 0 times it is NaN; the parts of P give infinities of
+        // both signs; an infinite query sets the scale of the piece's other queries. Each leaves a
+        // sum that is not finite, and the piece is then computed row by row.
+        float z = 0.f;
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt) {
+            z = __builtin_fmaf(l_run[rt], 0.f, z);
+#pragma unroll
+            for (int dt = 0; dt < Geom::kDT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) z = __builtin_fmaf(o[rt][dt][i], 0.f, z);
+        }
+        if (__builtin_expect(__syncthreads_or(z != 0.f), 0)) {
+            piece_by_rows<DT, HD>(a, kv, pd, min(nvalid_rows, 16 * NT), 16 * NT, &s_o[wave][0][0]);
+            return;
+        }
+    } else {
+        __syncthreads();
+    }
 
     const size_t zbase = (size_t)b * R;
     for (int rt = 0; rt < NT; ++rt) {

@@ -1,5 +1,6 @@
 // attention_rows.h — one partition of one (row, head) of the verify attention by one wave, keys
-// and dims in fp32: the phase-1 step of the per-row kernel.
+// and dims in fp32: the phase-1 step of the per-row kernel, and of pieces of the MFMA kernels
+// that are computed row by row (piece_by_rows).
 #pragma once
 #include "gg_common.h"
 #include "attention_common.h"

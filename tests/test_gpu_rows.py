@@ -114,3 +114,79 @@ def test_append_attention_at_a_negative_scale(gpu, monkeypatch, dt, Hq, H, D, R)
     monkeypatch.setitem(CONFIGS, 99, VerifyConfig("rows", len(ctx), R - 1, Hq, H, D, 16, ("list", *ctx), dt, "bf16", 1000,
                                                   "f32", "greedy", seed=D + R))
     _fused_vs_separate(99, dt, len(ctx), ("list", *ctx), False, scale=-0.125)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "fp8", "int8"])
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_values_that_are_not_finite(gpu, dt, shape):
+    """NaN and infinities in the K and V of draft rows, in the context's V and in a query row reach
+    the rows that the per-row kernel lets them reach, and no other; the append inside the call too."""
+    B, R, Hq, H, D, ctx = SHAPES[shape]
+    bs, inf, nan = 16, float("inf"), float("nan")
+    gen = torch.Generator(device="cuda").manual_seed(80 + shape)
+    keys = [c + R for c in ctx]
+    nbs = [(n + bs - 1) // bs for n in keys]
+    bt = torch.zeros(B, max(nbs), dtype=torch.int32)
+    slots, first = [], 1
+    for b in range(B):
+        bt[b, :nbs[b]] = torch.arange(first, first + nbs[b])
+        slots += [first * bs + t for t in range(keys[b])]
+        first += nbs[b]
+    draft = [sum(keys[:b]) + ctx[b] + j for b in range(B) for j in range(R)]
+    slots, draft = torch.tensor(slots, dtype=torch.int32).cuda(), torch.tensor(draft).cuda()
+    bt, kt = bt.cuda(), torch.tensor(keys, dtype=torch.int32).cuda()
+    src = torch.float16 if dt == "f16" else torch.bfloat16
+    for case in ("v nan", "v inf", "v both", "k nan", "context v", "q inf"):
+        if dt == "int8" and case != "q inf":
+            continue  # (a byte holds neither)
+        if dt == "fp8" and case not in ("v nan", "k nan", "q inf"):
+            continue  # (infinities saturate)
+        for q_dt in (torch.bfloat16, torch.float32):
+            say(f"rows not finite dt={dt} shape={shape} {case} q={q_dt}")
+            kx, vx = (torch.randn(len(slots), H, D, device="cuda", generator=gen).to(src) for _ in range(2))
+            q = torch.randn(B, R, Hq, D, device="cuda", generator=gen).to(q_dt)
+            last = draft[R - 1::R]  # (each sequence's last row)
+            if case in ("v nan", "v both"):
+                vx[last, :, 3] = nan
+            if case in ("v inf", "v both"):
+                vx[draft[R // 2::R], 0, 5:7] = inf
+                vx[last, -1, 5] = -inf
+            if case == "k nan":
+                kx[last, -1, 7] = nan
+            if case == "context v":
+                vx[draft[0::R] // 2, 0, 9] = inf
+            if case == "q inf":
+                q, kx = q * 1e5, kx * 1e-5
+                q[:, R // 2, Hq // 2, 1] = inf
+            outs = []
+            for mode in ("per-row", "separate", "fused"):
+                kv = make_cache(dt, H, D, bs, first)
+                if dt == "fp8":
+                    kv.set_head_scales(0, [1e-7 if case == "q inf" else 0.01] * H, [0.01] * H)
+                context = torch.ones(len(slots), dtype=torch.bool, device="cuda")
+                context[draft] = False
+                for rows in (context, ~context)[:1 if mode == "fused" else 2]:
+                    if rows.any():
+                        kv.append(0, kx[rows].contiguous(), vx[rows].contiguous(), slots[rows].contiguous())
+                out = torch.zeros(B, R, Hq, D, device="cuda")
+                if mode == "per-row":
+                    kv.attention(0, q, out, kt, bt, D ** -0.5, partition_tokens=64)
+                else:
+                    ws = kv.attention_workspace(B, R, Hq, bt.shape[1], 0)
+                    kv.attention_plan(kt, R, Hq, bt.shape[1], ws)
+                    if mode == "fused":
+                        new = [x[draft].contiguous() for x in (kx, vx)]
+                        kv.append_attention(0, *new, q, out, kt, bt, D ** -0.5, ws)
+                    else:
+                        kv.attention(0, q, out, kt, bt, D ** -0.5, workspace=ws, planned=True)
+                torch.cuda.synchronize()
+                outs.append(out.cpu())
+                kv.close()
+            ref = outs[0]
+            assert case == "v nan" or ref.isfinite().any(), case
+            for got in outs[1:]:
+                for f in (torch.isnan, torch.isposinf, torch.isneginf):
+                    assert torch.equal(f(got), f(ref)), (case, f)
+                fin = ref.isfinite()
+                # (Outputs below 5, each side within 2e-6 of its largest.)
+                assert (got[fin] - ref[fin]).abs().max() <= 2e-5, case
