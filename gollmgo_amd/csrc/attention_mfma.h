@@ -537,10 +537,9 @@ __device__ __forceinline__ void piece_by_rows(const AttnArgs& a, const KVView& k
             for (int c = 0; c < kDC; ++c) store_from_f32(a.out, a.out_dtype, obase + lane + 64 * c, acc[c] * inv);
         } else {
             const size_t q = (size_t)d.rec * rec_rows + r;
-            constexpr float kUnit = DT == GG_DTYPE_F16 ? 16384.f : 1.f;  // (P in units of 2^-14)
 #pragma unroll
-            for (int c = 0; c < kDC; ++c) store_agent(a.ws_acc + q * HD + lane + 64 * c, acc[c] * kUnit);
-            if (lane == 0) store_agent2(a.ws_ml + q * 2, m, l * kUnit);
+            for (int c = 0; c < kDC; ++c) store_agent(a.ws_acc + q * HD + lane + 64 * c, acc[c]);
+            if (lane == 0) store_agent2(a.ws_ml + q * 2, m, l);
         }
     }
 }
@@ -553,7 +552,7 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
     using T = PoolTraits<DT>;
     // FULL: FP8 and INT8 values go through bf16 as well, whose range holds any block scale.
     constexpr bool kIsBf16 = FULL ? DT != GG_DTYPE_F16 : T::kBf16;
-    constexpr int kNP_parts = FULL ? (kIsBf16 ? 3 : 2) : (kIsBf16 ? 2 : 1);  // operands P is split into
+    constexpr int kNP_parts = FULL ? 3 : kIsBf16 ? 2 : 1;  // operands P is split into
     constexpr int kEB = T::kEB;
     constexpr int TOK = attn_chunk_tokens(kEB, NT);
     using Geom = Geo<kEB, TOK, HD>;
@@ -582,7 +581,8 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
 
     // Score multiplier (log2 domain) and P.V multiplier per pool type.
     float sscale = a.scale * kLog2e;
-    float vfold = 1.f;
+    constexpr float kPUnits = 16384.f;  // FULL with f16 operands: P is multiplied in units of 2^-14
+    float vfold = FULL && !kIsBf16 ? 1.f / kPUnits : 1.f;
     if constexpr (DT == GG_DTYPE_FP8_E4M3) {
         sscale *= kv.k_head_scale[kvh];
         vfold = kv.v_head_scale[kvh];
@@ -974,14 +974,12 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
             }
             cmax = max_over_rows(cmax * mult);
             const float m_new = fmaxf(m_run[rt], cmax);
-            // FULL with f16 operands: P in units of 2^-14, so that its f16 parts stay normal.
-            const float m_exp = FULL && !kIsBf16 ? m_new - 14.f : m_new;
             const float alpha = __builtin_amdgcn_exp2f(m_run[rt] - m_new);
             m_run[rt] = m_new;
             float psum = 0.f;
 #pragma unroll
             for (int k = 0; k < kNP; ++k) {
-                sc[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[k], mult, -m_exp));
+                sc[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[k], mult, -m_new));
                 psum += sc[k];
             }
             l_run[rt] = l_run[rt] * alpha + psum;
@@ -1003,10 +1001,11 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
             for (int pv = 0; pv < Geom::kNPV; ++pv) {
                 const float* pp = sc + 8 * pv;
                 if constexpr (FULL) {
-                    // P as bf16 hi + mid + lo or f16 hi + lo: no fewer bits than the fp32 sums.
+                    // P as hi + mid + lo: three bf16 parts hold all 24 bits, three f16 ones those
+                    // above 2^-39 (in units of 2^-14 the smallest f16 is 2^-38).
                     float x[8];
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) x[k] = pp[k];
+                    for (int k = 0; k < 8; ++k) x[k] = kIsBf16 ? pp[k] : pp[k] * kPUnits;
 #pragma unroll
                     for (int part = 0; part < kNP_parts; ++part) {
                         uint32_t h[4];

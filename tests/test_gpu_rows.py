@@ -38,6 +38,27 @@ def test_no_less_exact_than_the_per_row_kernel(gpu, dt, shape):
         assert err <= max(2 * ref, 2e-6), (err, ref)
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16", "fp8", "int8"])
+def test_mean_error_of_the_per_row_kernel(gpu, monkeypatch, dt):
+    """The error's 2-norm over all shapes and query types, which averages over the roundings of some
+    hundred thousand outputs: no larger than the per-row kernel's."""
+    import test_gpu_kv
+
+    sums = {}
+
+    def norms(got, ref):
+        return float(((got.astype("f8") - ref) ** 2).sum() / (ref.astype("f8") ** 2).sum())
+
+    monkeypatch.setattr(test_gpu_kv, "rel_err_per_vector", norms)
+    for q_dt in ("bf16", "f16", "f32"):
+        say(f"rows mean error dt={dt} q={q_dt}")
+        for part in (0, 64):
+            sums[part] = sum(run_attention_case(dt, B, R, Hq, H, D, 16, ctx, src="bf16", q_dt=q_dt, seed=90 + i, partition=part)
+                             for i, (B, R, Hq, H, D, ctx) in enumerate(SHAPES)) ** 0.5
+        print(f"  {sums[0]:.2e}, per-row kernel {sums[64]:.2e}")
+        assert sums[0] <= 1.02 * sums[64], (q_dt, sums)  # (two estimates of a rounding error)
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("q_sd", [1e-6, 1e6])
 def test_queries_far_from_one(gpu, dt, q_sd):
