@@ -16,7 +16,7 @@
 // over nine shapes, as a share of the per-row kernel's, for bf16 / f16 / f32 queries: BF16
 // pools 0.77 / 0.89 / 0.83, F16 0.75 / 0.67 / 0.68, FP8 0.80 / 0.89 / 0.84, INT8 0.81 / 0.86 /
 // 0.82. (F16 with two parts of P, and the 2^14 inside the exponent, where it takes four of the
-// argument's bits: 1.38 / 1.20 / 0.99, for 0.4 µs a call less at head_dim 64.)
+// argument's bits: 1.38 / 1.20 / 0.99, for 0.1 µs a call less at head_dim 64.)
 #include "attention_mfma.h"
 
 namespace gg {

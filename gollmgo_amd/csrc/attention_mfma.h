@@ -1142,6 +1142,7 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
             s_l[wave][rt * 16 + c16] = lt;
         }
     }
+    __shared__ int s_bad[FULL ? kWaves : 1];
     if constexpr (FULL) {
         // A NaN or infinity among the queries, keys or values reaches rows that it should not
         // touch: a hidden key's P is 0, and 0 times it is NaN; the parts of P give infinities of
@@ -1156,12 +1157,15 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, const KVView& kv, 
 #pragma unroll
                 for (int i = 0; i < 4; ++i) z = __builtin_fmaf(o[rt][dt][i], 0.f, z);
         }
-        if (__builtin_expect(__syncthreads_or(z != 0.f), 0)) {
+        const bool any = __any(z != 0.f);
+        if (lane == 0) s_bad[wave] = any;
+    }
+    __syncthreads();
+    if constexpr (FULL) {
+        if (__builtin_expect(s_bad[0] | s_bad[1] | s_bad[2] | s_bad[3], 0)) {
             piece_by_rows<DT, HD>(a, kv, pd, min(nvalid_rows, 16 * NT), 16 * NT, &s_o[wave][0][0]);
             return;
         }
-    } else {
-        __syncthreads();
     }
 
     const size_t zbase = (size_t)b * R;
