@@ -344,11 +344,15 @@ __global__ void __launch_bounds__(256) append_int8_block_kernel(AppendArgs a) {
 
 // ---- block size 16: whole block runs ----
 //
-// The rows that follow each other in one block (a run, led by its first row; skipped rows do
-// not break it) are written by one workgroup per kv head as one tile: 16-byte source loads, K
-// rows stored whole, V transposed in LDS so that a dim's 16 offsets leave as one 16-byte store
-// (partial runs: the 4-byte words that are whole, the rest by element). INT8 pools follow
-// append_int8_block_kernel's rule for the run.
+// The rows that follow each other in one block (a run, led by its first row) are written by one
+// workgroup per kv head as one tile: 16-byte source loads, K rows stored whole, V transposed in
+// LDS so that a dim's 16 offsets leave as one 16-byte store (partial runs: the 4-byte words that
+// are whole, the rest by element). INT8 pools follow append_int8_block_kernel's rule for the run:
+// no number of skipped rows breaks it, so its ends may lie anywhere and are walked to, 256 rows a
+// step. In the other pools a block may be written in any number of runs, and kRunGap skipped rows
+// break one: every run lies in the slot window of its leader's workgroup, whatever is skipped
+// around it. 100 rows before 8092 skipped ones, FP8 / INT8: 1113 / 1103 µs when one thread walked,
+// 9.5 / 2367 in the element kernels, now 4.7 / 26; skipped ones first 1081 / 1321, 9.7 / 610, 5.0 / 33.
 // Workgroup (g, h) takes the runs led by rows [g * grp, (g + 1) * grp): 16 rows, about one run
 // of a prompt, in large calls, 4 in small INT8 ones, where the rows are the verify rows of many
 // sequences and a workgroup with several runs does them one after the other.
@@ -361,6 +365,9 @@ __global__ void __launch_bounds__(256) append_int8_block_kernel(AppendArgs a) {
 constexpr int kRunBs = 16;     // block size
 constexpr int kRunRows = 1024; // above: any pool (launch_kv_append)
 constexpr int kRunMaxD = 128;  // one 8-dim item per thread: 16 offsets x head_dim / 8 <= 256
+constexpr int kRunGap = 2;     // skipped rows that end a run (not INT8)
+// Leaders are among lanes 16 to 31 of the window, and a run's 16 rows lie at most kRunGap apart.
+static_assert(16 + kRunBs - 1 + (kRunBs - 1) * kRunGap < 64, "a run lies in its window");
 
 template <gg_dtype_t SRC, gg_dtype_t DST>
 __global__ void __launch_bounds__(256) append_run_kernel(AppendArgs a, int grp) {
@@ -378,23 +385,36 @@ __global__ void __launch_bounds__(256) append_run_kernel(AppendArgs a, int grp) 
     const int blk = slot_ok(slot, a.num_slots) ? slot / kRunBs : -1;
     const unsigned long long valid = __ballot(blk >= 0);
     // A row leads unless the nearest earlier row that is not skipped lands in its block.
-    bool lead = blk >= 0 && lane >= 16 && lane < 16 + grp;
-    {
-        const unsigned long long earlier = valid & ((1ull << lane) - 1);
-        const int p = earlier ? 63 - __builtin_clzll(earlier) : 0;
-        const int pblk = __shfl(blk, p);
-        if (lead && earlier) {
-            lead = pblk != blk;
-        } else if (lead) {
-            for (int q = r0 - 17; q >= 0; --q) {  // (sixteen or more skipped rows before it)
-                const int sq = a.slots[q];
-                if (!slot_ok(sq, a.num_slots)) continue;
-                lead = sq / kRunBs != blk;
-                break;
+    constexpr bool kInt8 = DST == GG_DTYPE_INT8;
+    const unsigned long long earlier = valid & ((1ull << lane) - 1);
+    const int p = earlier ? 63 - __builtin_clzll(earlier) : 0;
+    const int pblk = __shfl(blk, p);
+    const bool here = lane >= 16 && lane < 16 + grp;
+    bool first = blk >= 0 && (!earlier || pblk != blk || (!kInt8 && lane - p > kRunGap));
+    // Blocks of the 256 rows from row q on in direction dir (lane l: rows l, l + 64, ...; -1: none).
+    [[maybe_unused]] auto walk = [&](int q, int dir, int (&s4)[4], int (&b4)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int r = q + dir * (64 * u + lane);
+            s4[u] = r >= 0 && r < a.n_rows ? a.slots[r] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b4[u] = slot_ok(s4[u], a.num_slots) ? s4[u] / kRunBs : -1;
+    };
+    if (kInt8 && __any(here && first && !earlier)) {  // (one lane; sixteen or more skipped rows before it)
+        int pb = -1;
+        for (int q = r0 - 17; q >= 0 && pb < 0; q -= 256) {
+            int s4[4], b4[4];
+            walk(q, -1, s4, b4);
+            for (int u = 0; u < 4 && pb < 0; ++u) {
+                const unsigned long long m = __ballot(b4[u] >= 0);
+                if (m) pb = __shfl(b4[u], __builtin_ctzll(m));
             }
         }
+        if (!earlier) first = blk >= 0 && pb != blk;
     }
-    unsigned long long leaders = __ballot(lead);
+    const unsigned long long firsts = __ballot(first);
+    unsigned long long leaders = __ballot(here && first);
     if (!leaders) return;
     float kinv = 1.f, vinv = 1.f;
     if constexpr (DST == GG_DTYPE_FP8_E4M3) {
@@ -406,20 +426,32 @@ __global__ void __launch_bounds__(256) append_run_kernel(AppendArgs a, int grp) 
         const int i = __builtin_ctzll(leaders);
         leaders &= leaders - 1;
         const int B = __shfl(blk, i), lead_off = __shfl(slot, i) % kRunBs;
-        // The run ends at the first later row of another block.
+        // The run ends at the first later row of another block, or of another run.
         const unsigned long long from = ~0ull << i;
-        const unsigned long long other = __ballot(blk >= 0 && blk != B) & from;
+        const unsigned long long other = kInt8 ? __ballot(blk >= 0 && blk != B) & from : firsts & (from << 1);
         const unsigned long long upto = other ? (other & (0 - other)) - 1 : ~0ull;
         const bool mine = blk == B && ((from & upto) >> lane & 1);
         if (threadIdx.x < kRunBs) s_row[threadIdx.x] = -1;
         __syncthreads();
         if (wave == 0 && mine) s_row[slot % kRunBs] = wr;
-        if (!other && threadIdx.x == 0) {  // (only when skipped rows fill the rest of the window)
-            for (int q = r0 + 48; q < a.n_rows; ++q) {
+        if (kInt8 && !other && wave == 0) {  // (only when skipped rows fill the rest of the window)
+            unsigned long long end = 0;
+            for (int q = r0 + 48; q < a.n_rows && !end; q += 256) {
+                int s4[4], b4[4];
+                walk(q, 1, s4, b4);
+                for (int u = 0; u < 4 && !end; ++u) {
+                    end = __ballot(b4[u] >= 0 && b4[u] != B);
+                    const unsigned long long before = end ? (end & (0 - end)) - 1 : ~0ull;
+                    if (b4[u] == B && (before >> lane & 1)) s_row[s4[u] % kRunBs] = q + 64 * u + lane;
+                }
+            }
+        } else if (!kInt8 && !other && threadIdx.x == 0) {  // (rows past the window only when slots repeat)
+            int last = r0 - 16 + 63 - __builtin_clzll(valid);
+            for (int q = r0 + 48; q < a.n_rows && q - last <= kRunGap; ++q) {
                 const int sq = a.slots[q];
                 if (!slot_ok(sq, a.num_slots)) continue;
                 if (sq / kRunBs != B) break;
-                s_row[sq % kRunBs] = q;
+                s_row[sq % kRunBs] = last = q;
             }
         }
         __syncthreads();

@@ -3,6 +3,7 @@ the oracle mirror: prompts that start inside a block, head_dims below the larges
 skipped rows longer than the kernel's slot window, rows in no order."""
 import numpy as np
 import pytest
+import torch
 
 from helpers import PoolMirror, append_rows, say
 from test_gpu_kv import make_cache
@@ -60,3 +61,46 @@ def test_rows_in_no_order(gpu, dt):
     say(f"append runs shuffled dt={dt}")
     slots = np.random.default_rng(4).permutation(90 * 16)[:1300]
     check(dt, "bf16", 2, 128, [slots], 90, 8)
+
+
+@pytest.mark.parametrize("dt", ["fp8", "bf16", "int8"])
+@pytest.mark.parametrize("gaps", [(0, 1), (0, 1, 2), (1, 2, 3), (2,), (15, 31, 32, 47), (0, 0, 63, 64, 255, 256, 257)])
+def test_skipped_rows_inside_runs(gpu, dt, gaps):
+    """Gaps around the number of skipped rows that ends a run, at every place of a block, and runs
+    as long as they get."""
+    say(f"append runs gaps dt={dt} gaps={gaps}")
+    rng = np.random.default_rng(len(gaps))
+    order = rng.permutation(90)
+    slots = []
+    for slot in prompt(order, 7, 1100):
+        slots += [slot] + [-1] * rng.choice(gaps)
+    check(dt, "bf16", 2, 64, [slots], 90, 5)
+
+
+@pytest.mark.parametrize("dt", ["fp8", "bf16", "int8"])
+@pytest.mark.parametrize("first", [0, 8092])
+def test_skipped_rows_cost_no_more_than_written_ones(gpu, dt, first):
+    """A hundred rows of a prompt padded to 8192, before or after the skipped ones, against 8192
+    rows (walked row by row, the skipped ones took ninety times as long as these)."""
+    H, D, n = 8, 128, 8192
+    say(f"append runs padded dt={dt} first={first}")
+    kv = make_cache(dt, H, D, 16, n // 16)
+    if dt == "fp8":
+        kv.set_head_scales(0, [0.01] * H, [0.01] * H)
+    k = torch.randn(n, H, D, device="cuda", dtype=torch.bfloat16)
+    full = torch.arange(n, dtype=torch.int32, device="cuda")
+    padded = torch.full_like(full, -1)
+    padded[first:first + 100] = full[:100]
+    times = []
+    for slots in (full, padded):
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        for i in range(25):
+            if i == 5:
+                start.record()
+            kv.append(0, k, k, slots)
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end) / 20 * 1e3)
+    kv.close()
+    print(f"  full {times[0]:.1f} us, padded {times[1]:.1f} us")
+    assert times[1] < 4 * times[0]  # (launches and host noise included)
