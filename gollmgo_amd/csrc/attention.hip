@@ -212,6 +212,35 @@ AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int ma
     return {ATTN_SCHED_STREAMK, 0};
 }
 
+// Narrow tables at head_dim 64 or in row groups: the per-row kernel reads K/V once per query row,
+// the MFMA kernels once per item but at the price of a piece's start, and a call that plans for
+// itself runs the plan kernel first. Both are estimated in µs, at contexts of three quarters of
+// the table's width, from 1128 shapes measured on one box (head_dim 64 and 128, 1 to 512 sequences,
+// 1 to 512 query rows per kv head, F16, FP8 and INT8 pools; BF16 costs what F16 does). A call that
+// plans for itself takes its faster kernel but for 25 shapes, where it loses 10 to 45 %. 256
+// sequences of up to 32 keys, 32 heads of one row, INT8: 125.7 -> 14.4 µs, planned 92 -> 14.4; 64 of
+// 16 keys, 8 kv heads, BF16: 14.8 -> 5. Past 512 keys the per-row kernel needs more partitions than one
+// workgroup merges, and loses except for one row per head.
+bool attn_rows_faster(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks, bool plans) {
+    const AttnShape sh = attn_shape(kv, rows, num_q_heads);
+    const long long keys = (long long)max_blocks * kv->block_size;
+    if (!sh.full || keys > 64 * kFuseParts) return false;
+    const bool wide = kv->head_dim == 128, fp8 = kv->dtype == GG_DTYPE_FP8_E4M3, byte = fp8 || kv->dtype == GG_DTYPE_INT8;
+    const double k = (double)keys, heads = (double)num_seqs * rows * num_q_heads;
+    const double items = (double)num_seqs * kv->num_kv_heads * sh.groups;
+    // The latency of one workgroup, and its share per query row and head (FP8 decodes in software).
+    const double by_rows = (fp8 ? (wide ? 18 + 0.02 * k : 11.5 + 0.004 * k) : (wide ? 5.3 + 0.01 * k : 4.5 + 0.005 * k)) +
+                           heads * 1e-3 *
+                               (fp8 ? (wide ? 4 + 0.17 * k : 1.5 + 0.07 * k)
+                                    : (wide ? 0.8 + (byte ? 0.024 : 0.035) * k : 0.5 + (byte ? 0.018 : 0.02) * k));
+    // The latency of a piece, and the items past the resident ones.
+    double by_pieces = (wide ? (byte ? 12.3 : 10.7) : (byte ? 6.8 : 6.3) + 2 * (sh.nt - 1)) + 0.005 * k +
+                       (items > 512 ? (items - 512) * (wide ? (byte ? 0.022 : 0.019) : (byte ? 0.0108 : 0.0072)) : 0);
+    // A planned call's pieces append the draft rows too; the per-row kernel has a launch for them.
+    by_pieces += plans ? 4 + 0.07 * num_seqs + 0.0007 * items : -1;
+    return by_rows < by_pieces;
+}
+
 size_t attn_workspace_bytes(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks,
                             int partition) {
     const int max_parts = (max_blocks * kv->block_size + partition - 1) / partition;
@@ -226,16 +255,18 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
     const KV* kv = a.kv;
     KVView view = make_kv_view(kv, a.layer);
     const bool mfma = attn_mfma_scale(a.scale) &&
-                      (a.sched != ATTN_SCHED_GRID || (attn_mfma_supported(kv, a.rows, a.num_q_heads) &&
-                                                      a.partition % 64 == 0 && a.partition <= kMfmaMaxPartition));
+                      (a.sched != ATTN_SCHED_GRID
+                           ? !attn_rows_faster(kv, a.num_seqs, a.rows, a.num_q_heads, a.max_blocks, !a.plan_ready)
+                           : attn_mfma_supported(kv, a.rows, a.num_q_heads) && a.partition % 64 == 0 &&
+                                 a.partition <= kMfmaMaxPartition);
     // Draft rows of the call: the MFMA kernels append them piece by piece (start_piece);
     // the generic path takes a launch of its own first.
     bool combine = true;  // (the partition grid's merge launch)
     // So do the row groups of an INT8 item: each would re-quantise the block it appends to.
     AttnArgs m = a;
     if (!mfma && a.sched != ATTN_SCHED_GRID) {
-        // A planned shape at another scale: partitions that one workgroup merges, which need none
-        // of the workspace. (The schedules' shapes have head_dim 64 or 128.)
+        // A planned shape at another scale, or a narrow one: partitions that one workgroup merges,
+        // which need none of the workspace. (The schedules' shapes have head_dim 64 or 128.)
         const long long keys = (long long)a.max_blocks * kv->block_size;
         m.sched = ATTN_SCHED_GRID;
         m.partition = (int)(((keys + kFuseParts - 1) / kFuseParts + 63) / 64 * 64);

@@ -184,6 +184,9 @@ __host__ __device__ constexpr int lpt_pieces(int slots, int num_seqs, int heads)
 // Bound on the partial records: a split item of n > T chunks has at most 2 n / T pieces, so
 // split items have at most 2 C / T <= slots.
 __host__ __device__ constexpr int lpt_records(int slots) { return slots; }
+// Whether the per-row kernel is the faster one for a shape that attn_full_supported takes (attention.hip);
+// plans: the call makes its own plan.
+bool attn_rows_faster(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks, bool plans);
 // Automatic partition of the per-row kernel (tokens).
 int attn_generic_partition(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks);
 AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks,

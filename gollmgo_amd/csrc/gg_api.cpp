@@ -338,7 +338,10 @@ static gg_status_t verify_attention_impl(gg_kv_t kv, int layer, const void* q, g
         a.v_new = v_new;
         a.new_dtype = new_dtype;
     }
-    if (call == ATTN_CALL_PLAN_ONLY) return launch_attn_plan(a, (hipStream_t)stream);
+    if (call == ATTN_CALL_PLAN_ONLY)
+        return attn_rows_faster(kv, num_seqs, rows_per_seq, num_q_heads, max_blocks_per_seq, false)
+                   ? GG_OK  // (planned calls do without)
+                   : launch_attn_plan(a, (hipStream_t)stream);
     return launch_verify_attention(a, (hipStream_t)stream);
 }
 
