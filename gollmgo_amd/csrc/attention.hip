@@ -217,22 +217,20 @@ AttnPlan attn_plan(const KV* kv, int num_seqs, int rows, int num_q_heads, int ma
 // itself runs the plan kernel first. Both are estimated in µs, at contexts of three quarters of
 // the table's width, from 1128 shapes measured on one box (head_dim 64 and 128, 1 to 512 sequences,
 // 1 to 512 query rows per kv head, F16, FP8 and INT8 pools; BF16 costs what F16 does). A call that
-// plans for itself takes its faster kernel but for 25 shapes, where it loses 10 to 45 %. 256
-// sequences of up to 32 keys, 32 heads of one row, INT8: 125.7 -> 14.4 µs, planned 92 -> 14.4; 64 of
-// 16 keys, 8 kv heads, BF16: 14.8 -> 5. Past 512 keys the per-row kernel needs more partitions than one
+// plans for itself takes its faster kernel but for 14 shapes, where it loses 10 to 41 %. 256
+// sequences of up to 32 keys, 32 heads of one row, INT8: 125.7 -> 10.8 µs, planned 92 -> 10.8; 64,
+// 8 heads, BF16: 14.8 -> 5.3. Past 512 keys the per-row kernel needs more partitions than one
 // workgroup merges, and loses except for one row per head.
 bool attn_rows_faster(const KV* kv, int num_seqs, int rows, int num_q_heads, int max_blocks, bool plans) {
     const AttnShape sh = attn_shape(kv, rows, num_q_heads);
     const long long keys = (long long)max_blocks * kv->block_size;
     if (!sh.full || keys > 64 * kFuseParts) return false;
-    const bool wide = kv->head_dim == 128, fp8 = kv->dtype == GG_DTYPE_FP8_E4M3, byte = fp8 || kv->dtype == GG_DTYPE_INT8;
+    const bool wide = kv->head_dim == 128, byte = dtype_bytes(kv->dtype) == 1;
     const double k = (double)keys, heads = (double)num_seqs * rows * num_q_heads;
     const double items = (double)num_seqs * kv->num_kv_heads * sh.groups;
-    // The latency of one workgroup, and its share per query row and head (FP8 decodes in software).
-    const double by_rows = (fp8 ? (wide ? 18 + 0.02 * k : 11.5 + 0.004 * k) : (wide ? 5.3 + 0.01 * k : 4.5 + 0.005 * k)) +
-                           heads * 1e-3 *
-                               (fp8 ? (wide ? 4 + 0.17 * k : 1.5 + 0.07 * k)
-                                    : (wide ? 0.8 + (byte ? 0.024 : 0.035) * k : 0.5 + (byte ? 0.018 : 0.02) * k));
+    // The latency of one workgroup, and the throughput per query row and head.
+    const double by_rows = (wide ? 5.3 + 0.01 * k : 4.5 + 0.005 * k) +
+                           heads * 1e-3 * (wide ? 0.8 + (byte ? 0.024 : 0.035) * k : 0.5 + (byte ? 0.018 : 0.02) * k);
     // The latency of a piece, and the items past the resident ones.
     double by_pieces = (wide ? (byte ? 12.3 : 10.7) : (byte ? 6.8 : 6.3) + 2 * (sh.nt - 1)) + 0.005 * k +
                        (items > 512 ? (items - 512) * (wide ? (byte ? 0.022 : 0.019) : (byte ? 0.0108 : 0.0072)) : 0);

@@ -29,7 +29,11 @@ struct Pool16 {
             if constexpr (DT == GG_DTYPE_F32) f[k] = __uint_as_float(w[k]);
             else if constexpr (DT == GG_DTYPE_F16) f[k] = f16_bits_to_f32((uint16_t)(w[k >> 1] >> (16 * (k & 1))));
             else if constexpr (DT == GG_DTYPE_BF16) f[k] = bf16_bits_to_f32((uint16_t)(w[k >> 1] >> (16 * (k & 1))));
-            else if constexpr (DT == GG_DTYPE_FP8_E4M3) f[k] = fp8e4m3_to_f32((uint8_t)(w[k >> 2] >> (8 * (k & 3))));
+            else if constexpr (DT == GG_DTYPE_FP8_E4M3)
+                f[k] = (k & 3) == 0   ? fp8e4m3_to_f32<0>(w[k >> 2])
+                       : (k & 3) == 1 ? fp8e4m3_to_f32<1>(w[k >> 2])
+                       : (k & 3) == 2 ? fp8e4m3_to_f32<2>(w[k >> 2])
+                                      : fp8e4m3_to_f32<3>(w[k >> 2]);
             else f[k] = (float)(int8_t)(uint8_t)(w[k >> 2] >> (8 * (k & 3)));
         }
     }

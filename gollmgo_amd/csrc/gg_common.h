@@ -212,17 +212,13 @@ __device__ __forceinline__ void store_from_f32(void* p, gg_dtype_t dt, size_t i,
     }
 }
 
-// OCP FP8 E4M3 ("fn") decode: bias 7, no infinities, S.1111.111 = NaN.
-__device__ __forceinline__ float fp8e4m3_to_f32(uint8_t b) {
-    uint32_t s = (uint32_t)(b & 0x80) << 24;
-    uint32_t e = (b >> 3) & 0xF;
-    uint32_t m = b & 0x7;
-    if ((b & 0x7F) == 0x7F) return __uint_as_float(0x7fc00000u | s);
-    if (e == 0) {
-        float v = (float)m * 0.001953125f;  // m * 2^-9
-        return s ? -v : v;
-    }
-    return __uint_as_float(s | ((e + 120u) << 23) | (m << 20));
+// OCP FP8 E4M3 ("fn") decode: bias 7, no infinities, S.1111.111 = NaN. Byte SEL of a word, by the
+// gfx950 conversion v_cvt_f32_fp8 (exact). In integer code the tests for NaN and subnormals were
+// two divergent branches per element: 320 query rows on 64 x 4 heads, head_dim 96, 16 keys
+// 29.3 -> 7.7 µs.
+template <int SEL = 0>
+__device__ __forceinline__ float fp8e4m3_to_f32(uint32_t w) {
+    return __builtin_amdgcn_cvt_f32_fp8((int)w, SEL);
 }
 
 // fp32 -> E4M3 with round-to-nearest-even and saturation to +-448 (the __NV_SATFINITE

@@ -2,9 +2,12 @@
 (block size, pool type), every partition of a row in one workgroup or merged by a launch of its
 own, one to five 64-dim groups, rows that are no multiple of 16 bytes; against the oracle."""
 import pytest
+import torch
 
+from gollmgo_amd._lib import lib
+from gollmgo_amd.verify import device_bytes
 from helpers import TOL, say
-from test_gpu_kv import run_attention_case
+from test_gpu_kv import make_cache, run_attention_case
 
 pytestmark = pytest.mark.gpu
 
@@ -23,3 +26,23 @@ def test_ragged_rows(gpu):
     say("per-row ragged")
     err = run_attention_case("f32", 3, 4, 4, 2, 64, 16, [100, 7, 300], row_counts=[4, 1, 2], seed=1)
     assert err <= TOL["f32"]
+
+
+@pytest.mark.parametrize("bs", [16, 8])
+def test_fp8_codes(gpu, bs):
+    """All 256 E4M3 codes, as the V of a sequence's only key, come back exactly (NaN as NaN)."""
+    say(f"per-row fp8 codes bs={bs}")
+    H, D = 4, 64
+    kv = make_cache("fp8", H, D, bs, 1)
+    kv.set_head_scales(0, [1.0] * H, [1.0] * H)
+    kv.append(0, torch.zeros(1, H, D, device="cuda"), torch.zeros(1, H, D, device="cuda"),
+              torch.zeros(1, dtype=torch.int32, device="cuda"))
+    codes = torch.arange(256, dtype=torch.uint8)
+    v = device_bytes(lib().gg_kv_v_layer_ptr(kv.handle, 0), (2 * H - 1) * bs * D)
+    torch.as_strided(v, (H, D), (2 * bs * D, bs)).copy_(codes.view(H, D))
+    out = torch.zeros(1, 1, H, D, device="cuda")
+    kv.attention(0, torch.ones_like(out), out, torch.ones(1, dtype=torch.int32, device="cuda"),
+                 torch.zeros(1, 1, dtype=torch.int32, device="cuda"), 1.0, partition_tokens=64)
+    torch.cuda.synchronize()
+    assert torch.equal(out.cpu().flatten().nan_to_num(999.0), codes.view(torch.float8_e4m3fn).float().nan_to_num(999.0))
+    kv.close()
