@@ -62,7 +62,8 @@ using namespace fd;
 constexpr int kSeg = 8192;        // elements per block of the pass and kept launches
 constexpr int kSegThreads = 512;
 constexpr int kCap = 4096;        // items of one bin the select launch can gather
-constexpr int kTopK = 1024;       // largest top-k drawn from one list
+constexpr int kTopK = 768;        // largest top-k drawn from one list: with top-p,
+constexpr int kTopKAlone = 400;   //   without
 constexpr int kTopCap = kCap + kTopK;  // its list: the threshold bin, and fewer than kTopK elements above
 constexpr int kTopThreads = 512;
 constexpr int kTopSmall = 2 * kTopThreads;  // longest list ranked by comparing all pairs
@@ -1449,8 +1450,12 @@ __global__ void __launch_bounds__(kTopThreads) sample_topp_draw_kernel(DrawParam
 // kept sums. At most kTopK elements lie above the threshold bin, so the list down to that bin
 // holds everything the threshold, the nucleus and the draw need. 32 sequences of 128256 bf16
 // logits (25 drawn rows), top-k 50 and top-p 0.95: the draw's launches 95 -> 30 µs (count 8.7,
-// gather 8.4, draw 9.0, exact check 3.8), bound by their latency (6.4 MB each). kTopK bounds the
-// list's LDS; larger k take the general path.
+// gather 8.4, draw 9.0, exact check 3.8), bound by their latency (6.4 MB each). Ranking by pairs
+// grows with the list: larger k take the general path. List against general path, a whole call,
+// k = 50 / 400 / 512 / 640 / 768 / 900 / 1000: 32 rows of 128256 bf16 logits, top-p 0.9 38 / 56 / 64 /
+// 71 / 78 / 85 / 90 against 108 to 113 µs, without 37 / 55 / 64 / 71 / 78 / 85 / 89 against 64 to 69;
+// 8 rows of 1500 f32 logits 27 / 43 / 52 / 58 / 65 / 72 / 77 against 64 to 67, without 27 / 43 /
+// 51 / 58 / 65 / 71 / 77 against 43 to 45.
 
 // Per (segment, sequence): the bin where the count from the top first reaches k (every
 // block finds it from the row's histogram, next to its own loads in flight), and the
@@ -2021,7 +2026,7 @@ fd::DrawParams fd::final_draw_params(const FinalDraw& d, void* ws) {
     P.use_p = d.top_p > 0 && d.top_p < 1.0;
     P.filtered = P.use_k || P.use_p;
     P.hint_mode = d.spec_key && P.use_p && !P.use_k;
-    P.top_list = P.use_k && d.top_k <= kTopK && !d.draft_probs;
+    P.top_list = P.use_k && d.top_k <= (P.use_p ? kTopK : kTopKAlone) && !d.draft_probs;
     P.kept_launched = (d.draft_probs && (P.filtered || !d.spec_s)) || (P.use_k && P.use_p && !P.top_list);
     {
         const size_t eb = dtype_bytes(d.dt);

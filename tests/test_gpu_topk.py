@@ -49,3 +49,10 @@ def test_special_rows(gpu):
     for top_k, top_p in [(40, 0.9), (40, 0.0), (3, 0.5)]:
         for u in (0.0, 0.37, 0.999999):
             check(torch.from_numpy(host), host, drafts, n, np.full(B, u), 0.8, top_k, top_p, f"special k={top_k} p={top_p} u={u}")
+
+
+@pytest.mark.parametrize("top_k,top_p", [(400, 0.0), (401, 0.0), (401, 0.9), (768, 0.9), (769, 0.9), (768, 0.0)])
+@pytest.mark.parametrize("dt,V", [("bf16", 20011), ("f32", 900)])
+def test_k_around_the_largest_list(gpu, dt, V, top_k, top_p):
+    lg, host, drafts, n, u = case(6, 1, V, dt, seed=top_k + V, accept_all=1.0)
+    check(lg, host, drafts, n, u, 0.9, top_k, top_p, f"topk limit dt={dt} V={V} k={top_k} p={top_p}")
