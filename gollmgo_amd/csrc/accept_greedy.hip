@@ -11,6 +11,8 @@
 //      token; if none differs, row n supplies the bonus token.
 // Tie rule: first index of the maximum. NaN never wins; a NaN at element 0 makes
 // the row's argmax 0 (the reference scans with `>` from element 0).
+#include <type_traits>
+
 #include "gg_common.h"
 #include "gg_draw.h"
 
@@ -38,15 +40,15 @@ __device__ __forceinline__ ArgBest wave_best(ArgBest b) {
     return b;
 }
 
-// First maximum of elements [base, end) of a row, by one wave: 16-byte vectors aligned in
-// memory, lane l taking vectors l, l + 64, ..., all of a segment's loads in flight at once.
+// First maximum of elements [base, end) of a row, at most LEN, by one wave: 16-byte vectors
+// aligned in memory, lane l taking vectors l, l + 64, ..., all of their loads in flight at once.
 // A lane's indices ascend, so a strict `>` keeps its first maximum and never takes NaN. The
 // vectors that the segment cuts (a row need not start on 16 bytes) are read by element.
-template <gg_dtype_t DT>
+template <gg_dtype_t DT, int LEN>
 __device__ __forceinline__ ArgBest scan_segment(const void* row, int base, int end) {
     constexpr int kEB = DT == GG_DTYPE_F32 ? 4 : 2;
     constexpr int kPer = 16 / kEB;
-    constexpr int kIters = kSeg / (64 * kPer);
+    constexpr int kIters = LEN / (64 * kPer);
     const int lane = threadIdx.x & 63;
     const uint8_t* p = (const uint8_t*)row + (size_t)base * kEB;
     const int shift = (int)((uintptr_t)p & 15) / kEB;  // elements between the aligned start and base
@@ -91,21 +93,36 @@ __device__ __forceinline__ ArgBest scan_segment(const void* row, int base, int e
     return b;
 }
 
-// One wave per 4096-element segment. A 256-thread block per segment had two loads in flight
-// per thread and spent most of its life in the reduction: 32 x 5 rows of 128256 bf16 logits
+// One wave per 4096-element segment (SPLIT 1). A 256-thread block per segment had two loads in
+// flight per thread and spent most of its life in the reduction: 32 x 5 rows of 128256 bf16 logits
 // (41 MB) 15.4 -> 10.5 us, 128 x 6 rows (197 MB) 57 -> 34 us (5.8 TB/s).
-template <gg_dtype_t DT>
+// SPLIT 4, a wave per quarter: where the waves of whole segments are fewer than the SIMDs, a
+// wave's own chain of loads and compares is the time (launch_accept_greedy).
+template <gg_dtype_t DT, int SPLIT>
 __global__ void __launch_bounds__(kThreads) greedy_segment_kernel(const void* __restrict__ logits, int rows, int R, int V,
                                                                   int nseg, const int32_t* __restrict__ n_drafts,
                                                                   float2* __restrict__ ws) {
-    const int w = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);  // row * nseg + segment
+    constexpr int kWaves = kThreads / 64, kLen = kSeg / SPLIT;
+    static_assert(SPLIT == 1 || SPLIT == kWaves, "a block is one segment or a segment per wave");
+    const int wave = threadIdx.x >> 6;
+    const int w = SPLIT == 1 ? blockIdx.x * kWaves + wave : blockIdx.x;  // row * nseg + segment
     const int row = __builtin_amdgcn_readfirstlane(w / nseg), seg = __builtin_amdgcn_readfirstlane(w % nseg);
     if (row >= rows) return;
     const int b = row / R, j = row % R;
     const int nb = n_drafts[b];
     if (j > (nb < 0 ? 0 : nb)) return;  // rows 0..n, n clamped as the decide kernel clamps it
     const void* rowp = (const uint8_t*)logits + (size_t)row * V * dtype_bytes(DT);
-    const ArgBest best = wave_best(scan_segment<DT>(rowp, seg * kSeg, min(seg * kSeg + kSeg, V)));
+    const int base = __builtin_amdgcn_readfirstlane(seg * kSeg + (SPLIT == 1 ? 0 : wave * kLen));
+    ArgBest best = wave_best(scan_segment<DT, kLen>(rowp, base, min(base + kLen, V)));  // (none past the row)
+    if constexpr (SPLIT > 1) {
+        __shared__ ArgBest s_best[kWaves];
+        if ((threadIdx.x & 63) == 0) s_best[wave] = best;
+        __syncthreads();
+        if (threadIdx.x) return;
+        best = s_best[0];
+        for (int i = 1; i < kWaves; ++i)
+            if (s_best[i].v > best.v) best = s_best[i];  // (-inf where none; the first maximum wins)
+    }
     if ((threadIdx.x & 63) == 0) ws[(size_t)row * nseg + seg] = make_float2(best.v, __int_as_float(best.i));
 }
 
@@ -201,12 +218,23 @@ gg_status_t launch_accept_greedy(const void* logits, gg_dtype_t dt, int num_seqs
     if (R > kMaxRows) return fail(GG_ERR_INVALID, "accept_greedy: more than 64 drafts per sequence");
     const int nseg = (vocab + kSeg - 1) / kSeg;
     const int rows = num_seqs * R;
-    const unsigned grid = (unsigned)(((long long)rows * nseg + kThreads / 64 - 1) / (kThreads / 64));
+    // Quarters up to one segment per SIMD. Calls with whole / quarter segments, f32: 1 x 1 row of 1000
+    // (1 segment) 5.8 / 5.5 us, 1 x 9 of 1000 6.8 / 6.1, 8 x 1 of 128256 (256) 8.0 / 6.9, 32 x 1
+    // (1024) 8.3 / 7.7; bf16: 1 x 5 of 128256 (160) 7.8 / 6.7, 16 x 5 of 50257 (1040) 8.9 / 8.9, 16 x 3 of
+    // 128256 (1536) 8.2 / 8.5, 16 x 9 of 50257 (1872) 9.5 / 10.8.
+    const long long segs = (long long)rows * nseg;
+    const bool split = segs <= 4 * device_cu_count();
+    const unsigned grid = (unsigned)(split ? segs : (segs + kThreads / 64 - 1) / (kThreads / 64));
     float2* seg = (float2*)ws;
+    auto scan = [&](auto dt_tag) {
+        constexpr gg_dtype_t DT = decltype(dt_tag)::value;
+        if (split) greedy_segment_kernel<DT, 4><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg);
+        else greedy_segment_kernel<DT, 1><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg);
+    };
     switch (dt) {
-        case GG_DTYPE_F32: greedy_segment_kernel<GG_DTYPE_F32><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg); break;
-        case GG_DTYPE_BF16: greedy_segment_kernel<GG_DTYPE_BF16><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg); break;
-        default: greedy_segment_kernel<GG_DTYPE_F16><<<grid, kThreads, 0, s>>>(logits, rows, R, vocab, nseg, n_drafts, seg); break;
+        case GG_DTYPE_F32: scan(std::integral_constant<gg_dtype_t, GG_DTYPE_F32>{}); break;
+        case GG_DTYPE_BF16: scan(std::integral_constant<gg_dtype_t, GG_DTYPE_BF16>{}); break;
+        default: scan(std::integral_constant<gg_dtype_t, GG_DTYPE_F16>{}); break;
     }
     if (draw)
         greedy_decide_kernel<true><<<num_seqs, kDecideThreads, 0, s>>>(logits, dt, max_drafts, vocab, nseg, drafts, n_drafts,

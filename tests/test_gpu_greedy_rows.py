@@ -37,3 +37,20 @@ def test_argmax_of_rows_at_any_alignment(gpu, dt, V):
     acc, tok = gv.accept_greedy(logits, torch.from_numpy(drafts).cuda(), torch.full((B,), K, dtype=torch.int32, device="cuda"))
     assert acc.tolist() == [K, K, 1]
     assert tok.tolist() == [best[0, K], best[1, K], best[2, 1]]
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,V", [(342, 7), (341, 4097), (342, 4097), (342, 2051)])
+def test_argmax_of_many_rows(gpu, dt, B, V):
+    """More segments than a wave per SIMD (whole segments per wave), and around that number."""
+    say(f"greedy many rows {dt} B={B} V={V}")
+    K = 2
+    x = np.random.default_rng(V + B).integers(-4, 4, (B, K + 1, V)).astype(np.float32)
+    x[5, 0, :] = -np.inf
+    x[6, 1, 0] = np.nan
+    best = np.array([[argmax_first(row) for row in rows] for rows in x])
+    drafts = best[:, :K].astype(np.int32)
+    acc, tok = gv.accept_greedy(torch.from_numpy(x).to(dt).cuda(), torch.from_numpy(drafts).cuda(),
+                                torch.full((B,), K, dtype=torch.int32, device="cuda"))
+    assert acc.tolist() == [K] * B
+    assert tok.tolist() == best[:, K].tolist()
