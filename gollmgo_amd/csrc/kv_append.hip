@@ -354,8 +354,12 @@ __global__ void __launch_bounds__(256) append_int8_block_kernel(AppendArgs a) {
 // around it. 100 rows before 8092 skipped ones, FP8 / INT8: 1113 / 1103 µs when one thread walked,
 // 9.5 / 2367 in the element kernels, now 4.7 / 26; skipped ones first 1081 / 1321, 9.7 / 610, 5.0 / 33.
 // Workgroup (g, h) takes the runs led by rows [g * grp, (g + 1) * grp): 16 rows, about one run
-// of a prompt, in large calls, 4 in small INT8 ones, where the rows are the verify rows of many
-// sequences and a workgroup with several runs does them one after the other.
+// of a prompt, in large calls, fewer in small INT8 ones, where the rows are the verify rows of many
+// sequences and a workgroup with several runs does them one after the other (8 heads, 1 / 4 / 16
+// rows a workgroup: 64 x 1 rows 5.1 / 10.4 / 32 µs, 64 x 6 9.2 / 7.2 / 10.5, a prompt of 8192 187 /
+// 52 / 17). Where a workgroup of 16-bit or FP8 pools has kShortRuns runs or more it writes all their
+// rows at once, V by element: FP8 300 x 5 rows 11.2 -> 8.1 µs (the element kernels 10.1), 3000 x 1
+// 35.6 -> 22 (17.5).
 //
 // Bound by memory in large calls. The element kernels wrote V one element at a time, at the
 // tile's 16-offset stride, and INT8 started a workgroup per row, whose leader walked its run's
@@ -363,11 +367,44 @@ __global__ void __launch_bounds__(256) append_int8_block_kernel(AppendArgs a) {
 // layer: FP8 38.9 -> 14.6 µs (50 MB, 3.4 TB/s), BF16 41.3 -> 16.7, INT8 1388 -> 17.4; 2000
 // rows 9.8 -> 7.0, 10.1 -> 7.2 and 296 -> 7.4.
 constexpr int kRunBs = 16;     // block size
-constexpr int kRunRows = 1024; // above: any pool (launch_kv_append)
+constexpr int kRunRows = 1024; // more rows, and more than kRunGroups times kv heads: any pool
+constexpr int kRunGroups = 8192;  //   (launch_kv_append)
 constexpr int kRunMaxD = 128;  // one 8-dim item per thread: 16 offsets x head_dim / 8 <= 256
 constexpr int kRunGap = 2;     // skipped rows that end a run (not INT8)
+constexpr int kShortRuns = 3;  // runs of a workgroup that are written all at once (not INT8)
 // Leaders are among lanes 16 to 31 of the window, and a run's 16 rows lie at most kRunGap apart.
 static_assert(16 + kRunBs - 1 + (kRunBs - 1) * kRunGap < 64, "a run lies in its window");
+
+// Eight values in the pool's format (FP8 and INT8: the low two words).
+template <gg_dtype_t DST>
+__device__ __forceinline__ void pack8(const float (&x)[8], float inv, uint32_t (&w)[4]) {
+    if constexpr (DST == GG_DTYPE_FP8_E4M3 || DST == GG_DTYPE_INT8) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            if constexpr (DST == GG_DTYPE_FP8_E4M3) {
+                w[e >> 2] = f32x2_to_fp8e4m3_sat(x[e] * inv, x[e + 1] * inv) |
+                            (f32x2_to_fp8e4m3_sat(x[e + 2] * inv, x[e + 3] * inv) << 16);
+            } else {
+                w[e >> 2] = 0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w[e >> 2] |= (uint32_t)(uint8_t)f32_to_i8_sat(x[e + u] * inv) << (8 * u);
+            }
+        }
+        w[2] = w[3] = 0;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const uint16_t lo = DST == GG_DTYPE_BF16 ? f32_to_bf16_bits(x[e]) : f32_to_f16_bits(x[e]);
+            const uint16_t hi = DST == GG_DTYPE_BF16 ? f32_to_bf16_bits(x[e + 1]) : f32_to_f16_bits(x[e + 1]);
+            w[e >> 1] = lo | ((uint32_t)hi << 16);
+        }
+    }
+}
+template <int EB>
+__device__ __forceinline__ void store_packed8(uint8_t* base, size_t i, const uint32_t (&w)[4]) {
+    if constexpr (EB == 1) *(uint2*)(base + i) = make_uint2(w[0], w[1]);
+    else *(uint4*)((uint16_t*)base + i) = make_uint4(w[0], w[1], w[2], w[3]);
+}
 
 template <gg_dtype_t SRC, gg_dtype_t DST>
 __global__ void __launch_bounds__(256) append_run_kernel(AppendArgs a, int grp) {
@@ -422,6 +459,37 @@ __global__ void __launch_bounds__(256) append_run_kernel(AppendArgs a, int grp) 
         vinv = a.v_inv[h];
     }
     const int o = threadIdx.x / DG, g = threadIdx.x % DG;  // this thread's offset and dim group
+    if constexpr (!kInt8) {
+        // Several short runs: all their rows at once, V by element.
+        const unsigned long long next = firsts & (~0ull << (16 + grp));
+        const bool inside = next || 64 - (63 - __builtin_clzll(valid)) > kRunGap;  // (else slots repeat)
+        if (__popcll(leaders) >= kShortRuns && inside) {
+            const unsigned long long rows =
+                valid & (~0ull << __builtin_ctzll(leaders)) & (next ? (next & (0 - next)) - 1 : ~0ull);
+            for (int i0 = 0; i0 < 48 * DG && rows >> (16 + i0 / DG); i0 += 256) {
+                const int i = i0 + threadIdx.x, ln = 16 + i / DG, d0 = 8 * (i % DG);
+                const int sl = __shfl(slot, min(ln, 63));
+                if (ln > 63 || !(rows >> ln & 1)) continue;
+                const size_t src = ((size_t)(r0 - 16 + ln) * a.Hkv + h) * D + d0;
+                const size_t tile = ((size_t)(sl / kRunBs) * a.Hkv + h) * (2 * (size_t)kRunBs * D);
+                const int off = sl % kRunBs;
+                float x[8], y[8];
+                uint32_t kw[4], vw[4];
+                load8<SRC>(a.k, src, x);
+                load8<SRC>(a.v, src, y);
+                pack8<DST>(x, kinv, kw);
+                pack8<DST>(y, vinv, vw);
+                store_packed8<kEB>(a.kc, tile + (size_t)off * D + d0, kw);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const size_t vi = tile + (size_t)(d0 + e) * kRunBs + off;
+                    if constexpr (kEB == 1) a.vc[vi] = (uint8_t)(vw[e >> 2] >> (8 * (e & 3)));
+                    else ((uint16_t*)a.vc)[vi] = (uint16_t)(vw[e >> 1] >> (16 * (e & 1)));
+                }
+            }
+            return;
+        }
+    }
     while (leaders) {
         const int i = __builtin_ctzll(leaders);
         leaders &= leaders - 1;
@@ -496,38 +564,14 @@ __global__ void __launch_bounds__(256) append_run_kernel(AppendArgs a, int grp) 
             vinv = v_new > 0.f ? 1.0f / v_new : 0.f;
         }
         if (row >= 0) {
-            if constexpr (kEB == 1) {
-                uint32_t kw[2], vw[2];
+            uint32_t kw[4], vw[4];
+            pack8<DST>(kx, kinv, kw);
+            pack8<DST>(vx, vinv, vw);
+            store_packed8<kEB>(a.kc, tile + (size_t)o * D + 8 * g, kw);
 #pragma unroll
-                for (int e = 0; e < 8; e += 4) {
-                    if constexpr (DST == GG_DTYPE_FP8_E4M3) {
-                        kw[e >> 2] = f32x2_to_fp8e4m3_sat(kx[e] * kinv, kx[e + 1] * kinv) |
-                                     (f32x2_to_fp8e4m3_sat(kx[e + 2] * kinv, kx[e + 3] * kinv) << 16);
-                        vw[e >> 2] = f32x2_to_fp8e4m3_sat(vx[e] * vinv, vx[e + 1] * vinv) |
-                                     (f32x2_to_fp8e4m3_sat(vx[e + 2] * vinv, vx[e + 3] * vinv) << 16);
-                    } else {
-                        kw[e >> 2] = vw[e >> 2] = 0;
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            kw[e >> 2] |= (uint32_t)(uint8_t)f32_to_i8_sat(kx[e + u] * kinv) << (8 * u);
-                            vw[e >> 2] |= (uint32_t)(uint8_t)f32_to_i8_sat(vx[e + u] * vinv) << (8 * u);
-                        }
-                    }
-                }
-                *(uint2*)(a.kc + tile + (size_t)o * D + 8 * g) = make_uint2(kw[0], kw[1]);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) s_v[(8 * g + e) * kPitch + o] = (uint8_t)(vw[e >> 2] >> (8 * (e & 3)));
-            } else {
-                uint16_t kb[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    kb[e] = DST == GG_DTYPE_BF16 ? f32_to_bf16_bits(kx[e]) : f32_to_f16_bits(kx[e]);
-                    const uint16_t vb = DST == GG_DTYPE_BF16 ? f32_to_bf16_bits(vx[e]) : f32_to_f16_bits(vx[e]);
-                    *(uint16_t*)&s_v[(8 * g + e) * kPitch + 2 * o] = vb;
-                }
-                *(uint4*)((uint16_t*)a.kc + tile + (size_t)o * D + 8 * g) =
-                    make_uint4(kb[0] | ((uint32_t)kb[1] << 16), kb[2] | ((uint32_t)kb[3] << 16),
-                               kb[4] | ((uint32_t)kb[5] << 16), kb[6] | ((uint32_t)kb[7] << 16));
+            for (int e = 0; e < 8; ++e) {
+                if constexpr (kEB == 1) s_v[(8 * g + e) * kPitch + o] = (uint8_t)(vw[e >> 2] >> (8 * (e & 3)));
+                else *(uint16_t*)&s_v[(8 * g + e) * kPitch + 2 * o] = (uint16_t)(vw[e >> 1] >> (16 * (e & 1)));
             }
         }
         __syncthreads();
@@ -585,7 +629,8 @@ __global__ void __launch_bounds__(256) append_run_kernel(AppendArgs a, int grp) 
 
 template <gg_dtype_t SRC>
 void launch_run(const AppendArgs& a, hipStream_t s) {
-    const int grp = a.n_rows <= kRunRows ? 4 : kRunBs;
+    const long long wg = (long long)a.n_rows * a.Hkv;
+    const int grp = a.dst != GG_DTYPE_INT8 ? kRunBs : wg <= 1024 ? 1 : wg <= 2048 ? 2 : wg <= 8192 ? 4 : kRunBs;
     const dim3 grid((a.n_rows + grp - 1) / grp, a.Hkv);
     switch (a.dst) {
         case GG_DTYPE_F16: append_run_kernel<SRC, GG_DTYPE_F16><<<grid, 256, 0, s>>>(a, grp); break;
@@ -626,13 +671,14 @@ gg_status_t launch_kv_append(KV* kv, int layer, const void* k, const void* v, gg
         a.v_bscale = (uint16_t*)kv->v_scales + (size_t)layer * kv->scale_layer_elems;
     }
     const bool vec = a.D % 8 == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0;
-    // Block runs: INT8 calls of any size, FP8 and 16-bit pools past kRunRows rows. Below, a
-    // thread per element (append_dim_kernel) has no tile to wait for: 5 verify rows 2.3 against
-    // 3.2 µs, 64 x 6 rows 3.7 against 5.7 at best, a prompt of 1000 rows 7.2 against 6.9, 2000 rows
-    // 9.8 against 7.0; 512 x 6 verify rows 15.8 against 13.5. INT8: 64 x 6 rows 16.1 -> 8.3,
-    // one sequence's five 7.1 -> 3.9.
+    // Block runs: INT8 calls of any size, FP8 and 16-bit pools past kRunRows rows and kRunGroups
+    // (row, head) pairs. Below, a thread per element (append_dim_kernel) has no tile to wait for:
+    // 5 verify rows 2.3 against 3.2 µs, 64 x 6 rows 3.7 against 5.7 at best, a prompt of 1000 rows
+    // 7.2 against 6.9, 2000 rows 9.8 against 7.0; 512 x 6 verify rows 15.8 against 13.5; two heads,
+    // 300 x 5 bf16 rows 4.8 against 5.6 (from f32), a prompt of 2000 5.1 against 4.8. INT8: 64 x 6
+    // rows 16.1 -> 7.0, one sequence's five 7.1 -> 3.9.
     const bool int8 = kv->scale_mode == GG_SCALE_PER_BLOCK;
-    if (vec && a.bs == kRunBs && a.D <= kRunMaxD && a.dst != GG_DTYPE_F32 && (int8 || a.n_rows > kRunRows)) {
+    if (vec && a.bs == kRunBs && a.D <= kRunMaxD && a.dst != GG_DTYPE_F32 && (int8 || (a.n_rows > kRunRows && (long long)a.n_rows * a.Hkv > kRunGroups))) {
         switch (src) {
             case GG_DTYPE_F32: launch_run<GG_DTYPE_F32>(a, s); break;
             case GG_DTYPE_F16: launch_run<GG_DTYPE_F16>(a, s); break;

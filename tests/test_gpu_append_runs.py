@@ -74,7 +74,38 @@ def test_skipped_rows_inside_runs(gpu, dt, gaps):
     slots = []
     for slot in prompt(order, 7, 1100):
         slots += [slot] + [-1] * rng.choice(gaps)
-    check(dt, "bf16", 2, 64, [slots], 90, 5)
+    check(dt, "bf16", 8, 64, [slots], 90, 5)
+
+
+@pytest.mark.parametrize("dt", ["fp8", "bf16", "f16", "int8"])
+@pytest.mark.parametrize("src,H,D", [("bf16", 8, 128), ("f32", 9, 64), ("f16", 8, 96), ("bf16", 12, 8)])
+def test_runs_of_any_length(gpu, dt, src, H, D):
+    """Enough rows and heads for block runs in every pool: a prompt, verify rows of many sequences
+    (one to sixteen rows that start anywhere in a block and may cross into the next), rows in no
+    order, and short runs next to long ones, with skipped rows between."""
+    say(f"append runs any length dt={dt} src={src} H={H} D={D}")
+    rng = np.random.default_rng(H * D)
+    order = rng.permutation(180)
+
+    def sequences(lengths):
+        slots, blk = [], 0
+        for n in lengths:
+            first = rng.integers(0, 16)
+            if blk * 16 + first + n > 180 * 16:
+                break
+            slots += list(prompt(order, blk * 16 + first, n))
+            blk += (first + n + 15) // 16
+        return slots
+
+    one = [prompt(order, 16 * i + 3, 1)[0] for i in range(180)]
+    mixed = []
+    for slot in sequences(rng.choice([1, 2, 3, 5, 9, 16, 17, 40], 200)):
+        mixed += [slot] + [-1] * int(rng.choice([0, 0, 0, 0, 1, 5]))
+    calls = [prompt(order, 5, 1200), sequences([5] * 180), one, mixed]
+    if dt != "int8":  # (a block's scale follows its runs one after the other)
+        calls.append(rng.permutation(180 * 16)[:1300])
+    # (Calls below the limit are filled up with skipped rows.)
+    check(dt, src, H, D, [list(c) + [-1] * max(0, 1100 - len(c)) for c in calls], 180, D)
 
 
 @pytest.mark.parametrize("dt", ["fp8", "bf16", "int8"])
