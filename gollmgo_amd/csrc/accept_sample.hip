@@ -64,7 +64,8 @@ constexpr int kSegThreads = 512;
 constexpr int kCap = 4096;        // items of one bin the select launch can gather
 constexpr int kTopK = 768;        // largest top-k drawn from one list: with top-p,
 constexpr int kTopKAlone = 400;   //   without
-constexpr int kTopCap = kCap + kTopK;  // its list: the threshold bin, and fewer than kTopK elements above
+constexpr int kTopCap = kCap + kTopK;  // its list: the threshold bin, and fewer than kTopK elements above;
+                                      // places per sequence of every path's list
 constexpr int kTopThreads = 512;
 constexpr int kTopSmall = 2 * kTopThreads;  // longest list ranked by comparing all pairs
 constexpr int kRowThreads = 1024;
@@ -412,7 +413,7 @@ __device__ __forceinline__ void flush_hits(const DrawParams& P, int b, int* s_cn
     __syncthreads();
     if (n > 0 && n <= CAP)
         for (int i = threadIdx.x; i < n; i += blockDim.x)
-            if (*s_base + i < LIST) P.cand[(size_t)b * LIST + *s_base + i] = s_buf[i];
+            if (*s_base + i < LIST) P.cand[(size_t)b * kTopCap + *s_base + i] = s_buf[i];
 }
 
 // Per (segment, sequence): e of every element (the parallel exponential), the segment's
@@ -936,7 +937,7 @@ __device__ bool select2_row(const DrawParams& P, int b, RowInfo& ri, double* s_s
         return false;
     }
     for (int i = threadIdx.x; i < ng; i += blockDim.x) {
-        s_comp[i] = P.cand[(size_t)b * kCap + i];
+        s_comp[i] = P.cand[(size_t)b * kTopCap + i];
         s_e[i] = exp_term(key_value((uint32_t)(s_comp[i] >> 32)), inv_t, m);
     }
     if (threadIdx.x == 0) s_ok = 1;
@@ -1191,7 +1192,7 @@ __device__ void draw_seq(const DrawParams& P, int b, RowInfo ri, const double* k
         const float* qr = q_row(P, b, ri);
         const void* row = drawn_row(P, b, ri.row);
         for (int i = threadIdx.x; i < n; i += blockDim.x) {
-            const int e = (int)P.cand[(size_t)b * kCap + i];
+            const int e = (int)P.cand[(size_t)b * kTopCap + i];
             atomicAdd(&s_sums[e / kSeg], draw_weight(P, ri, qr[e], load_as_f32(row, P.dt, e), e, s_tab, inv));
         }
         __syncthreads();
@@ -1271,7 +1272,7 @@ __global__ void __launch_bounds__(kTopThreads) sample_topp_draw_kernel(DrawParam
     constexpr int kAhead = 4;
     unsigned long long ahead[kAhead];
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) ahead[j] = P.cand[(size_t)b * kCap + j * kTopThreads + threadIdx.x];
+    for (int j = 0; j < kAhead; ++j) ahead[j] = P.cand[(size_t)b * kTopCap + j * kTopThreads + threadIdx.x];
     const bool has = lane < P.nseg;
     const double segsum = has ? P.segsum[(size_t)b * P.nseg + lane] : 0.0;
     const double segabove = has ? P.segabove[(size_t)b * P.nseg + lane] : 0.0;
@@ -1305,7 +1306,7 @@ __global__ void __launch_bounds__(kTopThreads) sample_topp_draw_kernel(DrawParam
             for (int q = 0; q < kAhead; ++q)
                 if (q == j) c = ahead[q];
         } else {
-            c = P.cand[(size_t)b * kCap + i];
+            c = P.cand[(size_t)b * kTopCap + i];
         }
         const float l = key_value((uint32_t)(c >> 32));
         const double e = exp_term(l, inv_t, m);

@@ -57,8 +57,9 @@ struct DrawParams {
     double* segabove;         // per segment: e summed over the bins above cbin
     double* segep;            // per segment (estimated residuals): e of the sure-positive elements
     double* segqp;            //   and their q
-    int* ncand;               // per sequence: elements of cbin gathered
-    unsigned long long* cand; // per sequence: kCap gathered keys
+    int* ncand;               // per sequence: keys gathered (of cbin, or from the top down to it)
+    unsigned long long* cand; // gathered keys, kTopCap places per sequence (accept_sample.hip); a
+                              // list that holds fewer has the same places
     int32_t* out_tok;
 };
 
