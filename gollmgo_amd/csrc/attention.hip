@@ -15,12 +15,14 @@
 //   - attention_mfma.hip: gfx950 MFMA path for head_dim 128, block_size 16,
 //     BF16/F16/FP8/INT8 pools, G*R <= 64 rows per kv head;
 //   - attention_full.hip: the same pieces for head_dim 64 and for more rows per kv head, at
-//     the precision of the per-row kernel (automatic schedule, up to kLptMaxSeqs sequences);
+//     the precision of the per-row kernel (automatic schedule, up to kLptMaxSeqs sequences, where
+//     attn_rows_faster does not prefer the per-row kernel);
 //   - attn_generic_kernel (here): any head_dim <= 1024 / block size / pool dtype,
 //     one wave per (row, head, partition), scalar online softmax. Used for the
-//     shapes the MFMA tiling does not cover (fp32 pools, other head_dims and block sizes)
-//     and for explicit partitions of attention_full.hip's shapes. Its partitions and the
-//     MFMA partition grid share one partial format and one combine kernel.
+//     shapes the MFMA tiling does not cover (fp32 pools, other head_dims and block sizes), for
+//     narrow tables and explicit partitions of attention_full.hip's shapes, and for scales that
+//     the MFMA softmax does not take (attn_mfma_scale). Its partitions and the MFMA partition grid
+//     share one partial format and one combine kernel.
 #include <type_traits>
 
 #include "gg_common.h"
@@ -257,10 +259,7 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
                            ? !attn_rows_faster(kv, a.num_seqs, a.rows, a.num_q_heads, a.max_blocks, !a.plan_ready)
                            : attn_mfma_supported(kv, a.rows, a.num_q_heads) && a.partition % 64 == 0 &&
                                  a.partition <= kMfmaMaxPartition);
-    // Draft rows of the call: the MFMA kernels append them piece by piece (start_piece);
-    // the generic path takes a launch of its own first.
     bool combine = true;  // (the partition grid's merge launch)
-    // So do the row groups of an INT8 item: each would re-quantise the block it appends to.
     AttnArgs m = a;
     if (!mfma && a.sched != ATTN_SCHED_GRID) {
         // A planned shape at another scale, or a narrow one: partitions that one workgroup merges,
@@ -270,6 +269,9 @@ gg_status_t launch_verify_attention(const AttnArgs& a, hipStream_t s) {
         m.partition = (int)(((keys + kFuseParts - 1) / kFuseParts + 63) / 64 * 64);
         m.max_parts = (int)((keys + m.partition - 1) / m.partition);
     }
+    // Draft rows of the call: the MFMA kernels append them piece by piece (start_piece); the
+    // generic path takes a launch of its own first, and so do the row groups of an INT8 item: each
+    // would re-quantise the block it appends to.
     if (a.k_new && (!mfma || (a.row_groups > 1 && kv->dtype == GG_DTYPE_INT8))) {
         const gg_status_t st = launch_append_from_tables(a, view, s);
         if (st != GG_OK) return st;

@@ -11,7 +11,7 @@
 // The per-row kernel read every K/V row once per query row and head: 4 FLOPs per element
 // through L2, 1057 µs a call for 16 f16 sequences of 512-4096 keys at head_dim 64 (32 query
 // heads on 8, five rows; 79 MB of K/V) and 2504 µs for 80 rows per kv head at head_dim 128
-// (bf16, 41 MB). Here 28 and 43 µs: bound by the pieces' start, merge and dependency chain
+// (bf16, 41 MB). Here 22 and 30 µs: bound by the pieces' start, merge and dependency chain
 // (19 chunks of work per slot at most), no longer by re-reading. Error against fp64, 2-norm
 // over nine shapes, as a share of the per-row kernel's, for bf16 / f16 / f32 queries: BF16
 // pools 0.77 / 0.89 / 0.83, F16 0.75 / 0.67 / 0.68, FP8 0.80 / 0.89 / 0.84, INT8 0.81 / 0.86 /

@@ -198,14 +198,14 @@ __device__ __forceinline__ uint4 mask_bytes16(uint4 v, int nvalid) {
     }
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
-// Zero the 2-byte elements at offsets >= nvalid of an 8-offset run starting at `first`.
-// Bytes of an 8-byte run that starts at offset `first`: offsets >= nvalid cleared.
+// Zero the bytes at offsets >= nvalid of an 8-offset run starting at `first`.
 __device__ __forceinline__ uint2 mask_bytes8(uint2 v, int nvalid, int first) {
     const int n = nvalid - first;
     const uint32_t m0 = n >= 4 ? 0xFFFFFFFFu : (n <= 0 ? 0u : 0xFFFFFFFFu >> (8 * (4 - n)));
     const uint32_t m1 = n >= 8 ? 0xFFFFFFFFu : (n <= 4 ? 0u : 0xFFFFFFFFu >> (8 * (8 - n)));
     return make_uint2(v.x & m0, v.y & m1);
 }
+// The same for an 8-offset run of 2-byte elements.
 __device__ __forceinline__ uint4 mask_halves8(uint4 v, int nvalid, int first) {
     uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -384,10 +384,12 @@ constexpr int kAppRows = 8;
 static_assert(kAppRows * 2 <= (int)sizeof(uint4), "a dim's staged rows are one 16-byte word");
 
 // Start piece d (PieceIO::start) and, when the call carries draft rows (a.k_new), take
-// care of the rows whose key positions lie in the piece. A key position belongs to exactly
-// one piece, and only that piece reads it, so no other workgroup waits for these stores;
-// chunks are multiples of 16 tokens, so a block's tokens (its K rows and its V columns)
-// are all read by one chunk, and so by one wave.
+// care of the rows whose key positions lie in the piece. Every workgroup that reads a key
+// position appends its row itself first, so none waits for another's stores: without row groups
+// one piece alone holds the position; with them the piece of each group appends the same row, and
+// the stores write equal bytes (but for PER_BLOCK INT8 pools, whose blocks would be re-scaled by
+// each group: those calls append in a launch of their own). Chunks are multiples of 16 tokens, so
+// a block's tokens (its K rows and its V columns) are all read by one chunk, and so by one wave.
 //   - Rows inside the first chunks that `start` issues (short pieces), more rows than
 //     kAppRows, no `ap` (the stream-K loop over pieces, whose registers are full), or a
 //     PER_BLOCK INT8 pool (a block's new rows re-scale the whole block; a block lies in one

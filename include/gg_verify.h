@@ -172,7 +172,9 @@ gg_status_t gg_kv_append(gg_kv_t kv, int layer, const void* k, const void* v,
  *   partition_tokens: split-K partition length, a multiple of 64. 0 = automatic:
  *                 longest-first pieces (long items cut, split items merged in the
  *                 same launch); past 1024 sequences one workgroup per item, or a
- *                 stream-K split over a fixed grid where contexts are long
+ *                 stream-K split over a fixed grid where contexts are long; narrow
+ *                 tables at head_dim 64 or past 64 query rows per kv head may take one
+ *                 wave per row and head
  *                 (results equal to textbook attention in every case).
  * workspace must hold gg_verify_attention_workspace_size(...) bytes (may be 0). */
 size_t gg_verify_attention_workspace_size(gg_kv_t kv, int num_seqs, int rows_per_seq,
