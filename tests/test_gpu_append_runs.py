@@ -124,14 +124,17 @@ def test_skipped_rows_cost_no_more_than_written_ones(gpu, dt, first):
     padded[first:first + 100] = full[:100]
     times = []
     for slots in (full, padded):
-        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-        for i in range(25):
-            if i == 5:
-                start.record()
-            kv.append(0, k, k, slots)
-        end.record()
-        torch.cuda.synchronize()
-        times.append(start.elapsed_time(end) / 20 * 1e3)
+        kv.append(0, k, k, slots)
+        best = float("inf")
+        for _ in range(5):  # (the best of five: a host that stalls once does not count)
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(20):
+                kv.append(0, k, k, slots)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end) / 20 * 1e3)
+        times.append(best)
     kv.close()
     print(f"  full {times[0]:.1f} us, padded {times[1]:.1f} us")
     assert times[1] < 4 * times[0]  # (launches and host noise included)
